@@ -85,11 +85,12 @@ int pp_mlp_set_params(pp_mlp* m, const float* params);
  * n x n_out); n <= max_batch. */
 int pp_mlp_forward(pp_mlp* m, const float* x, int n, float* y);
 
-/* Inference kernel choice (no counterpart in the reference: a tuning and
- * test switch). fused = 1 (the default) runs every layer of a 64-row tile in
- * one kernel with the activations kept in LDS, where the network has hidden
- * width 256 and input and output widths <= 32; 0 runs one GEMM kernel per
- * layer. Both give bitwise identical outputs. */
+/* Kernel choice (no counterpart in the reference: a tuning and test switch).
+ * fused = 1 (the default) runs inference as one kernel with the activations
+ * kept in LDS, and a training step (or pp_mlp_loss_grad) as two, where the
+ * network has hidden width 256 and input and output widths <= 32 (training: up
+ * to 6 hidden layers); 0 runs one kernel per layer and reduction. Both give
+ * bitwise identical outputs, gradients and parameters. */
 int pp_mlp_set_fused(pp_mlp* m, int fused);
 
 /* Loss and gradient of one batch (host features n x n_in, labels n x
@@ -104,7 +105,8 @@ int pp_mlp_adam_step(pp_mlp* m, const pp_adam* opt);
 /* Training on a device-resident dataset: n samples of features and labels
  * (host arrays, uploaded once). Each step draws `batch` samples with
  * replacement (Philox on the device, key = seed), runs forward, loss,
- * backward and Adam; the step is one hipGraph replayed n_steps times.
+ * backward and Adam: two launches per step, or (see pp_mlp_set_fused) one
+ * hipGraph of the layer-by-layer kernels replayed n_steps times.
  * loss_curve (n_steps floats, host, may be NULL) receives the batch losses. */
 int pp_mlp_train(pp_mlp* m, const float* x, const float* labels, int64_t n, int batch,
                  int n_steps, const pp_adam* opt, uint64_t seed, float* loss_curve);

@@ -324,20 +324,42 @@ __global__ void bump_kernel(uint32_t* step) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *step += 1;
 }
 
-// Weights of one layer in the order the fused inference kernel loads them:
-// for 32-column tile T and 16-deep K fragment i, the 64 lanes' 8 bf16 each,
-// contiguous: chunk (T*nf + i)*64 + lane holds W[32T + lane%32][16i +
-// (lane/32)*8 + j], j = 0..7, zero beyond K and N.
-__global__ void pack_fused_kernel(const bf16* W, int K, int N, int nf, int64_t chunks,
-                                  bf16* out) {
+// Weights in the order the fused kernels load them: for 32-row tile T and
+// 16-deep K fragment i of an operand A(m, k), the 64 lanes' 8 bf16 each,
+// contiguous: chunk (T*nf + i)*64 + lane holds A(32T + lane%32, 16i +
+// (lane/32)*8 + j), j = 0..7, zero beyond the matrix. One launch packs every
+// layer's W (A = W: output units by inputs) and, for the training step, its
+// transpose (A = W^T); one launch per layer took 3 us each.
+constexpr int kPackMax = 16;
+
+struct PackArgs {
+    struct {
+        const bf16* W;       // rows x cols, row-major
+        bf16* out;
+        int M, K;            // operand shape; A(m, k) = W[m*sm + k*sk]
+        int sm, sk, nf;
+        int64_t first;       // first chunk of this operand in the launch
+    } op[kPackMax];
+    int n_op;
+    int64_t chunks;
+};
+
+__global__ void __launch_bounds__(256) pack_weights_kernel(PackArgs a) {
     const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= chunks) return;
-    const int lane = (int)(c & 63);
-    const int64_t ti = c >> 6;
-    const int i = (int)(ti % nf), T = (int)(ti / nf);
-    const int n = 32 * T + (lane & 31), k0 = 16 * i + (lane >> 5) * 8;
+    if (c >= a.chunks) return;
+    int o = 0;
+    for (int i = 1; i < a.n_op; ++i)
+        if (c >= a.op[i].first) o = i;
+    const auto& q = a.op[o];
+    const int64_t d = c - q.first;
+    const int lane = (int)(d & 63);
+    const int64_t ti = d >> 6;
+    const int i = (int)(ti % q.nf), T = (int)(ti / q.nf);
+    const int m = 32 * T + (lane & 31), k0 = 16 * i + (lane >> 5) * 8;
     for (int j = 0; j < 8; ++j)
-        out[c * 8 + j] = (n < N && k0 + j < K) ? W[(size_t)n * K + k0 + j] : (bf16)0.0f;
+        q.out[d * 8 + j] = (m < q.M && k0 + j < q.K)
+                               ? q.W[(int64_t)m * q.sm + (int64_t)(k0 + j) * q.sk]
+                               : (bf16)0.0f;
 }
 
 __global__ void to_bf16_kernel(const float* x, bf16* y, int64_t n) {
@@ -465,7 +487,7 @@ __global__ void __launch_bounds__(256) sur_head_kernel(const float* Y, int n_out
 // workgroup, the activations resident in LDS between layers (no HBM round
 // trip). The products are taken transposed, C^T = W . act^T: the weights are
 // MFMA operand A, held in registers and loaded straight from L2 in the packed
-// order of pack_fused_kernel (A row = output column n = lane%32 of the tile,
+// order of pack_weights_kernel (A row = output column n = lane%32 of the tile,
 // k = 16i + (lane/32)*8 + j; each wave load is 1 KB contiguous), the
 // activations operand B, read from LDS (B column = row m = lane%32). Wave w
 // owns output columns [64w, 64w+64) (two 32-column tiles) of all kFRows rows
@@ -491,7 +513,7 @@ struct FusedArgs {
     const bf16* X;   // rows x n_in (bf16); unused for pairs
     int64_t rows;
     int n_in, n_out, n_mat;
-    const bf16* W[kFMaxLayers];    // layer l packed by pack_fused_kernel
+    const bf16* W[kFMaxLayers];    // layer l packed by pack_weights_kernel
     const float* b[kFMaxLayers];
     float* Y;        // rows x n_out (fp32); unused for pairs
     // pairs: the rows are the (event, module) pairs of pr (ev, mod, n_mod,
@@ -656,6 +678,8 @@ __global__ void __launch_bounds__(kFThreads, 2) mlp_fused_kernel(FusedArgs f) {
     }
 }
 
+#include "pp_train.h"
+
 int fail(int code, const std::string& msg) {
     pp_set_error_message(msg.c_str());
     return code;
@@ -682,11 +706,19 @@ struct pp_mlp {
     std::vector<int64_t> w_off, b_off;
     int64_t n_int = 0, n_params = 0;
     bool fused = true;  // inference through mlp_fused_kernel where the shape allows
-    // the fused kernel's copy of the bf16 weights (pack_fused_kernel order),
+    // the fused kernel's copy of the bf16 weights (pack_weights_kernel order),
     // refreshed by the first inference after the weights change
     bf16* wpk = nullptr;
     std::vector<int64_t> pk_off;
     bool pk_ok = false;
+    // two-launch training step (pp_train.h): the transposed packed weights
+    // (pkb_off, refreshed with wpk) and the operands of the weight gradients
+    // for ws_rows rows, allocated by the first training call
+    bf16* wpb = nullptr;
+    std::vector<int64_t> pkb_off;
+    bool pkb_ok = false;
+    bf16* ws = nullptr;
+    int64_t ws_rows = 0;
     float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
     bf16* pb = nullptr;
     // activations (max_batch rows): H[l] bf16 with dims[l] columns (H[0] = the
@@ -740,17 +772,32 @@ bool fused_ok(const pp_mlp* M) {
     return true;
 }
 
-// the fused kernel's packed copy of the bf16 weights, refreshed after a change
-int ensure_packed(pp_mlp* M) {
-    if (M->pk_ok) return PP_OK;
-    for (int l = 0; l < M->n_mat; ++l) {
-        const int K = M->dims[l], N = M->dims[l + 1];
-        const int nf = (K + 31) / 32 * 2;
-        const int64_t chunks = (M->pk_off[l + 1] - M->pk_off[l]) / 8;
-        hipLaunchKernelGGL(pack_fused_kernel, dim3(blocks_for(chunks, 256)), dim3(256), 0,
-                           M->stream, M->pb + M->w_off[l], K, N, nf, chunks, M->wpk + M->pk_off[l]);
-        PP_HIP(hipGetLastError());
-    }
+// the packed copies of the bf16 weights (train: the transposed ones too),
+// refreshed after a change
+int ensure_packed(pp_mlp* M, bool train = false) {
+    PackArgs a{};
+    auto add = [&](int l, bool transposed) {
+        auto& q = a.op[a.n_op++];
+        const int n_i = M->dims[l], n_o = M->dims[l + 1];
+        q.W = M->pb + M->w_off[l];
+        q.M = transposed ? n_i : n_o;
+        q.K = transposed ? n_o : n_i;
+        q.sm = transposed ? 1 : n_i;
+        q.sk = transposed ? n_i : 1;
+        q.nf = (q.K + 31) / 32 * 2;
+        q.out = transposed ? M->wpb + M->pkb_off[l] : M->wpk + M->pk_off[l];
+        q.first = a.chunks;
+        a.chunks += (int64_t)((q.M + 31) / 32) * q.nf * 64;
+    };
+    if (!M->pk_ok)
+        for (int l = 0; l < M->n_mat; ++l) add(l, false);
+    if (train && !(M->pk_ok && M->pkb_ok))
+        for (int l = 1; l < M->n_mat; ++l) add(l, true);
+    if (a.n_op == 0) return PP_OK;
+    hipLaunchKernelGGL(pack_weights_kernel, dim3(blocks_for(a.chunks, 256)), dim3(256), 0,
+                       M->stream, a);
+    PP_HIP(hipGetLastError());
+    M->pkb_ok = train;
     M->pk_ok = true;
     return PP_OK;
 }
@@ -898,6 +945,127 @@ int backward(pp_mlp* M, int rows) {
         dcur = bufs[nb];
         nb ^= 1;
     }
+    return PP_OK;
+}
+
+// Whether a training step runs as the two launches of pp_train.h: the shapes
+// of the fused inference kernel with at most kTMaxHidden hidden layers, and the
+// workspace for `rows` rows, which is kept (2.1 KB per row for the default
+// network). Where it does not fit device memory the step runs layer by layer.
+// Measured (batch 4096 of the 8-256x4-10 network): 347 us a step layer by layer,
+// 47 us in two launches.
+bool train_fused(pp_mlp* M, int64_t rows) {
+    if (!M->fused || !M->wpk || M->n_mat - 1 > kTMaxHidden) return false;
+    const int NL = M->n_mat - 1;
+    if (!M->wpb) {
+        M->pkb_off.assign((size_t)M->n_mat + 1, 0);
+        for (int l = 1; l < M->n_mat; ++l)
+            M->pkb_off[l + 1] = M->pkb_off[l] + (int64_t)((M->dims[l] + 31) / 32) *
+                                                    ((M->dims[l + 1] + 31) / 32 * 2) * 512;
+        if (hipMalloc((void**)&M->wpb, M->pkb_off[M->n_mat] * 2) != hipSuccess) {
+            (void)hipGetLastError();
+            M->wpb = nullptr;
+            return false;
+        }
+        M->pkb_ok = false;
+    }
+    rows = (rows + kTRows - 1) / kTRows * kTRows;
+    if (rows > M->ws_rows) {
+        if (M->ws) {
+            (void)hipStreamSynchronize(M->stream);
+            (void)hipFree(M->ws);
+        }
+        M->ws = nullptr;
+        M->ws_rows = 0;
+        if (hipMalloc((void**)&M->ws, (size_t)rows * (2 * 32 + 2 * (size_t)NL * kFH) * 2) !=
+            hipSuccess) {
+            (void)hipGetLastError();
+            M->ws = nullptr;
+            return false;
+        }
+        M->ws_rows = rows;
+    }
+    return true;
+}
+
+// Forward, loss and gradients of `rows` rows in two launches: samples drawn
+// from the dataset X, L of n rows (sample) or the rows themselves; with `opt`
+// the Adam step that follows step `step`, otherwise the gradients into M->g.
+int train_step_fused(pp_mlp* M, const float* X, const float* L, int64_t n, int rows, bool sample,
+                     uint64_t seed, uint32_t step, float* loss, const pp_adam* opt) {
+    if (int rc = ensure_packed(M, true)) return rc;
+    const int NL = M->n_mat - 1;
+    const int64_t nrb = (rows + kTRows - 1) / kTRows * 2;
+    TrainArgs a{};
+    GradArgs q{};
+    bf16* ws = M->ws;
+    auto take = [&](int cols) {
+        bf16* p = ws;
+        ws += nrb * 16 * cols;
+        return p;
+    };
+    for (int l = 0; l <= NL; ++l) {
+        a.H[l] = take(l == 0 ? 32 : kFH);
+        a.D[l] = take(l == NL ? 32 : kFH);
+        a.Wf[l] = M->wpk + M->pk_off[l];
+        a.Wb[l] = l ? M->wpb + M->pkb_off[l] : nullptr;
+        a.b[l] = M->p + M->b_off[l];
+    }
+    a.X = X;
+    a.L = L;
+    a.n = n;
+    a.rows = rows;
+    a.n_in = M->dims.front();
+    a.n_out = M->dims.back();
+    a.sample = sample;
+    a.k0 = (uint32_t)seed;
+    a.k1 = (uint32_t)(seed >> 32);
+    a.step = step;
+    a.nrb = nrb;
+    a.inv_rows = 1.0f / (float)rows;
+    a.loss = loss;
+    using RowsFn = void (*)(TrainArgs);
+    static const RowsFn kRows[kTMaxHidden] = {train_rows_kernel<1>, train_rows_kernel<2>,
+                                              train_rows_kernel<3>, train_rows_kernel<4>,
+                                              train_rows_kernel<5>, train_rows_kernel<6>};
+    hipLaunchKernelGGL(kRows[NL - 1], dim3((unsigned)(nrb / 2)), dim3(kTThreads), 0, M->stream, a);
+    PP_HIP(hipGetLastError());
+    int blocks = 0;
+    for (int l = 0; l <= NL; ++l) {
+        GradLayer& y = q.layer[l];
+        y.H = a.H[l];
+        y.D = a.D[l];
+        y.Wf = M->wpk + M->pk_off[l];
+        y.Wb = l ? M->wpb + M->pkb_off[l] : nullptr;
+        y.w_off = M->w_off[l];
+        y.b_off = M->b_off[l];
+        y.n_i = M->dims[l];
+        y.n_o = M->dims[l + 1];
+        // the slices of backward()
+        const int s = split_count(M, rows, (int64_t)y.n_o * y.n_i);
+        y.k_chunk = ((rows + s - 1) / s + kBK - 1) / kBK * kBK;
+        y.slices = (rows + y.k_chunk - 1) / y.k_chunk;
+        y.tiles_i = (y.n_i + 31) / 32;
+        y.first_w = blocks;
+        blocks += y.tiles_i * ((y.n_o + 31) / 32);
+    }
+    for (int l = 0; l <= NL; ++l) {
+        q.layer[l].first_b = blocks;
+        blocks += (M->dims[l + 1] + 31) / 32;
+    }
+    q.n_mat = M->n_mat;
+    q.rows = rows;
+    q.nrb = nrb;
+    q.update = opt != nullptr;
+    q.g = M->g;
+    q.p = M->p;
+    q.m = M->m;
+    q.v = M->v;
+    q.pb = M->pb;
+    if (opt) q.o = *opt;
+    q.step = step;
+    hipLaunchKernelGGL(train_grads_kernel, dim3((unsigned)blocks), dim3(kTThreads), 0, M->stream, q);
+    PP_HIP(hipGetLastError());
     return PP_OK;
 }
 
@@ -1088,7 +1256,7 @@ int pp_mlp_destroy(pp_mlp* M) {
     (void)hipSetDevice(M->device);
     if (M->stream) (void)hipStreamSynchronize(M->stream);
     void* ptrs[] = {M->p, M->g, M->m, M->v, M->pb, M->Y, M->dY, M->dYb, M->dA, M->dB, M->Lb, M->xs,
-                    M->part, M->wpk,
+                    M->part, M->wpk, M->wpb, M->ws,
                     M->loss, M->step, M->dsX, M->dsL, M->logy, M->hits, M->mix, M->fb,
                     M->d_ev, M->d_mod};
     for (void* p : ptrs)
@@ -1150,13 +1318,22 @@ int pp_mlp_loss_grad(pp_mlp* M, const float* x, const float* labels, int n, floa
     if (!M || !x || !labels) return fail(PP_ERR_INVALID, "pp_mlp_loss_grad: NULL argument");
     if (n < 1 || n > M->max_batch) return fail(PP_ERR_INVALID, "pp_mlp_loss_grad: n out of range");
     if (int rc = set_dev(M)) return rc;
-    if (int rc = stage_x(M, x, n)) return rc;
+    const bool two = train_fused(M, n);
+    if (two)
+        PP_HIP(hipMemcpyAsync(M->xs, x, (size_t)n * M->dims[0] * 4, hipMemcpyHostToDevice,
+                              M->stream));
+    else if (int rc = stage_x(M, x, n))
+        return rc;
     PP_HIP(hipMemcpyAsync(M->Lb, labels, (size_t)n * PP_SUR_LABEL_FLOATS * 4,
                           hipMemcpyHostToDevice, M->stream));
     PP_HIP(hipMemsetAsync(M->loss, 0, 4, M->stream));
-    if (int rc = forward(M, n, true)) return rc;
-    if (int rc = loss_head(M, n, true, false)) return rc;
-    if (int rc = backward(M, n)) return rc;
+    if (two) {
+        if (int rc = train_step_fused(M, M->xs, M->Lb, n, n, false, 0, 0, M->loss, nullptr)) return rc;
+    } else {
+        if (int rc = forward(M, n, true)) return rc;
+        if (int rc = loss_head(M, n, true, false)) return rc;
+        if (int rc = backward(M, n)) return rc;
+    }
     float l = 0.0f;
     PP_HIP(hipMemcpyAsync(&l, M->loss, 4, hipMemcpyDeviceToHost, M->stream));
     std::vector<float> gi((size_t)M->n_int);
@@ -1182,7 +1359,8 @@ int pp_mlp_train(pp_mlp* M, const float* x, const float* labels, int64_t n, int 
     if (n < 1 || batch < 1 || batch > M->max_batch || n_steps < 0)
         return fail(PP_ERR_INVALID, "pp_mlp_train: bad sizes");
     if (int rc = set_dev(M)) return rc;
-    M->pk_ok = false;  // the replayed steps update the weights
+    const bool two = train_fused(M, batch);
+    if (!two) M->pk_ok = false;  // the replayed steps update the weights
     const int n_in = M->dims[0];
     if (n > M->ds_cap) {
         if (M->dsX) PP_HIP(hipFree(M->dsX));
@@ -1203,6 +1381,22 @@ int pp_mlp_train(pp_mlp* M, const float* x, const float* labels, int64_t n, int 
     PP_HIP(hipStreamSynchronize(M->stream));
     if (int rc = ensure_loss(M, (int64_t)t0 + n_steps + 1)) return rc;
     PP_HIP(hipMemsetAsync(M->loss, 0, ((size_t)t0 + n_steps + 1) * 4, M->stream));
+    if (two) {
+        // two launches per step, which the host queues ahead of the device
+        for (int s = 0; s < n_steps; ++s)
+            if (int rc = train_step_fused(M, M->dsX, M->dsL, n, batch, true, seed, t0 + (uint32_t)s,
+                                          M->loss + t0 + s, opt)) {
+                (void)hipStreamSynchronize(M->stream);
+                return rc;
+            }
+        const uint32_t t1 = t0 + (uint32_t)n_steps;
+        PP_HIP(hipMemcpyAsync(M->step, &t1, 4, hipMemcpyHostToDevice, M->stream));
+        if (loss_curve && n_steps > 0)
+            PP_HIP(hipMemcpyAsync(loss_curve, M->loss + t0, (size_t)n_steps * 4,
+                                  hipMemcpyDeviceToHost, M->stream));
+        PP_HIP(hipStreamSynchronize(M->stream));
+        return PP_OK;
+    }
     // one training step, captured once and replayed
     GatherArgs ga{M->dsX, M->dsL, n, n_in, batch, (uint32_t)seed, (uint32_t)(seed >> 32),
                   M->step, M->H[0], M->Lb};
