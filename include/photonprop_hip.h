@@ -146,7 +146,9 @@ enum pp_search_kind { PP_SEARCH_AUTO = 0, PP_SEARCH_BRUTE = 1, PP_SEARCH_GRID = 
  *   PP_BATCH_PER_SOURCE  one launch per source
  *   PP_BATCH_PERSISTENT  one launch for the whole list: waves take chunks of
  *                        cfg.chunk_photons photons of one source from a
- *                        global counter (work stealing); with several
+ *                        global counter (work stealing; a launch of fewer than
+ *                        768 photons per resident wave deals its chunks out by
+ *                        wave index instead); with several
  *                        sources the last two chunks per resident wave go
  *                        out in pieces of 256 photons
  *   PP_BATCH_GRAPH       PP_BATCH_PERSISTENT as a hipGraph (counter clear +
@@ -177,7 +179,8 @@ typedef struct pp_config {
     int32_t batch_mode;         /* enum pp_batch_mode                          */
     int32_t chunk_photons;      /* photons per work chunk (multiple of 64);
                                    0 = auto: about 32 chunks per resident
-                                   wave, at least 256 photons                  */
+                                   wave, at least 384 photons; one chunk per
+                                   wave, or 128 photons, in a small launch     */
     float grid_cell_z;          /* grid cell edge along z (m): 0 = cubic cells
                                    (automatic shape if grid_cell is 0 too),
                                    < 0 = one layer over the targets' height

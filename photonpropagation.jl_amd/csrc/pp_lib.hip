@@ -534,6 +534,12 @@ __device__ __forceinline__ void flush_counts(const KParams& p, unsigned long lon
 #define PP_PROPAGATE_ATTRS \
     __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(PP_WAVES_PER_EU)))
 
+// x of the wave's first lane, as a scalar
+__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
+    return ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(x >> 32)) << 32) |
+           __builtin_amdgcn_readfirstlane((uint32_t)x);
+}
+
 // *p read through the constant address space: a scalar load into SGPRs for
 // a wave-uniform address (the tables the kernels read are not written
 // during a launch)
@@ -614,9 +620,10 @@ __global__ void PP_PROPAGATE_ATTRS propagate_kernel(KParams p) {
 
 // Batch of sources in one persistent launch. Work items are chunks of
 // `chunk` consecutive photons of one source (chunk_prefix[s] = first chunk
-// of source s). Each wave takes the next work item from a global counter
-// (work stealing: waves that drew cheap photons simply take more chunks)
-// and exits when the counter passes the last item, so every wave ends.
+// of source s). Each wave starts with the item of its index and then takes the
+// next one from a global counter (work stealing: waves that drew cheap photons
+// simply take more chunks) or, in a small launch (dealt), every waves-th item
+// after it, and exits past the last item, so every wave ends.
 // Chunks from split_from on are handed out as `parts` pieces of `piece`
 // photons each (the last piece of a chunk may be shorter), so that the waves
 // end closer together. Photon ids and random streams are those of the
@@ -629,6 +636,7 @@ struct BatchParams {
     uint32_t chunk;                // multiple of 64
     uint32_t parts, piece;         // pieces per split chunk; photons per piece, a multiple of 64
     uint64_t split_from;           // first split chunk (chunk_prefix[n_sources]: none)
+    bool dealt;                    // every item by wave index, none from the counter
 };
 
 template <int PHASE, int SEARCH, bool COUNT = false>
@@ -645,11 +653,11 @@ __global__ void PP_PROPAGATE_ATTRS propagate_batch_kernel(KParams p, BatchParams
     unsigned long long n_done = 0, wave_done = 0, n_steps_done = 0;
     pp::Work work;
     bool overflow = false;
+    const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+    // the first item by the wave's index
+    uint64_t next = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     for (;;) {
-        unsigned long long got = 0;
-        if (lane == 0) got = atomicAdd(&p.counters->next_chunk, 1ull);
-        const uint64_t ck = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(got >> 32)) << 32) |
-                            __builtin_amdgcn_readfirstlane((uint32_t)got);
+        const uint64_t ck = uniform64(next);
         if (ck >= total) break;
         // chunk c, photons [off, off + len) of it
         uint64_t c = ck;
@@ -704,6 +712,9 @@ __global__ void PP_PROPAGATE_ATTRS propagate_batch_kernel(KParams p, BatchParams
             }
         }
         if (__ballot(overflow)) break;  // the call fails; stop taking chunks
+        next = ck;
+        if (!b.dealt && lane == 0) next = atomicAdd(&p.counters->next_chunk, 1ull);
+        next += waves;
     }
     flush_counts<COUNT>(p, n_done, wave_done, n_steps_done, work);
 }
@@ -1212,15 +1223,25 @@ int launch_batch(pp_ctx* c, const KParams& kp, const pp_source* sources,
     int64_t max_blocks = 0;
     if (int rc = max_resident_blocks(c, (const void*)kern, block, lds, max_blocks)) return rc;
     const int64_t waves = max_blocks * (block / 64);
-    // chunk: about 32 chunks per resident wave, so that the last chunks
-    // taken leave little tail, and at least 256 photons: every grab is an
-    // atomic on one counter, and the device serves those at about one per
-    // 12 ns (a 1e8-photon launch of 192-photon chunks took 6.7 ms on them
-    // alone; 5.2 ms with 512)
+    // Chunks of a small launch are dealt out: wave i takes items i, i + waves, ...
+    // and no counter is touched (the device serves its atomics at about one per
+    // 12 ns, so that 64-photon chunks from the counter cost more than their
+    // photons, and the 256-photon chunks taken before left most waves idle).
+    // One item per wave up to 256 photons, then 128-photon items. Large launches
+    // take theirs from the counter, since waves progress at rates that differ by
+    // a quarter (1e8-photon cascade: 7.6 ms taken, 9.7 ms dealt): about 32
+    // chunks per resident wave, at least 384 photons. The line lies where the
+    // two meet, at about 768 photons per wave (README point source, then
+    // cascade: 3e6 photons 0.209 / 0.329 ms dealt, 0.261 / 0.358 taken; 1e7
+    // photons 0.651 / 1.02 and 0.656 / 0.93).
     uint64_t chunk = (uint64_t)c->cfg.chunk_photons;
+    const uint64_t per_wave = total_ph / (uint64_t)waves;
+    const bool dealt = per_wave < 768;
     if (chunk == 0) {
-        chunk = total_ph / ((uint64_t)waves * 32) / 64 * 64;
-        chunk = std::min<uint64_t>(std::max<uint64_t>(chunk, 256), 8192);
+        if (dealt)
+            chunk = per_wave < 256 ? (per_wave / 64 + 1) * 64 : 128;
+        else
+            chunk = std::min<uint64_t>(std::max<uint64_t>(per_wave / 32 / 64 * 64, 384), 8192);
     }
     // table: sources | photon counts | chunk prefix, each 256-byte aligned
     const size_t off_n = ((n * sizeof(pp_source)) + 255) & ~(size_t)255;
@@ -1252,7 +1273,7 @@ int launch_batch(pp_ctx* c, const KParams& kp, const pp_source* sources,
     bp.piece = (uint32_t)chunk;
     bp.parts = 1;
     bp.split_from = n_chunks;
-    if (n > 1) {
+    if (n > 1 && !dealt) {
         bp.piece = (uint32_t)std::min<uint64_t>(chunk, 256);
         bp.parts = (uint32_t)((chunk + bp.piece - 1) / bp.piece);
         const uint64_t tail = (uint64_t)waves * 2;
@@ -1261,6 +1282,7 @@ int launch_batch(pp_ctx* c, const KParams& kp, const pp_source* sources,
     const uint64_t n_items = bp.split_from + (n_chunks - bp.split_from) * bp.parts;
     const int64_t want = (int64_t)((n_items + block / 64 - 1) / (block / 64));
     const unsigned blocks = (unsigned)std::min<int64_t>(want, max_blocks);
+    bp.dealt = dealt;
     PP_HIP(hipMemcpyAsync(c->d_batch, c->h_batch, bytes, hipMemcpyHostToDevice, c->stream));
     if (!use_graph) {
         PP_HIP(hipMemsetAsync(c->d_counters, 0, sizeof(Counters), c->stream));
