@@ -25,6 +25,7 @@
 #include "photonprop_surrogate.h"
 #include "pp_device.h"
 #include "pp_hits.h"
+#include "pp_stage.h"
 
 // pp_device.h turns contraction off for the propagation step functions; the
 // network's epilogues (bias, SiLU, Adam, loss) contract products and sums into
@@ -643,7 +644,7 @@ __global__ void __launch_bounds__(kFThreads, 2) mlp_fused_kernel(FusedArgs f) {
             if (row < f.rows) {
                 float feat[PP_SUR_N_FEATURES];
                 bool fb;
-                pair_row(f.pr, row, feat, logy[t], fb);
+                pair_row(f.pr, f.pr.row0 + row, feat, logy[t], fb);
                 f.pr.fb[row] = fb;
                 for (int k = 0; k < 32; ++k)
                     a[k] = k < f.n_in ? (bf16)(k < PP_SUR_N_FEATURES ? feat[k] : 0.0f) : (bf16)0.0f;
@@ -678,6 +679,135 @@ __global__ void __launch_bounds__(kFThreads, 2) mlp_fused_kernel(FusedArgs f) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// A 32-row tile by eight waves, wave w owning units [32w, 32w + 32) of a layer:
+// the form of the small inference launches and of the training step
+// (pp_train.h). The wave's weights of a layer are 16 fragments in registers.
+// ---------------------------------------------------------------------------
+constexpr int kTRows = 32;      // rows per workgroup: one MFMA row tile
+constexpr int kTThreads = 512;  // eight waves
+
+template <int NF>
+__device__ __forceinline__ void load_weights(const bf16* W, int tile, int lane, bf16x8 (&f)[kFFrag]) {
+    const bf16x8* src = reinterpret_cast<const bf16x8*>(W) + (size_t)tile * NF * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < NF; ++i) f[i] = src[i * 64];
+}
+
+// acc += W . act^T over NF fragments, K ascending (weights operand A, rows operand B)
+template <int NF>
+__device__ __forceinline__ f32x16 tile_product(f32x16 acc, const bf16x8 (&f)[kFFrag],
+                                               const bf16* act, int lane) {
+    const bf16* src = act + (lane & 31) * kFActLd + (lane >> 5) * 8;
+#pragma unroll
+    for (int i = 0; i < NF; ++i)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            f[i], *reinterpret_cast<const bf16x8*>(src + 16 * i), acc, 0, 0, 0);
+    return acc;
+}
+
+// The accumulator's bias block: entry 4g + j is unit unit0 + 8g + (lane/32)*4 + j
+__device__ __forceinline__ f32x16 bias_block(const float* b, int unit0, int n, int lane) {
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int u = unit0 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+        acc[r] = u < n ? b[u] : 0.0f;
+    }
+    return acc;
+}
+
+// SiLU activations of an accumulator into a [32 rows][kFActLd] LDS tile
+__device__ __forceinline__ void store_silu(const f32x16& acc, bf16* out, int w, int lane) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        bf16 h[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) h[j] = (bf16)(acc[4 * g + j] * sigmoid(acc[4 * g + j]));
+        *reinterpret_cast<uint2*>(out + (lane & 31) * kFActLd + 32 * w + 8 * g + (lane >> 5) * 4) =
+            *reinterpret_cast<const uint2*>(h);
+    }
+}
+
+// Inference of few rows: the network for a 32-row tile per workgroup of eight
+// waves, with mlp_fused_kernel's values (same products, order and epilogues).
+// A small list is bound by the latency of one tile: the 128-row tiles of
+// mlp_fused_kernel put 1000 pairs on 8 CUs, and each of their waves computes
+// eight times the products of a wave here. The next layer's weights are loaded
+// while a layer is computed. More rows than the CUs hold at one tile each make
+// the weight stream (128 KB per layer and tile) the bound.
+template <bool PAIRS>
+__global__ void __launch_bounds__(kTThreads) mlp_small_kernel(FusedArgs f) {
+    __shared__ __attribute__((aligned(16))) bf16 act[2][kTRows * kFActLd];
+    __shared__ float yv[kTRows][33];
+    __shared__ float logy[kTRows];
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int64_t row0 = (int64_t)blockIdx.x * kTRows;
+    const int valid = f.rows - row0 < kTRows ? (int)(f.rows - row0) : kTRows;
+    const int top = f.n_mat - 1;
+    bf16x8 wn[kFFrag], wc[kFFrag];
+    load_weights<2>(f.W[0], w, lane, wn);
+    if (PAIRS) {
+        if (t < kTRows) {
+            bf16* a = act[0] + t * kFActLd;
+            float feat[PP_SUR_N_FEATURES];
+            if (t < valid) {
+                bool fb;
+                pair_row(f.pr, f.pr.row0 + row0 + t, feat, logy[t], fb);
+                f.pr.fb[row0 + t] = fb;
+            }
+#pragma unroll
+            for (int k = 0; k < 32; ++k)
+                a[k] = k < PP_SUR_N_FEATURES && k < f.n_in && t < valid
+                           ? (bf16)feat[k < PP_SUR_N_FEATURES ? k : 0] : (bf16)0.0f;
+        }
+    } else {
+        for (int i = t; i < kTRows * 32; i += kTThreads) {
+            const int r = i >> 5, k = i & 31;
+            act[0][r * kFActLd + k] =
+                r < valid && k < f.n_in ? f.X[(row0 + r) * f.n_in + k] : (bf16)0.0f;
+        }
+    }
+    __syncthreads();
+    f32x16 acc = bias_block(f.b[0], 32 * w, kFH, lane);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) wc[i] = wn[i];
+    if (top > 1 || w == 0) load_weights<kFFrag>(f.W[1], top > 1 ? w : 0, lane, wn);
+    __builtin_amdgcn_sched_barrier(0);
+    acc = tile_product<2>(acc, wc, act[0], lane);
+    store_silu(acc, act[1], w, lane);
+    __syncthreads();
+    for (int l = 1; l < top; ++l) {
+        acc = bias_block(f.b[l], 32 * w, kFH, lane);
+#pragma unroll
+        for (int i = 0; i < kFFrag; ++i) wc[i] = wn[i];
+        if (l + 1 < top || w == 0) load_weights<kFFrag>(f.W[l + 1], l + 1 < top ? w : 0, lane, wn);
+        __builtin_amdgcn_sched_barrier(0);
+        acc = tile_product<kFFrag>(acc, wc, act[l & 1], lane);
+        store_silu(acc, act[(l + 1) & 1], w, lane);
+        __syncthreads();
+    }
+    if (w == 0) {
+        acc = bias_block(f.b[top], 0, f.n_out, lane);
+        acc = tile_product<kFFrag>(acc, wn, act[top & 1], lane);
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            yv[lane & 31][(r >> 2) * 8 + (lane >> 5) * 4 + (r & 3)] = acc[r];
+    }
+    __syncthreads();
+    if (PAIRS) {
+        if (t < valid) {
+            const int64_t row = row0 + t;
+            sur_head_row(yv[t], logy[t], f.hits + row, f.mix ? f.mix + row * 9 : nullptr);
+        }
+    } else {
+        for (int i = t; i < valid * f.n_out; i += kTThreads) {
+            const int r = i / f.n_out, c = i - r * f.n_out;
+            f.Y[row0 * f.n_out + i] = yv[r][c];
+        }
+    }
+}
+
 #include "pp_train.h"
 
 int fail(int code, const std::string& msg) {
@@ -697,9 +827,8 @@ unsigned blocks_for(int64_t n, int per) { return (unsigned)((n + per - 1) / per)
 }  // namespace
 
 struct pp_mlp {
-    int device = 0;
+    int device = 0, n_cu = 0;
     hipStream_t stream = nullptr;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::vector<int> dims;  // n_in, hidden..., n_out
     int n_mat = 0, max_batch = 0;
     // parameters: internal layout with every block at a 64-element boundary
@@ -739,15 +868,16 @@ struct pp_mlp {
     // training set
     float *dsX = nullptr, *dsL = nullptr;
     int64_t ds_cap = 0;
-    // pair evaluation
+    // pair evaluation: events | modules, the outputs of two slices of the list,
+    // the stream their copies run on and the slices' events
+    char* d_in = nullptr;
+    size_t in_cap = 0;
+    char* d_out = nullptr;
+    size_t out_cap = 0;
+    hipStream_t copy = nullptr;
+    hipEvent_t t0[2] = {nullptr, nullptr}, t1[2] = {nullptr, nullptr};
     float* logy = nullptr;
-    float* hits = nullptr;
-    float* mix = nullptr;
-    uint8_t* fb = nullptr;
-    int64_t out_cap = 0;
-    pp_cascade* d_ev = nullptr;
-    float* d_mod = nullptr;
-    int64_t ev_cap = 0, mod_cap = 0;
+    pp::PinnedPair pin;  // results on their way to pageable host memory
 };
 
 namespace {
@@ -820,15 +950,19 @@ int forward_fused(pp_mlp* M, int64_t rows, const PairArgs* pairs = nullptr, floa
         f.b[l] = M->p + M->b_off[l];
     }
     f.Y = M->Y;
-    const dim3 grid(blocks_for(rows, kFRows));
     if (pairs) {
         f.pr = *pairs;
         f.hits = hits;
         f.mix = mix;
-        hipLaunchKernelGGL(mlp_fused_kernel<true>, grid, dim3(kFThreads), 0, M->stream, f);
-    } else {
-        hipLaunchKernelGGL(mlp_fused_kernel<false>, grid, dim3(kFThreads), 0, M->stream, f);
     }
+    // one 32-row tile per CU at most takes the small kernel (10 us for up to
+    // 8192 pairs against 20 us in 128-row tiles); at 12000 pairs, two tiles on
+    // some CUs, the two are equal, and beyond it the larger tiles win
+    const bool small = rows <= (int64_t)M->n_cu * kTRows;
+    const auto fn = small ? (pairs ? mlp_small_kernel<true> : mlp_small_kernel<false>)
+                          : (pairs ? mlp_fused_kernel<true> : mlp_fused_kernel<false>);
+    hipLaunchKernelGGL(fn, dim3(blocks_for(rows, small ? kTRows : kFRows)),
+                       dim3(small ? kTThreads : kFThreads), 0, M->stream, f);
     PP_HIP(hipGetLastError());
     return PP_OK;
 }
@@ -947,6 +1081,9 @@ int backward(pp_mlp* M, int rows) {
     }
     return PP_OK;
 }
+
+constexpr int64_t kPairSlice = (int64_t)1 << 18;  // pairs per slice of a list
+constexpr size_t kPairPinnedIn = 256 << 10;       // inputs that go through pinned memory (bytes)
 
 // Whether a training step runs as the two launches of pp_train.h: the shapes
 // of the fused inference kernel with at most kTMaxHidden hidden layers, and the
@@ -1183,7 +1320,8 @@ int pp_mlp_create(pp_mlp** out, int device, int n_in, int n_hidden, int n_layers
     M->n_int = o;
     if (hipSetDevice(device) != hipSuccess) return bail(fail(PP_ERR_HIP, "hipSetDevice failed"));
     if (hipStreamCreateWithFlags(&M->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreate(&M->ev0) != hipSuccess || hipEventCreate(&M->ev1) != hipSuccess)
+        hipEventCreate(&M->t0[0]) != hipSuccess || hipEventCreate(&M->t1[0]) != hipSuccess ||
+        hipDeviceGetAttribute(&M->n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
         return bail(fail(PP_ERR_HIP, "pp_mlp_create: stream/event creation failed"));
     auto alloc = [&](void** p, size_t bytes) { return hipMalloc(p, std::max<size_t>(bytes, 256)); };
     const size_t rows = (size_t)max_batch;
@@ -1255,18 +1393,21 @@ int pp_mlp_destroy(pp_mlp* M) {
     if (!M) return PP_OK;
     (void)hipSetDevice(M->device);
     if (M->stream) (void)hipStreamSynchronize(M->stream);
+    if (M->copy) (void)hipStreamSynchronize(M->copy);
     void* ptrs[] = {M->p, M->g, M->m, M->v, M->pb, M->Y, M->dY, M->dYb, M->dA, M->dB, M->Lb, M->xs,
                     M->part, M->wpk, M->wpb, M->ws,
-                    M->loss, M->step, M->dsX, M->dsL, M->logy, M->hits, M->mix, M->fb,
-                    M->d_ev, M->d_mod};
+                    M->loss, M->step, M->dsX, M->dsL, M->logy, M->d_in,
+                    M->d_out};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto* p : M->H)
         if (p) (void)hipFree(p);
     for (auto* p : M->Z)
         if (p) (void)hipFree(p);
-    if (M->ev0) (void)hipEventDestroy(M->ev0);
-    if (M->ev1) (void)hipEventDestroy(M->ev1);
+    M->pin.release();
+    for (hipEvent_t e : {M->t0[0], M->t0[1], M->t1[0], M->t1[1]})
+        if (e) (void)hipEventDestroy(e);
+    if (M->copy) (void)hipStreamDestroy(M->copy);
     if (M->stream) (void)hipStreamDestroy(M->stream);
     delete M;
     return PP_OK;
@@ -1284,8 +1425,7 @@ int pp_mlp_get_params(pp_mlp* M, float* params) {
     if (!M || !params) return fail(PP_ERR_INVALID, "pp_mlp_get_params: NULL argument");
     if (int rc = set_dev(M)) return rc;
     std::vector<float> internal((size_t)M->n_int);
-    PP_HIP(hipMemcpyAsync(internal.data(), M->p, M->n_int * 4, hipMemcpyDeviceToHost, M->stream));
-    PP_HIP(hipStreamSynchronize(M->stream));
+    PP_HIP(M->pin.copy_out(M->stream, internal.data(), M->p, M->n_int * 4));
     pack_params(M, internal, params);
     return PP_OK;
 }
@@ -1307,9 +1447,7 @@ int pp_mlp_forward(pp_mlp* M, const float* x, int n, float* y) {
     if (int rc = set_dev(M)) return rc;
     if (int rc = stage_x(M, x, n)) return rc;
     if (int rc = forward(M, n, false)) return rc;
-    PP_HIP(hipMemcpyAsync(y, M->Y, (size_t)n * M->dims.back() * 4, hipMemcpyDeviceToHost,
-                          M->stream));
-    PP_HIP(hipStreamSynchronize(M->stream));
+    PP_HIP(M->pin.copy_out(M->stream, y, M->Y, (size_t)n * M->dims.back() * 4));
     return PP_OK;
 }
 
@@ -1337,8 +1475,7 @@ int pp_mlp_loss_grad(pp_mlp* M, const float* x, const float* labels, int n, floa
     float l = 0.0f;
     PP_HIP(hipMemcpyAsync(&l, M->loss, 4, hipMemcpyDeviceToHost, M->stream));
     std::vector<float> gi((size_t)M->n_int);
-    if (grads)
-        PP_HIP(hipMemcpyAsync(gi.data(), M->g, M->n_int * 4, hipMemcpyDeviceToHost, M->stream));
+    if (grads) PP_HIP(M->pin.copy_out(M->stream, gi.data(), M->g, M->n_int * 4));
     PP_HIP(hipStreamSynchronize(M->stream));
     if (loss) *loss = l;
     if (grads) pack_params(M, gi, grads);
@@ -1528,78 +1665,120 @@ int pp_sur_eval_pairs(pp_mlp* M, const pp_cascade* events, int n_events, const f
     const int64_t n = (int64_t)n_events * n_modules;
     if (n == 0) return PP_OK;
     if (int rc = set_dev(M)) return rc;
-    // device outputs for all pairs, inputs per event / module
-    if (n > M->out_cap) {
-        for (void** p : {(void**)&M->hits, (void**)&M->mix, (void**)&M->fb, (void**)&M->logy})
-            if (*p) {
-                PP_HIP(hipFree(*p));
-                *p = nullptr;
-            }
-        M->out_cap = 0;
-        PP_HIP(hipMalloc(&M->hits, n * 4));
-        PP_HIP(hipMalloc(&M->mix, n * 9 * 4));
-        PP_HIP(hipMalloc(&M->fb, n));
-        PP_HIP(hipMalloc(&M->logy, (size_t)M->max_batch * 4));
-        M->out_cap = n;
+    // Lists of up to kPairSlice pairs run at once; longer ones in slices, whose
+    // results go to pinned memory on a stream of their own and from there to the
+    // caller while the next slice is computed (5e6 pairs: 4.2 ms with the copies
+    // after the kernel, 2.9 ms sliced). A slice is a whole number of rounds of
+    // the 128-row tiles (two per CU), so that no CU waits for the last of them.
+    const bool fused = M->fused && M->wpk;
+    const int64_t slice = std::min<int64_t>(n, fused ? kPairSlice : std::min<int64_t>(kPairSlice,
+                                                                                     M->max_batch));
+    const size_t off_mod = ((size_t)n_events * sizeof(pp_cascade) + 255) & ~(size_t)255;
+    const size_t in_b = off_mod + (size_t)n_modules * 12;
+    const size_t off_mix = (size_t)slice * 4;
+    const size_t off_fb = off_mix + (mixture ? (size_t)slice * 36 : 0);
+    const size_t out_b = (off_fb + (size_t)slice + 255) & ~(size_t)255;
+    const int n_buf = slice < n ? 2 : 1;
+    auto grow = [&](char** p, size_t* cap, size_t need) -> int {
+        if (need <= *cap) return PP_OK;
+        if (*p) PP_HIP(hipFree(*p));
+        *p = nullptr;
+        *cap = 0;
+        PP_HIP(hipMalloc((void**)p, need));
+        *cap = need;
+        return PP_OK;
+    };
+    if (int rc = grow(&M->d_in, &M->in_cap, in_b)) return rc;
+    if (int rc = grow(&M->d_out, &M->out_cap, out_b * n_buf)) return rc;
+    if (!fused && !M->logy) PP_HIP(hipMalloc(&M->logy, (size_t)M->max_batch * 4));
+    if (n_buf == 2 && !M->copy) {
+        PP_HIP(hipStreamCreateWithFlags(&M->copy, hipStreamNonBlocking));
+        PP_HIP(hipEventCreate(&M->t0[1]));
+        PP_HIP(hipEventCreate(&M->t1[1]));
     }
-    if (n_events > M->ev_cap) {
-        if (M->d_ev) PP_HIP(hipFree(M->d_ev));
-        M->d_ev = nullptr;
-        PP_HIP(hipMalloc(&M->d_ev, (size_t)n_events * sizeof(pp_cascade)));
-        M->ev_cap = n_events;
+    PP_HIP(M->pin.ensure(std::max(out_b, in_b <= kPairPinnedIn ? in_b : (size_t)0)));
+    auto* d_ev = (pp_cascade*)M->d_in;
+    auto* d_mod = (float*)(M->d_in + off_mod);
+    if (in_b <= kPairPinnedIn) {  // one copy from pinned memory
+        std::memcpy(M->pin.at(1), events, (size_t)n_events * sizeof(pp_cascade));
+        std::memcpy(M->pin.at(1) + off_mod, module_xyz, (size_t)n_modules * 12);
+        PP_HIP(hipMemcpyAsync(M->d_in, M->pin.at(1), in_b, hipMemcpyHostToDevice, M->stream));
+    } else {
+        PP_HIP(hipMemcpyAsync(d_ev, events, (size_t)n_events * sizeof(pp_cascade),
+                              hipMemcpyHostToDevice, M->stream));
+        PP_HIP(hipMemcpyAsync(d_mod, module_xyz, (size_t)n_modules * 12, hipMemcpyHostToDevice,
+                              M->stream));
     }
-    if (n_modules > M->mod_cap) {
-        if (M->d_mod) PP_HIP(hipFree(M->d_mod));
-        M->d_mod = nullptr;
-        PP_HIP(hipMalloc(&M->d_mod, (size_t)n_modules * 12));
-        M->mod_cap = n_modules;
-    }
-    PP_HIP(hipMemcpyAsync(M->d_ev, events, (size_t)n_events * sizeof(pp_cascade),
-                          hipMemcpyHostToDevice, M->stream));
-    PP_HIP(hipMemcpyAsync(M->d_mod, module_xyz, (size_t)n_modules * 12, hipMemcpyHostToDevice,
-                          M->stream));
-    PP_HIP(hipEventRecord(M->ev0, M->stream));
-    if (M->fused && M->wpk) {
-        // one launch over every pair: features, network and head in one kernel
+    const hipStream_t out_stream = n_buf == 2 ? M->copy : M->stream;
+    float device_ms = 0.0f;
+    // the slice's launches and, behind them, the copy of its results
+    auto start = [&](int64_t k) -> int {
+        const int b = (int)(k & 1);
+        const int64_t r0 = k * slice;
+        const int64_t rows = std::min<int64_t>(slice, n - r0);
+        char* out = M->d_out + (n_buf == 2 ? b : 0) * out_b;
         PairArgs a{};
-        a.ev = M->d_ev;
-        a.mod = M->d_mod;
-        a.n_mod = n_modules;
-        a.rows = n;
-        a.n_in = M->dims[0];
-        a.fb = M->fb;
-        a.dom = *dom;
-        if (int rc = forward_fused(M, n, &a, M->hits, mixture ? M->mix : nullptr)) return rc;
-    }
-    for (int64_t r0 = 0; !(M->fused && M->wpk) && r0 < n; r0 += M->max_batch) {
-        const int rows = (int)std::min<int64_t>(M->max_batch, n - r0);
-        PairArgs a{};
-        a.ev = M->d_ev;
-        a.mod = M->d_mod;
+        a.ev = d_ev;
+        a.mod = d_mod;
         a.n_mod = n_modules;
         a.row0 = r0;
         a.rows = rows;
         a.n_in = M->dims[0];
-        a.xb = M->H[0];
-        a.logy = M->logy;
-        a.fb = M->fb + r0;
+        a.fb = (uint8_t*)(out + off_fb);
         a.dom = *dom;
-        hipLaunchKernelGGL(pair_features_kernel, dim3(blocks_for(rows, 256)), dim3(256), 0,
-                           M->stream, a);
-        PP_HIP(hipGetLastError());
-        if (int rc = forward(M, rows, false)) return rc;
-        hipLaunchKernelGGL(sur_head_kernel, dim3(blocks_for(rows, 256)), dim3(256), 0, M->stream,
-                           M->Y, M->dims.back(), (int64_t)rows, M->logy, M->hits + r0,
-                           mixture ? M->mix + r0 * 9 : nullptr);
-        PP_HIP(hipGetLastError());
+        float* hits = (float*)out;
+        float* mix = mixture ? (float*)(out + off_mix) : nullptr;
+        PP_HIP(hipEventRecord(M->t0[b], M->stream));
+        if (fused) {
+            // features, network and head in one kernel
+            if (int rc = forward_fused(M, rows, &a, hits, mix)) return rc;
+        } else {
+            a.xb = M->H[0];
+            a.logy = M->logy;
+            hipLaunchKernelGGL(pair_features_kernel, dim3(blocks_for(rows, 256)), dim3(256), 0,
+                               M->stream, a);
+            PP_HIP(hipGetLastError());
+            if (int rc = forward(M, (int)rows, false)) return rc;
+            hipLaunchKernelGGL(sur_head_kernel, dim3(blocks_for(rows, 256)), dim3(256), 0,
+                               M->stream, M->Y, M->dims.back(), rows, M->logy, hits, mix);
+            PP_HIP(hipGetLastError());
+        }
+        PP_HIP(hipEventRecord(M->t1[b], M->stream));
+        if (n_buf == 2) PP_HIP(hipStreamWaitEvent(M->copy, M->t1[b], 0));
+        PP_HIP(hipMemcpyAsync(M->pin.at(b), out, out_b, hipMemcpyDeviceToHost, out_stream));
+        PP_HIP(hipEventRecord(M->pin.ev[b], out_stream));
+        return PP_OK;
+    };
+    // the slice's results to the caller
+    auto finish = [&](int64_t k) -> int {
+        const int b = (int)(k & 1);
+        const int64_t r0 = k * slice;
+        const size_t rows = (size_t)std::min<int64_t>(slice, n - r0);
+        PP_HIP(hipEventSynchronize(M->pin.ev[b]));
+        const char* src = M->pin.at(b);
+        std::memcpy(expected_hits + r0, src, rows * 4);
+        if (mixture) std::memcpy(mixture + r0 * 9, src + off_mix, rows * 36);
+        if (fallback) std::memcpy(fallback + r0, src + off_fb, rows);
+        if (kernel_ms) {
+            float ms = 0.0f;
+            PP_HIP(hipEventElapsedTime(&ms, M->t0[b], M->t1[b]));
+            device_ms += ms;
+        }
+        return PP_OK;
+    };
+    const int64_t slices = (n + slice - 1) / slice;
+    int rc = PP_OK;
+    // the second pinned half holds the inputs until the first slice has run
+    for (int64_t k = 0; k <= slices && rc == PP_OK; ++k) {
+        if (k < slices) rc = start(k);
+        if (k > 0 && rc == PP_OK) rc = finish(k - 1);
     }
-    PP_HIP(hipEventRecord(M->ev1, M->stream));
-    PP_HIP(hipMemcpyAsync(expected_hits, M->hits, n * 4, hipMemcpyDeviceToHost, M->stream));
-    if (mixture)
-        PP_HIP(hipMemcpyAsync(mixture, M->mix, n * 9 * 4, hipMemcpyDeviceToHost, M->stream));
-    if (fallback) PP_HIP(hipMemcpyAsync(fallback, M->fb, n, hipMemcpyDeviceToHost, M->stream));
-    PP_HIP(hipStreamSynchronize(M->stream));
-    if (kernel_ms) PP_HIP(hipEventElapsedTime(kernel_ms, M->ev0, M->ev1));
+    if (rc != PP_OK) {  // nothing may still use the workspace
+        (void)hipStreamSynchronize(M->stream);
+        if (M->copy) (void)hipStreamSynchronize(M->copy);
+        return rc;
+    }
+    if (kernel_ms) *kernel_ms = device_ms;
     return PP_OK;
 }
 

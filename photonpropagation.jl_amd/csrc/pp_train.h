@@ -18,8 +18,6 @@
 // slices of the batch summed in the same order, the same epilogues, and the
 // loss's sums over the bins taken bin by bin.
 
-constexpr int kTRows = 32;      // rows per workgroup: one MFMA row tile, 128 workgroups at 4096
-constexpr int kTThreads = 512;  // eight waves; wave w owns units [32w, 32w + 32) of every layer
 constexpr int kTMaxHidden = 6;  // hidden layers (their pre-activations stay in registers)
 
 // Row operands of the weight gradients, H (a layer's input) and D (the gradient
@@ -65,36 +63,6 @@ __device__ __forceinline__ void store_operand(const bf16* act, bf16* out, int ti
         *reinterpret_cast<uint4*>(out + ((tile * nrb + rb0 + half) * 64 + lane) * 8) =
             *reinterpret_cast<const uint4*>(v);
     }
-}
-
-template <int NF>
-__device__ __forceinline__ void load_weights(const bf16* W, int tile, int lane, bf16x8 (&f)[kFFrag]) {
-    const bf16x8* src = reinterpret_cast<const bf16x8*>(W) + (size_t)tile * NF * 64 + lane;
-#pragma unroll
-    for (int i = 0; i < NF; ++i) f[i] = src[i * 64];
-}
-
-// acc += W . act^T over NF fragments, K ascending (weights operand A, rows operand B)
-template <int NF>
-__device__ __forceinline__ f32x16 tile_product(f32x16 acc, const bf16x8 (&f)[kFFrag],
-                                               const bf16* act, int lane) {
-    const bf16* src = act + (lane & 31) * kFActLd + (lane >> 5) * 8;
-#pragma unroll
-    for (int i = 0; i < NF; ++i)
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            f[i], *reinterpret_cast<const bf16x8*>(src + 16 * i), acc, 0, 0, 0);
-    return acc;
-}
-
-// The accumulator's bias block: entry 4g + j is unit unit0 + 8g + (lane/32)*4 + j
-__device__ __forceinline__ f32x16 bias_block(const float* b, int unit0, int n, int lane) {
-    f32x16 acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int u = unit0 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-        acc[r] = u < n ? b[u] : 0.0f;
-    }
-    return acc;
 }
 
 // One workgroup: 32 rows of the batch through the forward pass, the loss and
@@ -160,14 +128,7 @@ __global__ void __launch_bounds__(kTThreads) train_rows_kernel(TrainArgs a) {
         __builtin_amdgcn_sched_barrier(0);
         acc = l == 0 ? tile_product<2>(acc, wc, in, lane) : tile_product<kFFrag>(acc, wc, in, lane);
         z[l] = acc;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            bf16 h[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) h[j] = (bf16)(acc[4 * g + j] * sigmoid(acc[4 * g + j]));
-            *reinterpret_cast<uint2*>(out + (lane & 31) * kFActLd + 32 * w + 8 * g +
-                                      (lane >> 5) * 4) = *reinterpret_cast<const uint2*>(h);
-        }
+        store_silu(acc, out, w, lane);
         store_operand(in, a.H[l], l == 0 ? 1 : kFH / 32, a.nrb, rb0, valid);
         __syncthreads();
     }
