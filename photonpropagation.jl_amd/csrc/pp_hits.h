@@ -34,6 +34,15 @@ struct PmtSetup {
     float inv_s2[2];
     int32_t n_wl;
     uint32_t k0, k1;
+    bool acc_ok;  // every acceptance is >= 0
+};
+
+// Constants of the detection kernel's approximate weights, per PMT group.
+struct PmtFast {
+    float k2[2];     // -log2(e) / (2 sigma^2)
+    float scale[2];  // 1 / (4 sigma^2)
+    float far[2];    // bound of the far PMTs' summed weight per unit of acceptance
+    float rel;       // bound of a weight's relative error
 };
 
 // Validates the model and its acceptance table and fills `s` and the table

@@ -75,9 +75,41 @@ struct PmtRecords {
     }
 };
 
+// The 16 PMT directions are 8 antipodal pairs of one group each: PMT j and
+// kAntipode[j], j < 8 (the layout of pom_angles; fast_setup checks it).
+constexpr int kAntipode[8] = {11, 10, 9, 8, 14, 13, 12, 15};
+
+// Constants of the approximate weights (pmt_fast) of a set-up; false where
+// they do not serve: directions that are not antipodal pairs to 1e-6, a
+// negative acceptance, or widths whose error bounds leave too much to evaluate in full (sigma below 0.02 or,
+// with its far PMTs' weights, above 0.4 or so). With k = 1 / (2 sigma^2), a
+// weight's relative error has three parts: the cosine, off by 2.5e-7 at most in
+// either evaluation, times d ln p / dc <= pi k + 2; the fit of acos, 2e-7 times
+// 1 + 2 k pt^2 <= 1 + 5 k; and 1e-5 for the roundings of both evaluations.
+bool fast_setup(const pp::PmtSetup& s, pp::PmtFast* f) {
+    if (!s.acc_ok) return false;
+    for (int j = 0; j < 8; ++j)
+        for (int r = 0; r < 3; ++r)
+            if (!(std::fabs(s.dir[j][r] + s.dir[kAntipode[j]][r]) <= 1e-6f)) return false;
+    f->rel = 0.0f;
+    for (int g = 0; g < 2; ++g) {
+        const double k = 0.5 * s.inv_s2[g];
+        f->k2[g] = (float)(-k * 1.4426950408889634);
+        f->scale[g] = s.inv_s2[g] * 0.25f;
+        f->rel = std::max(f->rel, (float)(2.5e-7 * (M_PI * k + 2.0) + 2e-7 * (1.0 + 5.0 * k) + 1e-5));
+        // four far PMTs a group, each at most pt exp(-k pt^2) / sin(pt) per unit
+        // of scale and acceptance: up to 3 pi/4, and from there to the pole that
+        // is left out (sin pt >= 1.41e-3)
+        const double most = std::max(3.34 * std::exp(-2.467 * k), 2222.0 * std::exp(-5.55 * k));
+        f->far[g] = (float)(4.0 * 0.25 * s.inv_s2[g] * most);
+    }
+    return f->rel <= 1e-3f && f->far[0] <= 1e-3f && f->far[1] <= 1e-3f;
+}
+
 template <typename In>
 struct PmtArgs {
     pp::PmtSetup s;
+    pp::PmtFast f;
     const float* tab;  // wl | acc1 | acc2, n_wl each
     In in;
     int64_t n;
@@ -85,9 +117,12 @@ struct PmtArgs {
     unsigned long long* n_det;
 };
 
-// linear interpolation in a sorted table, 0 outside (extrapolation_bc = 0)
-__device__ __forceinline__ float interp0(const float* x, const float* y, int n, float v) {
-    if (!(v >= x[0] && v <= x[n - 1])) return 0.0f;
+// Both groups' acceptances: linear interpolation in a sorted table, 0 outside
+// (extrapolation_bc = 0)
+__device__ __forceinline__ void interp0(const float* x, const float* y1, const float* y2, int n,
+                                        float v, float* acc) {
+    acc[0] = acc[1] = 0.0f;
+    if (!(v >= x[0] && v <= x[n - 1])) return;
     int lo = 0, hi = n - 1;
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
@@ -95,13 +130,117 @@ __device__ __forceinline__ float interp0(const float* x, const float* y, int n, 
         else hi = mid;
     }
     const float t = (v - x[lo]) / (x[hi] - x[lo]);
-    return y[lo] + t * (y[hi] - y[lo]);
+    acc[0] = y1[lo] + t * (y1[hi] - y1[lo]);
+    acc[1] = y2[lo] + t * (y2[hi] - y2[lo]);
+}
+
+// Weight of PMT j for a hit at p (see the header): the reference value of every
+// decision below
+__device__ __forceinline__ float pmt_weight(const pp::PmtSetup& s, int j, float px, float py,
+                                            float pz, const float* acc) {
+    const int g = (j >> 2) & 1;
+    const float c = fminf(fmaxf(px * s.dir[j][0] + py * s.dir[j][1] + pz * s.dir[j][2], -1.0f), 1.0f);
+    const float pt = acosf(c);
+    // sin(acos c) = sqrt((1 - c)(1 + c)), exact factors (no sinf)
+    const float st = __builtin_amdgcn_sqrtf((1.0f - c) * (1.0f + c));
+    // Rayleigh pdf over the density 0.5 sin(pt) of a uniform flux
+    const float pdf = pt * s.inv_s2[g] * __expf(-0.5f * pt * pt * s.inv_s2[g]);
+    return st != 0.0f ? pdf * (2.0f * __builtin_amdgcn_rcpf(st)) * acc[g] * 0.125f : 0.0f;
+}
+
+// The PMT of one hit, 1..16 or 0, from its weights in full: the hit draw u1
+// against their sum, then the first j whose cumulative weight exceeds u2 * sum.
+template <int UNROLL>
+__device__ __forceinline__ int pmt_exact(const pp::PmtSetup& s, float px, float py, float pz,
+                                         const float* acc, float u1, float u2) {
+    float p[kPmts], sum = 0.0f;
+    if (UNROLL) {
+#pragma unroll
+        for (int j = 0; j < kPmts; ++j) {
+            p[j] = pmt_weight(s, j, px, py, pz, acc);
+            sum += p[j];
+        }
+    } else {
+#pragma unroll 1
+        for (int j = 0; j < kPmts; ++j) sum += pmt_weight(s, j, px, py, pz, acc);
+    }
+    int pmt = 0;
+    if (u1 < sum) {
+        const float u = u2 * sum;
+        float cum = 0.0f;
+#pragma unroll 1
+        for (int j = 0; j < kPmts; ++j) {
+            const float pj = UNROLL ? p[j] : pmt_weight(s, j, px, py, pz, acc);
+            cum += pj;
+            if (pj > 0.0f) {
+                pmt = j + 1;  // the last PMT with weight if rounding leaves u >= cum
+                if (u < cum) break;
+            }
+        }
+    }
+    return pmt;
+}
+
+// Approximate weights of one hit and the PMT they decide, or -1 where the
+// draws come too close to a decision's edge to tell. Per pair only the near
+// PMT's weight is formed, with pt = acos(c) as sqrt(1 - c) P(c) (a fit of the
+// form of Abramowitz & Stegun 4.4.46, relative error 1.7e-7), so that the
+// weight is P(c) / sqrt(1 + c) exp(-k (1 - c) P(c)^2) times a constant of the
+// group: 23 instruction slots a pair against 55 a PMT. f.rel bounds the
+// relative error of a weight, f.far the weights of the far PMTs of a group.
+__device__ __forceinline__ int pmt_fast(const pp::PmtSetup& s, const pp::PmtFast& f, float px,
+                                        float py, float pz, const float* acc, float u1, float u2) {
+    float v[8];  // the near PMT's weight, negative where that is kAntipode[j]
+    float sum = 0.0f, pole = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int g = (j >> 2) & 1;
+        const float c = fmaf(pz, s.dir[j][2], fmaf(py, s.dir[j][1], px * s.dir[j][0]));
+        const float a = fminf(fabsf(c), 1.0f);
+        float P = fmaf(0.00227945002f, a, -0.0110968914f);
+        P = fmaf(P, a, 0.0268447617f);
+        P = fmaf(P, a, -0.0487741235f);
+        P = fmaf(P, a, 0.0887490559f);
+        P = fmaf(P, a, -0.21458471f);
+        P = fmaf(P, a, 1.57079617f);
+        const float e = __builtin_amdgcn_exp2f(f.k2[g] * ((1.0f - a) * (P * P)));
+        const float w = P * __builtin_amdgcn_rsqf(1.0f + a) * e * (f.scale[g] * acc[g]);
+        pole = fmaxf(pole, a);
+        sum += w;
+        v[j] = copysignf(w, c);
+    }
+    const float edge = fmaf(f.rel, sum, fmaf(f.far[0], acc[0], f.far[1] * acc[1]));
+    int pmt = u1 < sum ? 1 : 0;
+    // at a pole of a pair the far weight is not small (and sin pt may be 0)
+    float gap = pole < 0.999999f ? fabsf(u1 - sum) : 0.0f;
+    if (__ballot(pmt)) {
+        const float t = u2 * sum;
+        float cum = 0.0f, near = t;  // the edge at 0 counts: PMTs of no weight precede it
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < kPmts; ++i) {
+            // pairs in the order of their PMT index: 0..7, then the antipodes 8..15
+            constexpr int kPair[8] = {3, 2, 1, 0, 6, 5, 4, 7};
+            cum += i < 8 ? fmaxf(v[i], 0.0f) : fmaxf(-v[kPair[i & 7]], 0.0f);
+            n += cum <= t ? 1 : 0;
+            near = fminf(near, fabsf(t - cum));
+        }
+        if (pmt) {
+            pmt = n + 1;
+            gap = fminf(gap, 0.5f * near);  // the edge of t is twice that of the sum
+            if (n >= kPmts) gap = 0.0f;
+        }
+    }
+    return gap > edge ? pmt : -1;
 }
 
 // Grid-stride over the hits (a few workgroups per CU), so that the detected
 // count takes one atomic per workgroup: a wave ballot per pass, the waves'
-// sums in LDS at the end.
-template <typename In>
+// sums in LDS at the end. FAST decides each hit from approximate weights and
+// evaluates in full only those that are too close to call (about 3 in 10^4, so
+// one wave in 50): bound by the vector ALU at 1000 instructions per wave before,
+// 215 us for 2^23 hits. The result is that of the full evaluation.
+template <typename In, bool FAST>
 __global__ void __launch_bounds__(256) pom_pmt_kernel(PmtArgs<In> a) {
     __shared__ float tab[3 * kMaxWl];
     __shared__ unsigned long long wave_det[4];
@@ -112,48 +251,26 @@ __global__ void __launch_bounds__(256) pom_pmt_kernel(PmtArgs<In> a) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < a.n; base += stride) {
         const int64_t i = base + threadIdx.x;
-        bool det = false;
+        int pmt = 0;
         if (i < a.n) {
             float px, py, pz, wl;
             uint64_t id;
             uint32_t sx;
             a.in.load(i, px, py, pz, wl, id, sx);
-            const float acc[2] = {interp0(tab, tab + n_wl, n_wl, wl),
-                                  interp0(tab, tab + 2 * n_wl, n_wl, wl)};
-            float p[kPmts], sum = 0.0f;
-#pragma unroll
-            for (int j = 0; j < kPmts; ++j) {
-                const int g = (j >> 2) & 1;
-                const float c = fminf(fmaxf(px * a.s.dir[j][0] + py * a.s.dir[j][1] +
-                                                pz * a.s.dir[j][2],
-                                            -1.0f), 1.0f);
-                const float pt = acosf(c);
-                // sin(acos c) = sqrt((1 - c)(1 + c)), exact factors (no sinf)
-                const float st = __builtin_amdgcn_sqrtf((1.0f - c) * (1.0f + c));
-                // Rayleigh pdf over the density 0.5 sin(pt) of a uniform flux
-                const float pdf = pt * a.s.inv_s2[g] * __expf(-0.5f * pt * pt * a.s.inv_s2[g]);
-                p[j] = st != 0.0f ? pdf * (2.0f * __builtin_amdgcn_rcpf(st)) * acc[g] * 0.125f : 0.0f;
-                sum += p[j];
-            }
+            float acc[2];
+            interp0(tab, tab + n_wl, tab + 2 * n_wl, n_wl, wl, acc);
             const uint4 r = pp::philox(make_uint4(PP_CTR_PMT, (uint32_t)id, (uint32_t)(id >> 32), sx),
                                        a.s.k0, a.s.k1);
-            int pmt = 0;
-            if (pp::u01(r.x) < sum) {
-                // categorical draw: first j whose cumulative weight exceeds u * sum
-                const float u = pp::u01(r.y) * sum;
-                float cum = 0.0f;
-                for (int j = 0; j < kPmts; ++j) {
-                    cum += p[j];
-                    if (p[j] > 0.0f) {
-                        pmt = j + 1;  // the last PMT with weight if rounding leaves u >= cum
-                        if (u < cum) break;
-                    }
-                }
-                det = true;
+            const float u1 = pp::u01(r.x), u2 = pp::u01(r.y);
+            if (FAST) {
+                pmt = pmt_fast(a.s, a.f, px, py, pz, acc, u1, u2);
+                if (pmt < 0) pmt = pmt_exact<0>(a.s, px, py, pz, acc, u1, u2);
+            } else {
+                pmt = pmt_exact<1>(a.s, px, py, pz, acc, u1, u2);
             }
             a.out[i] = pmt;
         }
-        n_det += (unsigned long long)__popcll(__ballot(det));
+        n_det += (unsigned long long)__popcll(__ballot(pmt != 0));
     }
     if (__lane_id() == 0) wave_det[threadIdx.x >> 6] = n_det;
     __syncthreads();
@@ -165,10 +282,13 @@ __global__ void __launch_bounds__(256) pom_pmt_kernel(PmtArgs<In> a) {
 }
 
 template <typename In>
-int launch(const PmtArgs<In>& a, hipStream_t stream, int n_cu) {
+int launch(PmtArgs<In>& a, hipStream_t stream, int n_cu) {
     const int64_t blocks = std::min<int64_t>((a.n + 255) / 256, (int64_t)std::max(n_cu, 1) * 8);
-    hipLaunchKernelGGL(pom_pmt_kernel<In>, dim3((unsigned)std::max<int64_t>(blocks, 1)), dim3(256),
-                       0, stream, a);
+    const dim3 grid((unsigned)std::max<int64_t>(blocks, 1));
+    if (fast_setup(a.s, &a.f))
+        hipLaunchKernelGGL((pom_pmt_kernel<In, true>), grid, dim3(256), 0, stream, a);
+    else
+        hipLaunchKernelGGL((pom_pmt_kernel<In, false>), grid, dim3(256), 0, stream, a);
     PP_HIP(hipGetLastError());
     return PP_OK;
 }
@@ -225,10 +345,12 @@ int pmt_setup(const pp_pom_model* m, const float* wl_grid, const float* acc1, co
     s->k0 = (uint32_t)seed;
     s->k1 = (uint32_t)(seed >> 32);
     const size_t nw = (size_t)m->n_wl;
+    s->acc_ok = true;
     for (size_t k = 0; k < nw; ++k) {
         tab[k] = wl_grid[k];
         tab[nw + k] = acc1[k];
         tab[2 * nw + k] = acc2[k];
+        s->acc_ok = s->acc_ok && acc1[k] >= 0.0f && acc2[k] >= 0.0f;
     }
     return PP_OK;
 }
