@@ -34,13 +34,15 @@ struct PmtSetup {
     float inv_s2[2];
     int32_t n_wl;
     uint32_t k0, k1;
-    bool acc_ok;  // every acceptance is >= 0
+    bool acc_ok;   // every acceptance is >= 0
+    float inv_dx;  // 1 / knot spacing of a nearly equidistant table, else 0
 };
 
 // Constants of the detection kernel's approximate weights, per PMT group.
 struct PmtFast {
     float k2[2];     // -log2(e) / (2 sigma^2)
     float scale[2];  // 1 / (4 sigma^2)
+    float reach[2];  // bound of all near weights together per unit of the larger group's acceptance
     float far[2];    // bound of the far PMTs' summed weight per unit of acceptance
     float rel;       // bound of a weight's relative error
 };

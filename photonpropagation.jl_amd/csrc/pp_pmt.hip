@@ -75,27 +75,64 @@ struct PmtRecords {
     }
 };
 
+// PMT (theta, phi) of the POM, src/pom.jl:108-128
+void pom_angles(double th[kPmts], double ph[kPmts]) {
+    const double d2r = M_PI / 180.0;
+    for (int k = 0; k < 4; ++k) {
+        th[k] = (90.0 - 25.0) * d2r;
+        ph[k] = k * M_PI / 2;
+        th[4 + k] = (90.0 - 57.5) * d2r;
+        ph[4 + k] = M_PI / 4 + k * M_PI / 2;
+        th[8 + k] = (90.0 + 25.0) * d2r;
+        th[12 + k] = (90.0 + 57.5) * d2r;
+    }
+    const double lower2[4] = {M_PI / 2, 0.0, 3 * M_PI / 2, M_PI};
+    const double lower[4] = {M_PI / 4, 7 * M_PI / 4, 5 * M_PI / 4, 3 * M_PI / 4};
+    for (int k = 0; k < 4; ++k) {
+        ph[8 + k] = lower2[k];
+        ph[12 + k] = lower[k];
+    }
+}
+
 // The 16 PMT directions are 8 antipodal pairs of one group each: PMT j and
 // kAntipode[j], j < 8 (the layout of pom_angles; fast_setup checks it).
 constexpr int kAntipode[8] = {11, 10, 9, 8, 14, 13, 12, 15};
 
-// Constants of the approximate weights (pmt_fast) of a set-up; false where
-// they do not serve: directions that are not antipodal pairs to 1e-6, a
-// negative acceptance, or widths whose error bounds leave too much to evaluate in full (sigma below 0.02 or,
-// with its far PMTs' weights, above 0.4 or so). With k = 1 / (2 sigma^2), a
+// Constants of the approximate weights (pmt_fast) of a set-up; false where they
+// do not serve: a module orientation that is not a rotation (or reflection) to
+// 1e-5, a negative acceptance, or widths whose error bounds leave too much to
+// evaluate in full (sigma below 0.02 or above 0.4). With k = 1 / (2 sigma^2), a
 // weight's relative error has three parts: the cosine, off by 2.5e-7 at most in
 // either evaluation, times d ln p / dc <= pi k + 2; the fit of acos, 2e-7 times
 // 1 + 2 k pt^2 <= 1 + 5 k; and 1e-5 for the roundings of both evaluations.
+// Per unit of acceptance a group's weight is at most scale, at its PMTs' axes,
+// and falls with the angle. The near weights of both groups, each in units of its
+// own largest, add up to at most 1.1455 for widths up to 0.3 and 1.7101 up to
+// 0.4 (the sum grows with either width; the largest value over the sphere, at
+// 0.075 degree steps), so that no position's sum exceeds that times the larger
+// group's acceptance x scale: reach, with 1% to spare.
 bool fast_setup(const pp::PmtSetup& s, pp::PmtFast* f) {
     if (!s.acc_ok) return false;
     for (int j = 0; j < 8; ++j)
         for (int r = 0; r < 3; ++r)
             if (!(std::fabs(s.dir[j][r] + s.dir[kAntipode[j]][r]) <= 1e-6f)) return false;
+    double th[kPmts], ph[kPmts];
+    pom_angles(th, ph);
+    for (int j = 0; j < 8; ++j)
+        for (int k = 0; k <= j; ++k) {
+            double want = std::cos(th[j]) * std::cos(th[k]) +
+                          std::sin(th[j]) * std::sin(th[k]) * std::cos(ph[j] - ph[k]);
+            for (int r = 0; r < 3; ++r) want -= (double)s.dir[j][r] * s.dir[k][r];
+            if (!(std::fabs(want) <= 1e-5)) return false;
+        }
+    const float width = std::max(1.0f / std::sqrt(s.inv_s2[0]), 1.0f / std::sqrt(s.inv_s2[1]));
+    if (!(width <= 0.4f)) return false;
     f->rel = 0.0f;
     for (int g = 0; g < 2; ++g) {
         const double k = 0.5 * s.inv_s2[g];
         f->k2[g] = (float)(-k * 1.4426950408889634);
         f->scale[g] = s.inv_s2[g] * 0.25f;
+        f->reach[g] = f->scale[g] * (width <= 0.3f ? 1.16f : 1.73f);
         f->rel = std::max(f->rel, (float)(2.5e-7 * (M_PI * k + 2.0) + 2e-7 * (1.0 + 5.0 * k) + 1e-5));
         // four far PMTs a group, each at most pt exp(-k pt^2) / sin(pt) per unit
         // of scale and acceptance: up to 3 pi/4, and from there to the pole that
@@ -118,16 +155,24 @@ struct PmtArgs {
 };
 
 // Both groups' acceptances: linear interpolation in a sorted table, 0 outside
-// (extrapolation_bc = 0)
+// (extrapolation_bc = 0). inv_dx > 0: the knots are so nearly equidistant that
+// (v - x[0]) inv_dx is at most one interval off (pmt_setup), and a compare with the
+// interval's ends settles it; otherwise a binary search.
 __device__ __forceinline__ void interp0(const float* x, const float* y1, const float* y2, int n,
-                                        float v, float* acc) {
+                                        float inv_dx, float v, float* acc) {
     acc[0] = acc[1] = 0.0f;
     if (!(v >= x[0] && v <= x[n - 1])) return;
     int lo = 0, hi = n - 1;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (x[mid] <= v) lo = mid;
-        else hi = mid;
+    if (inv_dx > 0.0f) {
+        lo = min((int)((v - x[0]) * inv_dx), n - 2);
+        lo += (v >= x[lo + 1] && lo < n - 2) - (v < x[lo] && lo > 0);
+        hi = lo + 1;
+    } else {
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (x[mid] <= v) lo = mid;
+            else hi = mid;
+        }
     }
     const float t = (v - x[lo]) / (x[hi] - x[lo]);
     acc[0] = y1[lo] + t * (y1[hi] - y1[lo]);
@@ -234,15 +279,25 @@ __device__ __forceinline__ int pmt_fast(const pp::PmtSetup& s, const pp::PmtFast
     return gap > edge ? pmt : -1;
 }
 
+// The workgroup's detected hits (n_det per wave) in one atomic
+__device__ __forceinline__ void count_detected(unsigned long long* wave_det,
+                                               unsigned long long n_det,
+                                               unsigned long long* total) {
+    if (__lane_id() == 0) wave_det[threadIdx.x >> 6] = n_det;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long s = 0;
+        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) s += wave_det[w];
+        if (s) atomicAdd(total, s);
+    }
+}
+
 // Grid-stride over the hits (a few workgroups per CU), so that the detected
 // count takes one atomic per workgroup: a wave ballot per pass, the waves'
-// sums in LDS at the end. FAST decides each hit from approximate weights and
-// evaluates in full only those that are too close to call (about 3 in 10^4, so
-// one wave in 50): bound by the vector ALU at 1000 instructions per wave before,
-// 215 us for 2^23 hits. The result is that of the full evaluation.
-template <typename In, bool FAST>
-__global__ void __launch_bounds__(256) pom_pmt_kernel(PmtArgs<In> a) {
-    __shared__ float tab[3 * kMaxWl];
+// sums in LDS at the end.
+template <typename In>
+__global__ void __launch_bounds__(256) pom_pmt_full_kernel(PmtArgs<In> a) {
+    extern __shared__ float tab[];
     __shared__ unsigned long long wave_det[4];
     const int n_wl = a.s.n_wl;
     for (int i = threadIdx.x; i < 3 * n_wl; i += blockDim.x) tab[i] = a.tab[i];
@@ -258,58 +313,116 @@ __global__ void __launch_bounds__(256) pom_pmt_kernel(PmtArgs<In> a) {
             uint32_t sx;
             a.in.load(i, px, py, pz, wl, id, sx);
             float acc[2];
-            interp0(tab, tab + n_wl, tab + 2 * n_wl, n_wl, wl, acc);
+            interp0(tab, tab + n_wl, tab + 2 * n_wl, n_wl, a.s.inv_dx, wl, acc);
             const uint4 r = pp::philox(make_uint4(PP_CTR_PMT, (uint32_t)id, (uint32_t)(id >> 32), sx),
                                        a.s.k0, a.s.k1);
-            const float u1 = pp::u01(r.x), u2 = pp::u01(r.y);
-            if (FAST) {
-                pmt = pmt_fast(a.s, a.f, px, py, pz, acc, u1, u2);
-                if (pmt < 0) pmt = pmt_exact<0>(a.s, px, py, pz, acc, u1, u2);
-            } else {
-                pmt = pmt_exact<1>(a.s, px, py, pz, acc, u1, u2);
-            }
+            pmt = pmt_exact<1>(a.s, px, py, pz, acc, pp::u01(r.x), pp::u01(r.y));
             a.out[i] = pmt;
         }
         n_det += (unsigned long long)__popcll(__ballot(pmt != 0));
     }
-    if (__lane_id() == 0) wave_det[threadIdx.x >> 6] = n_det;
+    count_detected(wave_det, n_det, a.n_det);
+}
+
+// A hit with weights still to come, in the wave's LDS list
+struct Pending {
+    float px, py, pz, u1;
+    float acc0, acc1, u2;
+    uint32_t i;
+};
+
+// The same decisions with few weights evaluated. Bound by the vector ALU (1000
+// instructions per 64 hits with every weight in full: 215 us for 2^23 hits), so
+//   - a hit whose draw u1 lies above the largest sum of weights any position
+//     could have at its wavelength (f.reach) is not detected: three in four of
+//     them, at the POM's acceptances, need no weight;
+//   - the others are gathered in an LDS list of the wave and taken 64 at a time,
+//     so that every lane works, with approximate weights (pmt_fast);
+//   - what those leave open (3 in 10^4) is evaluated in full.
+// 215 -> 103 us with pmt_fast alone, 62 us with the list.
+template <typename In>
+__global__ void __launch_bounds__(256) pom_pmt_kernel(PmtArgs<In> a) {
+    extern __shared__ float tab[];
+    __shared__ unsigned long long wave_det[4];
+    __shared__ __attribute__((aligned(16))) Pending list[4][128];
+    const int n_wl = a.s.n_wl;
+    for (int i = threadIdx.x; i < 3 * n_wl; i += blockDim.x) tab[i] = a.tab[i];
     __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long s = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) s += wave_det[w];
-        if (s) atomicAdd(a.n_det, s);
+    const uint32_t lane = threadIdx.x & 63;
+    Pending* const mine = list[threadIdx.x >> 6];
+    unsigned long long n_det = 0;  // wave-uniform
+    uint32_t count = 0;            // pending hits, wave-uniform; below 64 after every pass
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    int64_t base = (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
+    for (;;) {
+        const bool more = base < a.n;
+        if (more) {
+            const int64_t i = base + lane;
+            Pending h;
+            bool keep = false;
+            if (i < a.n) {
+                float wl, acc[2];
+                uint64_t id;
+                uint32_t sx;
+                a.in.load(i, h.px, h.py, h.pz, wl, id, sx);
+                interp0(tab, tab + n_wl, tab + 2 * n_wl, n_wl, a.s.inv_dx, wl, acc);
+                const uint4 r = pp::philox(
+                    make_uint4(PP_CTR_PMT, (uint32_t)id, (uint32_t)(id >> 32), sx), a.s.k0, a.s.k1);
+                h.u1 = pp::u01(r.x);
+                h.u2 = pp::u01(r.y);
+                h.acc0 = acc[0];
+                h.acc1 = acc[1];
+                h.i = (uint32_t)i;
+                const float most = fmaxf(a.f.reach[0] * acc[0], a.f.reach[1] * acc[1]) +
+                                   fmaf(a.f.far[0], acc[0], a.f.far[1] * acc[1]);
+                // the bound holds on the unit sphere (and for 0 acceptance u1 >= 0)
+                const float r2 = fmaf(h.pz, h.pz, fmaf(h.py, h.py, h.px * h.px));
+                keep = !(h.u1 >= most && r2 <= 1.0002f);
+                if (!keep) a.out[i] = 0;
+            }
+            const uint64_t m = __ballot(keep);
+            if (keep) {
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                mine[count + rank] = h;
+            }
+            count += (uint32_t)__popcll(m);
+            base += stride;
+        } else if (count == 0) {
+            break;
+        }
+        if (count >= 64 || !more) {
+            const uint32_t n = count < 64 ? count : 64;
+            count -= n;
+            // one wave's LDS accesses run in order; only the compiler must not
+            // move them across
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            int pmt = 0;
+            if (lane < n) {
+                const Pending h = mine[count + lane];
+                const float acc[2] = {h.acc0, h.acc1};
+                pmt = pmt_fast(a.s, a.f, h.px, h.py, h.pz, acc, h.u1, h.u2);
+                if (pmt < 0) pmt = pmt_exact<0>(a.s, h.px, h.py, h.pz, acc, h.u1, h.u2);
+                a.out[h.i] = pmt;
+            }
+            n_det += (unsigned long long)__popcll(__ballot(pmt != 0));
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
     }
+    count_detected(wave_det, n_det, a.n_det);
 }
 
 template <typename In>
 int launch(PmtArgs<In>& a, hipStream_t stream, int n_cu) {
     const int64_t blocks = std::min<int64_t>((a.n + 255) / 256, (int64_t)std::max(n_cu, 1) * 8);
     const dim3 grid((unsigned)std::max<int64_t>(blocks, 1));
-    if (fast_setup(a.s, &a.f))
-        hipLaunchKernelGGL((pom_pmt_kernel<In, true>), grid, dim3(256), 0, stream, a);
-    else
-        hipLaunchKernelGGL((pom_pmt_kernel<In, false>), grid, dim3(256), 0, stream, a);
+    const size_t lds = 3 * sizeof(float) * (size_t)a.s.n_wl;
+    hipLaunchKernelGGL(fast_setup(a.s, &a.f) ? pom_pmt_kernel<In> : pom_pmt_full_kernel<In>, grid,
+                       dim3(256), lds, stream, a);
     PP_HIP(hipGetLastError());
     return PP_OK;
-}
-
-// PMT (theta, phi) of the POM, src/pom.jl:108-128
-void pom_angles(double th[kPmts], double ph[kPmts]) {
-    const double d2r = M_PI / 180.0;
-    for (int k = 0; k < 4; ++k) {
-        th[k] = (90.0 - 25.0) * d2r;
-        ph[k] = k * M_PI / 2;
-        th[4 + k] = (90.0 - 57.5) * d2r;
-        ph[4 + k] = M_PI / 4 + k * M_PI / 2;
-        th[8 + k] = (90.0 + 25.0) * d2r;
-        th[12 + k] = (90.0 + 57.5) * d2r;
-    }
-    const double lower2[4] = {M_PI / 2, 0.0, 3 * M_PI / 2, M_PI};
-    const double lower[4] = {M_PI / 4, 7 * M_PI / 4, 5 * M_PI / 4, 3 * M_PI / 4};
-    for (int k = 0; k < 4; ++k) {
-        ph[8 + k] = lower2[k];
-        ph[12 + k] = lower[k];
-    }
 }
 
 int validate(const pp_pom_model* m) {
@@ -351,6 +464,13 @@ int pmt_setup(const pp_pom_model* m, const float* wl_grid, const float* acc1, co
         tab[nw + k] = acc1[k];
         tab[2 * nw + k] = acc2[k];
         s->acc_ok = s->acc_ok && acc1[k] >= 0.0f && acc2[k] >= 0.0f;
+    }
+    // equidistant enough for interp0: every knot's own guess is its interval or
+    // the one before
+    s->inv_dx = (float)(m->n_wl - 1) / (wl_grid[m->n_wl - 1] - wl_grid[0]);
+    for (int k = 0; k < m->n_wl; ++k) {
+        const float g = (wl_grid[k] - wl_grid[0]) * s->inv_dx;
+        if (!(g >= (float)(k - 1) && g < (float)(k + 1))) s->inv_dx = 0.0f;
     }
     return PP_OK;
 }
