@@ -52,12 +52,17 @@ struct PmtFast {
 int pmt_setup(const pp_pom_model* m, const float* wl_grid, const float* acc1, const float* acc2,
               uint64_t seed, PmtSetup* s, float* tab);
 
+// Acceptance tables of up to this many knots (the POM's has 26) travel with the
+// launch, so that a detection call is one launch: the table's copy, the
+// counter's clearing and their gaps took 18 us of a call on device arrays.
+constexpr int kArgKnots = 64;
+
 // The detection kernel over n context hit records (module centre and radius
 // from `targets`, one (x, y, z, radius) per target, indexed by the record's
-// 1-based module index), writing out[i] and adding the detected count to
-// *count (which the caller clears). `tab` is the device copy of the table.
-int pmt_launch_records(const PmtSetup& s, const float* tab, const HitRecord* rec, int64_t n,
-                       const float4* targets, int32_t* out, unsigned long long* count,
+// 1-based module index), writing out[i]. `tab` is the table, `d_tab` its device
+// copy, which is only needed (and read) beyond kArgKnots knots.
+int pmt_launch_records(const PmtSetup& s, const float* tab, const float* d_tab,
+                       const HitRecord* rec, int64_t n, const float4* targets, int32_t* out,
                        hipStream_t stream, int n_cu);
 
 // The hit records of a context's last propagation (device pointer, in

@@ -24,6 +24,7 @@
 #include "pp_grid_build.h"
 #include "pp_hits.h"
 #include "pp_search.h"
+#include "pp_stage.h"
 
 #include <rocprim/device/device_radix_sort.hpp>
 
@@ -997,6 +998,7 @@ struct pp_ctx {
     // pinned host staging of hit records for pp_copy_hits
     HitRecord* h_rec = nullptr;
     int64_t h_rec_cap = 0;
+    pp::PinnedPair pin;  // PMT ids on their way to pageable host memory
     // device sort of the hits by (source, photon id): the records in that
     // order, keys, indices and the radix sort's scratch, in one allocation
     char* d_sort = nullptr;
@@ -1009,7 +1011,7 @@ struct pp_ctx {
     void* h_batch = nullptr;
     size_t batch_cap = 0;  // bytes of each
     // PMT detection of the context's hits: targets as (x, y, z, radius), and
-    // one device block holding the acceptance table | detected count | PMT ids
+    // one device block holding the acceptance table | PMT ids
     float4* d_tgt_r = nullptr;
     char* d_pmt = nullptr;
     size_t pmt_cap = 0;
@@ -1447,6 +1449,7 @@ int pp_destroy(pp_ctx* ctx) {
     if (ctx->d_sort) (void)hipFree(ctx->d_sort);
     if (ctx->d_tgt_r) (void)hipFree(ctx->d_tgt_r);
     if (ctx->d_pmt) (void)hipFree(ctx->d_pmt);
+    ctx->pin.release();
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -2112,6 +2115,7 @@ int pp_release_scratch(pp_ctx* ctx) {
     ctx->h_rec_cap = 0;
     ctx->d_pmt = nullptr;
     ctx->pmt_cap = 0;
+    ctx->pin.release();
     std::vector<int64_t>().swap(ctx->perm);
     ctx->perm_valid = false;
     return PP_OK;
@@ -2146,9 +2150,8 @@ int pp_pom_pmt_hits_ctx(pp_ctx* ctx, const pp_pom_model* m, const float* wl_grid
     const bool host_sort = ordered && (ctx->cfg.deterministic_order == 2 || !ctx->sorted_valid);
     const HitRecord* src = ordered && !host_sort ? (const HitRecord*)ctx->d_sort : ctx->hits.rec;
     const int64_t lo = host_sort ? 0 : first, cnt = host_sort ? ctx->n_hits : n;
-    // table | detected count | PMT ids, kept by the context and grown when needed
-    const size_t off_cnt = align256(tab.size() * sizeof(float));
-    const size_t off_out = off_cnt + 256;
+    // table | PMT ids, kept by the context and grown when needed
+    const size_t off_out = align256(tab.size() * sizeof(float));
     const size_t need = off_out + (size_t)cnt * sizeof(int32_t);
     if (need > ctx->pmt_cap) {
         PP_HIP(hipStreamSynchronize(ctx->stream));
@@ -2162,13 +2165,12 @@ int pp_pom_pmt_hits_ctx(pp_ctx* ctx, const pp_pom_model* m, const float* wl_grid
         ctx->pmt_cap = need;
     }
     float* d_tab = (float*)ctx->d_pmt;
-    auto* d_cnt = (unsigned long long*)(ctx->d_pmt + off_cnt);
     auto* d_out = (int32_t*)(ctx->d_pmt + off_out);
-    PP_HIP(hipMemcpyAsync(d_tab, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice,
-                          ctx->stream));
-    PP_HIP(hipMemsetAsync(d_cnt, 0, sizeof(unsigned long long), ctx->stream));
+    if (m->n_wl > pp::kArgKnots)
+        PP_HIP(hipMemcpyAsync(d_tab, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice,
+                              ctx->stream));
     PP_HIP(hipEventRecord(ctx->ev0, ctx->stream));
-    if (int rc = pp::pmt_launch_records(st, d_tab, src + lo, cnt, ctx->d_tgt_r, d_out, d_cnt,
+    if (int rc = pp::pmt_launch_records(st, tab.data(), d_tab, src + lo, cnt, ctx->d_tgt_r, d_out,
                                         ctx->stream, ctx->n_cu))
         return rc;
     PP_HIP(hipEventRecord(ctx->ev1, ctx->stream));
@@ -2178,9 +2180,7 @@ int pp_pom_pmt_hits_ctx(pp_ctx* ctx, const pp_pom_model* m, const float* wl_grid
         all.resize((size_t)cnt);
         dst = all.data();
     }
-    PP_HIP(hipMemcpyAsync(dst, d_out, (size_t)cnt * sizeof(int32_t), hipMemcpyDeviceToHost,
-                          ctx->stream));
-    PP_HIP(hipStreamSynchronize(ctx->stream));
+    PP_HIP(ctx->pin.copy_out(ctx->stream, dst, d_out, (size_t)cnt * sizeof(int32_t)));
     if (kernel_ms) PP_HIP(hipEventElapsedTime(kernel_ms, ctx->ev0, ctx->ev1));
     if (host_sort) {
         if (!ctx->perm_valid) {

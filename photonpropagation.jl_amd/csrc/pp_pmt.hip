@@ -20,6 +20,7 @@ namespace {
 
 constexpr int kPmts = 16;
 constexpr int kMaxWl = 1024;
+using pp::kArgKnots;
 // PMT group of PMT j (src/pom.jl:172-174): PMTs 0-3 and 8-11 (25 deg from the
 // equator) are group 1, 4-7 and 12-15 (57.5 deg) group 2: index (j >> 2) & 1
 
@@ -147,12 +148,21 @@ template <typename In>
 struct PmtArgs {
     pp::PmtSetup s;
     pp::PmtFast f;
-    const float* tab;  // wl | acc1 | acc2, n_wl each
+    const float* tab;  // wl | acc1 | acc2, n_wl each; NULL: in `knots`
+    float knots[3 * kArgKnots];
     In in;
     int64_t n;
     int32_t* out;
-    unsigned long long* n_det;
+    unsigned long long* n_det;  // may be NULL
 };
+
+// The acceptance table into LDS
+template <typename Args>
+__device__ __forceinline__ void stage_table(const Args& a, float* tab) {
+    for (int i = threadIdx.x; i < 3 * a.s.n_wl; i += blockDim.x)
+        tab[i] = a.tab ? a.tab[i] : a.knots[i];
+    __syncthreads();
+}
 
 // Both groups' acceptances: linear interpolation in a sorted table, 0 outside
 // (extrapolation_bc = 0). inv_dx > 0: the knots are so nearly equidistant that
@@ -283,6 +293,7 @@ __device__ __forceinline__ int pmt_fast(const pp::PmtSetup& s, const pp::PmtFast
 __device__ __forceinline__ void count_detected(unsigned long long* wave_det,
                                                unsigned long long n_det,
                                                unsigned long long* total) {
+    if (!total) return;
     if (__lane_id() == 0) wave_det[threadIdx.x >> 6] = n_det;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -300,8 +311,7 @@ __global__ void __launch_bounds__(256) pom_pmt_full_kernel(PmtArgs<In> a) {
     extern __shared__ float tab[];
     __shared__ unsigned long long wave_det[4];
     const int n_wl = a.s.n_wl;
-    for (int i = threadIdx.x; i < 3 * n_wl; i += blockDim.x) tab[i] = a.tab[i];
-    __syncthreads();
+    stage_table(a, tab);
     unsigned long long n_det = 0;  // wave-uniform
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < a.n; base += stride) {
@@ -339,32 +349,41 @@ struct Pending {
 //   - the others are gathered in an LDS list of the wave and taken 64 at a time,
 //     so that every lane works, with approximate weights (pmt_fast);
 //   - what those leave open (3 in 10^4) is evaluated in full.
-// 215 -> 103 us with pmt_fast alone, 62 us with the list.
+// 215 -> 103 us with pmt_fast alone, 69 us of kernel
+// with the list.
 template <typename In>
 __global__ void __launch_bounds__(256) pom_pmt_kernel(PmtArgs<In> a) {
     extern __shared__ float tab[];
     __shared__ unsigned long long wave_det[4];
     __shared__ __attribute__((aligned(16))) Pending list[4][128];
     const int n_wl = a.s.n_wl;
-    for (int i = threadIdx.x; i < 3 * n_wl; i += blockDim.x) tab[i] = a.tab[i];
-    __syncthreads();
+    stage_table(a, tab);
     const uint32_t lane = threadIdx.x & 63;
     Pending* const mine = list[threadIdx.x >> 6];
     unsigned long long n_det = 0;  // wave-uniform
     uint32_t count = 0;            // pending hits, wave-uniform; below 64 after every pass
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     int64_t base = (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
+    // the next pass's hit, loaded while this one's is worked on (69 -> 67 us)
+    float nx = 0.0f, ny = 0.0f, nz = 0.0f, nw = 0.0f;
+    uint64_t nid = 0;
+    uint32_t nsx = 0;
+    if (base + lane < a.n) a.in.load(base + lane, nx, ny, nz, nw, nid, nsx);
     for (;;) {
         const bool more = base < a.n;
         if (more) {
             const int64_t i = base + lane;
             Pending h;
+            h.px = nx;
+            h.py = ny;
+            h.pz = nz;
+            const float wl = nw;
+            const uint64_t id = nid;
+            const uint32_t sx = nsx;
             bool keep = false;
+            if (i + stride < a.n) a.in.load(i + stride, nx, ny, nz, nw, nid, nsx);
             if (i < a.n) {
-                float wl, acc[2];
-                uint64_t id;
-                uint32_t sx;
-                a.in.load(i, h.px, h.py, h.pz, wl, id, sx);
+                float acc[2];
                 interp0(tab, tab + n_wl, tab + 2 * n_wl, n_wl, a.s.inv_dx, wl, acc);
                 const uint4 r = pp::philox(
                     make_uint4(PP_CTR_PMT, (uint32_t)id, (uint32_t)(id >> 32), sx), a.s.k0, a.s.k1);
@@ -475,17 +494,19 @@ int pmt_setup(const pp_pom_model* m, const float* wl_grid, const float* acc1, co
     return PP_OK;
 }
 
-int pmt_launch_records(const PmtSetup& s, const float* tab, const HitRecord* rec, int64_t n,
-                       const float4* targets, int32_t* out, unsigned long long* count,
+int pmt_launch_records(const PmtSetup& s, const float* tab, const float* d_tab,
+                       const HitRecord* rec, int64_t n, const float4* targets, int32_t* out,
                        hipStream_t stream, int n_cu) {
     PmtArgs<PmtRecords> a{};
     a.s = s;
-    a.tab = tab;
+    if (s.n_wl <= kArgKnots)
+        std::copy(tab, tab + 3 * s.n_wl, a.knots);
+    else
+        a.tab = d_tab;
     a.in.rec = rec;
     a.in.targets = targets;
     a.n = n;
     a.out = out;
-    a.n_det = count;
     return launch(a, stream, n_cu);
 }
 
@@ -653,19 +674,26 @@ int pp_pom_pmt_hits_noalloc(int device, const pp_pom_model* m, const float* wl_g
     if (int rc = pp::pmt_setup(m, wl_grid, acc1, acc2, seed, &a.s, tab)) return rc;
     const hipStream_t st = (hipStream_t)stream;
     auto* d_cnt = (unsigned long long*)(sc + kScratchTableBytes);
-    // from pageable host memory: HIP stages the bytes before the call returns,
-    // so the stack copy may go out of scope while the transfer is queued
-    PP_HIP(hipMemcpyAsync(sc, tab, 3 * (size_t)m->n_wl * sizeof(float), hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(clear_count_kernel, dim3(1), dim3(64), 0, st, d_cnt);
-    PP_HIP(hipGetLastError());
-    a.tab = (const float*)sc;
+    if (m->n_wl <= kArgKnots) {
+        std::copy(tab, tab + 3 * m->n_wl, a.knots);
+    } else {
+        // from pageable host memory: HIP stages the bytes before the call returns,
+        // so the stack copy may go out of scope while the transfer is queued
+        PP_HIP(hipMemcpyAsync(sc, tab, 3 * (size_t)m->n_wl * sizeof(float), hipMemcpyHostToDevice,
+                              st));
+        a.tab = (const float*)sc;
+    }
+    if (n_detected) {
+        hipLaunchKernelGGL(clear_count_kernel, dim3(1), dim3(64), 0, st, d_cnt);
+        PP_HIP(hipGetLastError());
+        a.n_det = d_cnt;
+    }
     a.in.rel_pos = d_rel_pos3;
     a.in.wl = d_wavelength;
     a.in.pid = d_photon_id;
     a.in.src = d_source_ix;
     a.n = n;
     a.out = d_pmt_id_out;
-    a.n_det = d_cnt;
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
         cus <= 0)
