@@ -47,7 +47,7 @@ struct HitCols {
 
 struct Counters {
     unsigned long long n_hits;    // reserved slots (may exceed capacity)
-    unsigned long long n_ph_sim;  // completed photons
+    unsigned long long n_lost;    // photons of started work that an overflow left incomplete
     unsigned int err;             // 1 = overflow
     unsigned int pad;
     // work counts of the instrumented kernel (pp_config.count_work)
@@ -507,14 +507,14 @@ __device__ __forceinline__ bool transport_group(const KParams& p, const pp_sourc
     return hit;
 }
 
-// n_done: this lane's completed photons; wave_done: the wave's (the same
-// value in every lane, added once)
+// lost: the wave's photons that were not completed, 0 unless the hit buffer
+// overflowed (the completed ones are the launch's photons less these: counting
+// them took an atomic per lane or wave at the end of every launch, 18 us of the
+// README example's 36)
 template <bool COUNT>
-__device__ __forceinline__ void flush_counts(const KParams& p, unsigned long long n_done,
-                                             unsigned long long wave_done,
+__device__ __forceinline__ void flush_counts(const KParams& p, unsigned long long lost,
                                              unsigned long long n_steps_done, const pp::Work& work) {
-    if (n_done) atomicAdd(&p.counters->n_ph_sim, n_done);
-    if (wave_done && __lane_id() == 0) atomicAdd(&p.counters->n_ph_sim, wave_done);
+    if (lost && __lane_id() == 0) atomicAdd(&p.counters->n_lost, lost);
     if (COUNT) {
         atomicAdd(&p.counters->steps, n_steps_done);
         atomicAdd(&p.counters->tests, (unsigned long long)work.tests);
@@ -569,6 +569,30 @@ __device__ __forceinline__ pp_source source_record(const pp_source* sp, uint32_t
 #endif
 }
 
+// One photon per lane (active lanes), the whole wave together, hits stored.
+// False where this lane's hit did not fit the buffer.
+template <bool COUNT, int SEARCH>
+__device__ __forceinline__ bool propagate_group(const KParams& p, const pp_source& src,
+                                                uint32_t src_ix, uint64_t pid, bool active,
+                                                const float* spec, const SearchT<SEARCH>& search,
+                                                const pp::Phase& phase, const WaveQueue& q,
+                                                pp::Work& work, unsigned long long& n_steps_done) {
+    bool stored = true;
+    if constexpr (kDeferredWalk<SEARCH>) {
+        HitRec h;
+        const bool hit = transport_group<COUNT>(p, src, src_ix, pid, active, spec, search, phase, q,
+                                                work, n_steps_done, h);
+        stored = store_hits(hit, h, src_ix, p.hits, p.counters);
+    } else if (active) {
+        HitRec h;
+        const bool hit = transport_photon<COUNT>(p, src, src_ix, pid, spec, search, phase, work,
+                                                 n_steps_done, h);
+        stored = store_hits(hit, h, src_ix, p.hits, p.counters);
+    }
+    if (!stored) atomicOr(&p.counters->err, 1u);
+    return stored;
+}
+
 template <int PHASE, int SEARCH, bool COUNT = false>
 __global__ void PP_PROPAGATE_ATTRS propagate_kernel(KParams p) {
     const Lds l = stage_lds<SEARCH>(p);
@@ -576,47 +600,31 @@ __global__ void PP_PROPAGATE_ATTRS propagate_kernel(KParams p) {
     phase.kind = PHASE;
     const auto search = make_search<SEARCH>(p, l);
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    // photons completed: per lane in the one-photon loop, per wave (a scalar,
-    // never spilled) in the wave loop
-    unsigned long long n_done = 0, wave_done = 0, n_steps_done = 0;
+    unsigned long long lost = 0, n_steps_done = 0;
     pp::Work work;
-    if constexpr (kDeferredWalk<SEARCH>) {
-        // whole waves of photons, the loop condition uniform across the wave
-        const WaveQueue q = wave_queue(p);
-        bool overflow = false;
-        for (uint64_t base = (uint64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
-             base < p.n_photons; base += stride) {
-            uint32_t si = p.src_ix;
-            const pp_source src = source_record(p.sources + p.src_ix, si);
-            const uint64_t pid = base + __lane_id();
-            const bool active = pid < p.n_photons && !overflow;
-            HitRec h;
-            const bool hit = transport_group<COUNT>(p, src, si, pid, active, l.spec, search,
-                                                    phase, q, work, n_steps_done, h);
-            const bool stored = store_hits(hit, h, si, p.hits, p.counters);
-            if (!stored) {
-                atomicOr(&p.counters->err, 1u);
-                overflow = true;
-            }
-            wave_done += (unsigned long long)__popcll(__ballot(stored && active));
-            if (__ballot(overflow)) break;
-        }
-    } else {
-        for (uint64_t pid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; pid < p.n_photons;
-             pid += stride) {
-            uint32_t si = p.src_ix;
-            const pp_source src = source_record(p.sources + p.src_ix, si);
-            HitRec h;
-            const bool hit = transport_photon<COUNT>(p, src, si, pid, l.spec, search,
-                                                     phase, work, n_steps_done, h);
-            if (!store_hits(hit, h, si, p.hits, p.counters)) {
-                atomicOr(&p.counters->err, 1u);
+    WaveQueue q{};
+    if constexpr (kDeferredWalk<SEARCH>) q = wave_queue(p);
+    // whole waves of photons, the loop condition uniform across the wave
+    bool overflow = false;
+    for (uint64_t base = (uint64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
+         base < p.n_photons; base += stride) {
+        uint32_t si = p.src_ix;
+        const pp_source src = source_record(p.sources + p.src_ix, si);
+        const uint64_t pid = base + __lane_id();
+        overflow |= !propagate_group<COUNT, SEARCH>(p, src, si, pid, pid < p.n_photons && !overflow,
+                                                    l.spec, search, phase, q, work, n_steps_done);
+        const uint64_t bad = __ballot(overflow);
+        if (bad) {
+            lost += (unsigned long long)__popcll(__ballot(overflow && pid < p.n_photons));
+            if constexpr (kDeferredWalk<SEARCH>) {
+                // the wave ends here: its later groups too
+                for (uint64_t k = base + stride; k < p.n_photons; k += stride)
+                    lost += p.n_photons - k < 64 ? p.n_photons - k : 64;
                 break;
             }
-            ++n_done;
         }
     }
-    flush_counts<COUNT>(p, n_done, wave_done, n_steps_done, work);
+    flush_counts<COUNT>(p, lost, n_steps_done, work);
 }
 
 // Batch of sources in one persistent launch. Work items are chunks of
@@ -640,6 +648,39 @@ struct BatchParams {
     bool dealt;                    // every item by wave index, none from the counter
 };
 
+struct BatchItem {
+    int source;
+    uint64_t first, end;  // its photons
+};
+
+// Work item k of the batch (k wave-uniform).
+__device__ __forceinline__ BatchItem batch_item(const BatchParams& b, uint64_t k) {
+    // chunk c, photons [off, off + len) of it
+    uint64_t c = k;
+    uint32_t off = 0, len = b.chunk;
+    if (k >= b.split_from) {
+        const uint32_t j = (uint32_t)(k - b.split_from);
+        c = b.split_from + j / b.parts;
+        off = (j % b.parts) * b.piece;
+        len = b.chunk - off < b.piece ? b.chunk - off : b.piece;
+    }
+    // source of this chunk: last s with chunk_prefix[s] <= c
+    int lo = 0, hi = b.n_sources - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (load_constant(b.chunk_prefix + mid) <= c) lo = mid;
+        else hi = mid - 1;
+    }
+    BatchItem it;
+    it.source = lo;
+    const uint64_t n_src = load_constant(b.n_photons + lo);
+    const uint64_t first = (c - load_constant(b.chunk_prefix + lo)) * b.chunk + off;
+    // the last chunk's pieces may lie beyond the source's photons
+    it.end = first + len < n_src ? first + len : n_src;
+    it.first = first < it.end ? first : it.end;
+    return it;
+}
+
 template <int PHASE, int SEARCH, bool COUNT = false>
 __global__ void PP_PROPAGATE_ATTRS propagate_batch_kernel(KParams p, BatchParams b) {
     const Lds l = stage_lds<SEARCH>(p);
@@ -651,7 +692,7 @@ __global__ void PP_PROPAGATE_ATTRS propagate_batch_kernel(KParams p, BatchParams
     const uint32_t lane = __lane_id();
     WaveQueue q{};
     if constexpr (kDeferredWalk<SEARCH>) q = wave_queue(p);
-    unsigned long long n_done = 0, wave_done = 0, n_steps_done = 0;
+    unsigned long long lost = 0, n_steps_done = 0;
     pp::Work work;
     bool overflow = false;
     const uint32_t waves = gridDim.x * (blockDim.x >> 6);
@@ -660,65 +701,45 @@ __global__ void PP_PROPAGATE_ATTRS propagate_batch_kernel(KParams p, BatchParams
     for (;;) {
         const uint64_t ck = uniform64(next);
         if (ck >= total) break;
-        // chunk c, photons [off, off + len) of it
-        uint64_t c = ck;
-        uint32_t off = 0, len = b.chunk;
-        if (ck >= b.split_from) {
-            const uint32_t j = (uint32_t)(ck - b.split_from);
-            c = b.split_from + j / b.parts;
-            off = (j % b.parts) * b.piece;
-            len = b.chunk - off < b.piece ? b.chunk - off : b.piece;
-        }
-        // source of this chunk: last s with chunk_prefix[s] <= c
-        int lo = 0, hi = b.n_sources - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (load_constant(b.chunk_prefix + mid) <= c) lo = mid;
-            else hi = mid - 1;
-        }
-        const int si0 = lo;
-        const uint64_t n_src = load_constant(b.n_photons + si0);
-        const uint64_t first = (c - load_constant(b.chunk_prefix + si0)) * b.chunk + off;
-        const uint64_t end = first + len < n_src ? first + len : n_src;
-        for (uint64_t base = first; base < end; base += 64) {
+        const BatchItem it = batch_item(b, ck);
+        for (uint64_t base = it.first; base < it.end; base += 64) {
             // the source index and record, opaque to the optimiser in every
             // iteration: what the emission derives from them is computed here
             // (one scalar reload per 64 photons) instead of being hoisted out
             // of the loop into registers that then spill to scratch
-            uint32_t si = (uint32_t)si0;
-            const pp_source src = source_record(b.sources + si0, si);
+            uint32_t si = (uint32_t)it.source;
+            const pp_source src = source_record(b.sources + it.source, si);
             const uint64_t pid = base + lane;
-            if constexpr (kDeferredWalk<SEARCH>) {
-                const bool active = pid < end && !overflow;
-                HitRec h;
-                const bool hit = transport_group<COUNT>(p, src, (uint32_t)si, pid, active, l.spec,
-                                                        search, phase, q, work, n_steps_done, h);
-                const bool stored = store_hits(hit, h, (uint32_t)si, p.hits, p.counters);
-                if (!stored) {
-                    atomicOr(&p.counters->err, 1u);
-                    overflow = true;
-                }
-                wave_done += (unsigned long long)__popcll(__ballot(stored && active));
-            } else {
-                if (pid >= end || overflow) continue;
-                HitRec h;
-                const bool hit = transport_photon<COUNT>(p, src, (uint32_t)si, pid, l.spec, search,
-                                                         phase, work, n_steps_done, h);
-                if (!store_hits(hit, h, (uint32_t)si, p.hits, p.counters)) {
-                    atomicOr(&p.counters->err, 1u);
-                    overflow = true;
-                    continue;
-                }
-                ++n_done;
-            }
+            overflow |= !propagate_group<COUNT, SEARCH>(p, src, si, pid, pid < it.end && !overflow,
+                                                        l.spec, search, phase, q, work,
+                                                        n_steps_done);
+            lost += (unsigned long long)__popcll(__ballot(overflow && pid < it.end));
         }
-        if (__ballot(overflow)) break;  // the call fails; stop taking chunks
+        if (__ballot(overflow)) {
+            // the call fails; take no more chunks, and give those dealt to this wave up
+            if (b.dealt)
+                for (uint64_t k = ck + waves; k < total; k += waves) {
+                    const BatchItem rest = batch_item(b, k);
+                    lost += rest.end - rest.first;
+                }
+            break;
+        }
         next = ck;
         if (!b.dealt && lane == 0) next = atomicAdd(&p.counters->next_chunk, 1ull);
         next += waves;
     }
-    flush_counts<COUNT>(p, n_done, wave_done, n_steps_done, work);
+    flush_counts<COUNT>(p, lost, n_steps_done, work);
 }
+
+// The counters to pinned host memory, where the host reads them once the stream
+// is done (a copy of their own took 10 us of a call).
+__device__ __forceinline__ void publish(const Counters* c, Counters* host) {
+    const unsigned long long* a = reinterpret_cast<const unsigned long long*>(c);
+    unsigned long long* b = reinterpret_cast<unsigned long long*>(host);
+    if (threadIdx.x < sizeof(Counters) / 8) b[threadIdx.x] = a[threadIdx.x];
+}
+
+__global__ void publish_counters_kernel(const Counters* c, Counters* host) { publish(c, host); }
 
 // Completion of the hit records of the deferred-walk kernels (transport_group):
 // a record holds the photon id, module (target + 1), step k and source. One
@@ -728,7 +749,9 @@ __global__ void PP_PROPAGATE_ATTRS propagate_batch_kernel(KParams p, BatchParams
 // target from the walk's own sphere test on the same operands, and writes
 // position, directions, wavelength, time and distance.
 // sources: the call's source list on the device.
-__global__ void __launch_bounds__(256) replay_hits_kernel(KParams p, const pp_source* sources) {
+__global__ void __launch_bounds__(256) replay_hits_kernel(KParams p, const pp_source* sources,
+                                                          Counters* host) {
+    if (blockIdx.x == 0) publish(p.counters, host);
     const pp::Phase phase = p.med.phase;
     const unsigned long long n_hits = p.counters->n_hits;
     const uint64_t n = n_hits < (unsigned long long)p.hits.capacity ? n_hits : p.hits.capacity;
@@ -953,6 +976,16 @@ bool finite3(const float* v) {
 
 }  // namespace
 
+// What the automatic block size of a launch depends on.
+struct OccKey {
+    const void* fn = nullptr;
+    size_t queue_off = 0, lds = 0;
+    bool grid = false;
+    bool operator==(const OccKey& o) const {
+        return fn == o.fn && queue_off == o.queue_off && lds == o.lds && grid == o.grid;
+    }
+};
+
 struct pp_ctx {
     int device = 0;
     int n_cu = 0;
@@ -961,7 +994,8 @@ struct pp_ctx {
     pp_config cfg{};
     void* hit_mem = nullptr;
     HitCols hits{};
-    Counters* d_counters = nullptr;
+    Counters* d_counters = nullptr;  // at the front of d_batch
+    Counters* h_counters = nullptr;  // pinned: the last propagation's, written by its last kernel
     bool has_medium = false;
     pp_medium medium_in{};
     pp::Medium medium{};
@@ -1005,11 +1039,19 @@ struct pp_ctx {
     size_t d_sort_cap = 0;
     bool sorted_valid = false;  // d_sort holds the sorted records of the last propagation
     int32_t last_n_sources = 0;
-    // source table of the persistent batch kernel: device copy and pinned
-    // host staging, laid out sources | photon counts | chunk prefix
-    void* d_batch = nullptr;
-    void* h_batch = nullptr;
-    size_t batch_cap = 0;  // bytes of each
+    // one propagation's table: device copy and pinned host staging, laid out
+    // counters (uploaded as zeros: one copy clears them and brings the sources) |
+    // sources | photon counts | chunk prefix
+    char* d_batch = nullptr;
+    char* h_batch = nullptr;
+    size_t batch_cap = 0;     // bytes of each
+    bool table_busy = false;  // a copy of h_batch may still be under way
+    // the last batch launch, for the photons that an overflow left untaken
+    BatchParams last_batch{};
+    uint64_t last_waves = 0, last_items = 0;
+    // block size and resident blocks of the last launch shape (OccKey)
+    OccKey occ_key{};
+    int occ_block = 0;
     // PMT detection of the context's hits: targets as (x, y, z, radius), and
     // one device block holding the acceptance table | PMT ids
     float4* d_tgt_r = nullptr;
@@ -1020,6 +1062,7 @@ struct pp_ctx {
     hipGraphExec_t graph_exec = nullptr;
     hipGraphNode_t graph_prop = nullptr;
     const void* graph_fn = nullptr;
+    const Counters* graph_counters = nullptr;
     unsigned graph_blocks = 0, graph_block = 0;
     size_t graph_lds = 0;
 };
@@ -1128,20 +1171,58 @@ int max_resident_blocks(pp_ctx* c, const void* fn, int block, size_t lds, int64_
     return PP_OK;
 }
 
-// The context's source table (device) and its pinned staging, grown to at
-// least `bytes`; waits for the stream first, since earlier work may read them.
+constexpr size_t kTableSources = 256;  // offset of the sources in the table, after the counters
+static_assert(sizeof(Counters) <= kTableSources, "counters precede the sources");
+
+// The context's table (device) and its pinned staging, grown to at least
+// `bytes`, the staged counters zeroed. Waits for the stream where earlier work
+// may still read them (a call that failed half way).
 int ensure_batch_table(pp_ctx* c, size_t bytes) {
-    PP_HIP(hipStreamSynchronize(c->stream));
-    if (bytes <= c->batch_cap) return PP_OK;
-    if (c->d_batch) PP_HIP(hipFree(c->d_batch));
-    if (c->h_batch) PP_HIP(hipHostFree(c->h_batch));
-    c->d_batch = c->h_batch = nullptr;
-    c->batch_cap = 0;
-    const size_t cap = std::max<size_t>(bytes, 64 * 1024);
-    PP_HIP(hipMalloc(&c->d_batch, cap));
-    PP_HIP(hipHostMalloc(&c->h_batch, cap, hipHostMallocDefault));
-    c->batch_cap = cap;
+    if (c->table_busy) PP_HIP(hipStreamSynchronize(c->stream));
+    c->table_busy = false;
+    if (bytes > c->batch_cap) {
+        if (c->d_batch) PP_HIP(hipFree(c->d_batch));
+        if (c->h_batch) PP_HIP(hipHostFree(c->h_batch));
+        c->d_batch = c->h_batch = nullptr;
+        c->d_counters = nullptr;
+        c->batch_cap = 0;
+        const size_t cap = std::max<size_t>(bytes, 64 * 1024);
+        PP_HIP(hipMalloc((void**)&c->d_batch, cap));
+        PP_HIP(hipHostMalloc((void**)&c->h_batch, cap, hipHostMallocDefault));
+        c->batch_cap = cap;
+        c->d_counters = (Counters*)c->d_batch;
+    }
+    std::memset(c->h_batch, 0, kTableSources);
     return PP_OK;
+}
+
+// The staged table to the device
+int upload_batch_table(pp_ctx* c, size_t bytes) {
+    c->table_busy = true;
+    PP_HIP(hipMemcpyAsync(c->d_batch, c->h_batch, bytes, hipMemcpyHostToDevice, c->stream));
+    return PP_OK;
+}
+
+// Photons of the items that no wave took before every wave had met the overflow
+// (taken from the counter: item waves + next_chunk on).
+uint64_t photons_not_taken(const pp_ctx* c, const Counters& hc, const std::vector<uint64_t>& nph) {
+    const BatchParams& b = c->last_batch;
+    uint64_t n = 0;
+    if (c->last_items == 0 || b.dealt) return 0;
+    size_t s = 0;
+    uint64_t chunk0 = 0;  // first chunk of source s
+    for (uint64_t k = c->last_waves + hc.next_chunk; k < c->last_items; ++k) {
+        uint64_t ch = k, off = 0, len = b.chunk;
+        if (k >= b.split_from) {
+            ch = b.split_from + (k - b.split_from) / b.parts;
+            off = (k - b.split_from) % b.parts * b.piece;
+            len = std::min<uint64_t>(b.chunk - off, b.piece);
+        }
+        for (uint64_t m; ch >= chunk0 + (m = (nph[s] + b.chunk - 1) / b.chunk); ++s) chunk0 += m;
+        const uint64_t first = (ch - chunk0) * b.chunk + off;
+        if (first < nph[s]) n += std::min(len, nph[s] - first);
+    }
+    return n;
 }
 
 // The persistent kernel of a search kind and phase: the one whose occupancy
@@ -1158,7 +1239,7 @@ const void* batch_kernel_fn(int skind, int phase) {
 }
 
 // One launch per source, as src/photon_prop_cuda.jl:925-944.
-int launch_per_source(pp_ctx* c, KParams kp, const pp_source* sources,
+int launch_per_source(pp_ctx* c, KParams& kp, const pp_source* sources,
                       const std::vector<uint64_t>& nph, int skind, int phase, bool count, size_t lds) {
     using KernelFn = void (*)(KParams);
 #define PP_K(PH, S, C) propagate_kernel<PH, S, C>
@@ -1176,12 +1257,12 @@ int launch_per_source(pp_ctx* c, KParams kp, const pp_source* sources,
     int64_t max_blocks = 0;
     if (int rc = max_resident_blocks(c, (const void*)kern, block, lds, max_blocks)) return rc;
     // the source list on the device (the kernels read their source from it)
-    const size_t bytes = nph.size() * sizeof(pp_source);
+    const size_t bytes = kTableSources + nph.size() * sizeof(pp_source);
     if (int rc = ensure_batch_table(c, bytes)) return rc;
-    std::memcpy(c->h_batch, sources, bytes);
-    PP_HIP(hipMemcpyAsync(c->d_batch, c->h_batch, bytes, hipMemcpyHostToDevice, c->stream));
-    kp.sources = (const pp_source*)c->d_batch;
-    PP_HIP(hipMemsetAsync(c->d_counters, 0, sizeof(Counters), c->stream));
+    if (!nph.empty()) std::memcpy(c->h_batch + kTableSources, sources, bytes - kTableSources);
+    if (int rc = upload_batch_table(c, bytes)) return rc;
+    kp.sources = (const pp_source*)(c->d_batch + kTableSources);
+    kp.counters = c->d_counters;
     PP_HIP(hipEventRecord(c->ev0, c->stream));
     for (size_t i = 0; i < nph.size(); ++i) {
         if (nph[i] == 0) continue;
@@ -1198,7 +1279,7 @@ int launch_per_source(pp_ctx* c, KParams kp, const pp_source* sources,
 
 // The whole source list in one persistent launch (propagate_batch_kernel);
 // with use_graph, as a hipGraph of counter clear + propagation.
-int launch_batch(pp_ctx* c, const KParams& kp, const pp_source* sources,
+int launch_batch(pp_ctx* c, KParams& kp, const pp_source* sources,
                  const std::vector<uint64_t>& nph, int skind, int phase, bool count, size_t lds,
                  bool use_graph) {
     using BatchFn = void (*)(KParams, BatchParams);
@@ -1218,7 +1299,9 @@ int launch_batch(pp_ctx* c, const KParams& kp, const pp_source* sources,
     for (uint64_t v : nph) total_ph += v;
     if (total_ph == 0) {
         // nothing to run; the counters still have to read zero
-        PP_HIP(hipMemsetAsync(c->d_counters, 0, sizeof(Counters), c->stream));
+        if (int rc = ensure_batch_table(c, kTableSources)) return rc;
+        if (int rc = upload_batch_table(c, kTableSources)) return rc;
+        kp.counters = c->d_counters;
         PP_HIP(hipEventRecord(c->ev0, c->stream));
         return PP_OK;
     }
@@ -1245,13 +1328,13 @@ int launch_batch(pp_ctx* c, const KParams& kp, const pp_source* sources,
         else
             chunk = std::min<uint64_t>(std::max<uint64_t>(per_wave / 32 / 64 * 64, 384), 8192);
     }
-    // table: sources | photon counts | chunk prefix, each 256-byte aligned
-    const size_t off_n = ((n * sizeof(pp_source)) + 255) & ~(size_t)255;
+    // table: counters | sources | photon counts | chunk prefix, each 256-byte aligned
+    const size_t off_n = (kTableSources + n * sizeof(pp_source) + 255) & ~(size_t)255;
     const size_t off_p = off_n + ((n * 8 + 255) & ~(size_t)255);
     const size_t bytes = off_p + (n + 1) * 8;
     if (int rc = ensure_batch_table(c, bytes)) return rc;
-    char* h = (char*)c->h_batch;
-    std::memcpy(h, sources, n * sizeof(pp_source));
+    char* h = c->h_batch;
+    std::memcpy(h + kTableSources, sources, n * sizeof(pp_source));
     uint64_t* hn = (uint64_t*)(h + off_n);
     uint64_t* hp = (uint64_t*)(h + off_p);
     hp[0] = 0;
@@ -1260,9 +1343,10 @@ int launch_batch(pp_ctx* c, const KParams& kp, const pp_source* sources,
         hp[i + 1] = hp[i] + (nph[i] + chunk - 1) / chunk;
     }
     const uint64_t n_chunks = hp[n];
-    char* d = (char*)c->d_batch;
+    char* d = c->d_batch;
+    kp.counters = c->d_counters;
     BatchParams bp{};
-    bp.sources = (const pp_source*)d;
+    bp.sources = (const pp_source*)(d + kTableSources);
     bp.n_photons = (const uint64_t*)(d + off_n);
     bp.chunk_prefix = (const uint64_t*)(d + off_p);
     bp.n_sources = (int32_t)n;
@@ -1285,9 +1369,11 @@ int launch_batch(pp_ctx* c, const KParams& kp, const pp_source* sources,
     const int64_t want = (int64_t)((n_items + block / 64 - 1) / (block / 64));
     const unsigned blocks = (unsigned)std::min<int64_t>(want, max_blocks);
     bp.dealt = dealt;
-    PP_HIP(hipMemcpyAsync(c->d_batch, c->h_batch, bytes, hipMemcpyHostToDevice, c->stream));
+    c->last_batch = bp;
+    c->last_waves = (uint64_t)blocks * (block / 64);
+    c->last_items = n_items;
+    if (int rc = upload_batch_table(c, bytes)) return rc;
     if (!use_graph) {
-        PP_HIP(hipMemsetAsync(c->d_counters, 0, sizeof(Counters), c->stream));
         PP_HIP(hipEventRecord(c->ev0, c->stream));
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(block), lds, c->stream, kp, bp);
         PP_HIP(hipGetLastError());
@@ -1303,7 +1389,8 @@ int launch_batch(pp_ctx* c, const KParams& kp, const pp_source* sources,
     np.sharedMemBytes = (unsigned)lds;
     np.kernelParams = args;
     np.extra = nullptr;
-    const bool same_shape = c->graph_exec && c->graph_fn == (const void*)kern &&
+    // (a table that has grown since moves the counters: the clear node's argument)
+    const bool same_shape = c->graph_exec && c->graph_counters == c->d_counters && c->graph_fn == (const void*)kern &&
                             c->graph_blocks == blocks && c->graph_block == (unsigned)block &&
                             c->graph_lds == lds;
     bool updated = false;
@@ -1331,6 +1418,7 @@ int launch_batch(pp_ctx* c, const KParams& kp, const pp_source* sources,
         PP_HIP(hipGraphAddKernelNode(&c->graph_prop, c->graph, &clear, 1, &np));
         PP_HIP(hipGraphInstantiate(&c->graph_exec, c->graph, nullptr, nullptr, 0));
         c->graph_fn = (const void*)kern;
+        c->graph_counters = c->d_counters;
         c->graph_blocks = blocks;
         c->graph_block = (unsigned)block;
         c->graph_lds = lds;
@@ -1425,7 +1513,7 @@ int pp_create(pp_ctx** out, int device, int64_t hit_capacity, const pp_config* c
     }
     ctx->hits.rec = (HitRecord*)ctx->hit_mem;
     ctx->hits.capacity = cap;
-    if (hipMalloc(&ctx->d_counters, sizeof(Counters)) != hipSuccess)
+    if (hipHostMalloc((void**)&ctx->h_counters, sizeof(Counters), hipHostMallocDefault) != hipSuccess)
         return cleanup(fail(PP_ERR_NOMEM, "pp_create: counters"));
     *out = ctx;
     return PP_OK;
@@ -1436,7 +1524,7 @@ int pp_destroy(pp_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->hit_mem) (void)hipFree(ctx->hit_mem);
-    if (ctx->d_counters) (void)hipFree(ctx->d_counters);
+    if (ctx->h_counters) (void)hipHostFree(ctx->h_counters);
     if (ctx->d_spec) (void)hipFree(ctx->d_spec);
     if (ctx->d_targets) (void)hipFree(ctx->d_targets);
     if (ctx->d_cells) (void)hipFree(ctx->d_cells);
@@ -1695,8 +1783,10 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
     // (1000 targets: 768 threads, two workgroups of 12 waves, where 256 and
     // 512 threads leave 16 waves.)
     int block = ctx->cfg.block_size;
+    const OccKey key{batch_kernel_fn(skind, ctx->medium.phase.kind), queue_off, lds, grid};
+    if (block == 0 && key == ctx->occ_key) block = ctx->occ_block;
     if (block == 0) {
-        const void* fn = batch_kernel_fn(skind, ctx->medium.phase.kind);
+        const void* fn = key.fn;
         int best_waves = 0;
         for (int b : {256, 384, 512, 768, 1024}) {
             const size_t need = grid ? queue_off + (size_t)(b / 64) * kWaveQueueBytes : lds;
@@ -1711,6 +1801,8 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
             }
         }
         if (block == 0) block = 64;  // the LDS check below reports what does not fit
+        ctx->occ_key = key;
+        ctx->occ_block = block;
     }
     ctx->block = block;
     if (grid) lds = queue_off + (size_t)(block / 64) * kWaveQueueBytes;
@@ -1740,7 +1832,6 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
     kp.spec_lastf = (float)(ctx->spec_n - 1);
     kp.spec = ctx->d_spec;
     kp.hits = ctx->hits;
-    kp.counters = ctx->d_counters;
     // photon count of src/photon_prop_cuda.jl:456 (Float32 product)
     std::vector<uint64_t> nph((size_t)n_sources);
     for (int i = 0; i < n_sources; ++i) {
@@ -1752,6 +1843,7 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
         nph[(size_t)i] = prod > 0.0f ? (uint64_t)prod : 0;
     }
     ctx->n_launch = 0;
+    ctx->last_items = 0;
     const int mode = ctx->cfg.batch_mode == PP_BATCH_AUTO ? PP_BATCH_PERSISTENT : ctx->cfg.batch_mode;
     if (mode == PP_BATCH_PER_SOURCE) {
         if (int rc = launch_per_source(ctx, kp, sources, nph, skind, phase, count, lds)) return rc;
@@ -1762,16 +1854,22 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
     // the grid kernels leave their hit records to be completed
     if (skind == kSearchGrid || skind == kSearchGridGlobal) {
         hipLaunchKernelGGL(replay_hits_kernel, dim3((unsigned)(4 * ctx->n_cu)), dim3(256), 0,
-                           ctx->stream, kp, (const pp_source*)ctx->d_batch);
-        PP_HIP(hipGetLastError());
+                           ctx->stream, kp, (const pp_source*)(ctx->d_batch + kTableSources),
+                           ctx->h_counters);
+    } else {
+        hipLaunchKernelGGL(publish_counters_kernel, dim3(1), dim3(64), 0, ctx->stream, kp.counters,
+                           ctx->h_counters);
     }
+    PP_HIP(hipGetLastError());
     PP_HIP(hipEventRecord(ctx->ev1, ctx->stream));
-    Counters hc{};
-    PP_HIP(hipMemcpyAsync(&hc, ctx->d_counters, sizeof hc, hipMemcpyDeviceToHost, ctx->stream));
     PP_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->table_busy = false;
+    const Counters hc = *ctx->h_counters;
     PP_HIP(hipEventElapsedTime(&ctx->last_ms, ctx->ev0, ctx->ev1));
     ctx->n_hits = (int64_t)std::min<unsigned long long>(hc.n_hits, ctx->hits.capacity);
-    ctx->n_ph_sim = (int64_t)hc.n_ph_sim;
+    uint64_t n_sim = 0;
+    for (uint64_t v : nph) n_sim += v;
+    ctx->n_ph_sim = (int64_t)(n_sim - hc.n_lost - (hc.err ? photons_not_taken(ctx, hc, nph) : 0));
     ctx->work_steps = (int64_t)hc.steps;
     ctx->work_tests = (int64_t)hc.tests;
     ctx->work_cells = (int64_t)hc.cells;
@@ -1946,6 +2044,48 @@ __global__ void gather_hits_kernel(const HitRecord* __restrict__ rec,
     dst[3] = d;
 }
 
+// The order of up to kRankMost hits in one launch: the rank of a hit is the
+// number of keys below its own (keys are unique), and its record goes straight to
+// that place, in device memory and, where `host` is set, in pinned host memory
+// too (the copy of a small hit table). 64 hits per workgroup, the keys in tiles
+// of LDS, a quarter of each tile per wave. For a few thousand hits the radix sort
+// is five launches of a few workgroups and the copy a sixth: 25-45 us of a call
+// for the README example's 14 hits or a small shower's 1200; 3-9 us here. The
+// compares grow with the square of the count, and at 4096 the two are near.
+constexpr int kRankMost = 4096;
+
+__global__ void __launch_bounds__(256) rank_hits_kernel(const HitRecord* __restrict__ rec, int n,
+                                                        HitRecord* __restrict__ out,
+                                                        HitRecord* __restrict__ host) {
+    __shared__ uint64_t key[1024];
+    __shared__ uint32_t part[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int k = blockIdx.x * 64 + lane;
+    auto key_of = [&](int i) {
+        return ((uint64_t)(uint32_t)rec[i].source_ix << kPidBits) |
+               (rec[i].id & (kMaxPhotonsPerSource - 1));
+    };
+    const uint64_t own = k < n ? key_of(k) : 0;
+    uint32_t below = 0;
+    for (int t0 = 0; t0 < n; t0 += 1024) {
+        for (int i = threadIdx.x; i < 1024; i += 256)
+            key[i] = t0 + i < n ? key_of(t0 + i) : ~0ull;
+        __syncthreads();
+        const int most = n - t0 < 1024 ? n - t0 : 1024;
+        const int i1 = min((w + 1) * 256, most);
+#pragma unroll 8
+        for (int i = w * 256; i < i1; ++i) below += key[i] < own ? 1u : 0u;
+        __syncthreads();
+    }
+    part[w][lane] = below;
+    __syncthreads();
+    if (k >= n) return;
+    const uint32_t rank = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
+    const uint4 v = reinterpret_cast<const uint4*>(rec + k)[w];  // a quarter of the record each
+    reinterpret_cast<uint4*>(out + rank)[w] = v;
+    if (host) reinterpret_cast<uint4*>(host + rank)[w] = v;
+}
+
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // The hits in (source, photon id) order, written by the device to the front
@@ -1954,12 +2094,33 @@ static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // are unique), then a gather writes the records in that order.  Sets
 // *done = false and does nothing when the keys do not fit 64 bits, the
 // indices 32 bits or the buffer device memory; the caller then sorts on the
-// host.
-static int sort_hits_device(pp_ctx* ctx, bool* done) {
+// host. Up to kRankMost hits are ordered by rank_hits_kernel, to `host` too.
+static int sort_hits_device(pp_ctx* ctx, bool* done, HitRecord* host = nullptr) {
     *done = false;
     const int64_t n = ctx->n_hits;
     const int32_t ns = ctx->last_n_sources;
     if (n <= 0 || n > INT32_MAX || ns <= 0 || ns > (1 << 24)) return PP_OK;
+    auto grow = [&](size_t need) {
+        if (need <= ctx->d_sort_cap) return true;
+        if (ctx->d_sort) (void)hipFree(ctx->d_sort);
+        ctx->d_sort = nullptr;
+        ctx->d_sort_cap = 0;
+        if (hipMalloc((void**)&ctx->d_sort, need) != hipSuccess) {
+            (void)hipGetLastError();  // out of device memory: sort on the host
+            ctx->d_sort = nullptr;
+            return false;
+        }
+        ctx->d_sort_cap = need;
+        return true;
+    };
+    if (n <= kRankMost) {
+        if (!grow(align256((size_t)kRankMost * sizeof(HitRecord)))) return PP_OK;
+        hipLaunchKernelGGL(rank_hits_kernel, dim3((unsigned)((n + 63) / 64)), dim3(256), 0,
+                           ctx->stream, ctx->hits.rec, (int)n, (HitRecord*)ctx->d_sort, host);
+        PP_HIP(hipGetLastError());
+        *done = true;
+        return PP_OK;
+    }
     int end_bit = (int)kPidBits;
     for (uint32_t v = (uint32_t)(ns - 1); v; v >>= 1) ++end_bit;
     size_t temp = 0;
@@ -1969,17 +2130,7 @@ static int sort_hits_device(pp_ctx* ctx, bool* done) {
     const size_t br = align256((size_t)n * sizeof(HitRecord));
     const size_t bk = align256((size_t)n * 8), bv = align256((size_t)n * 4);
     const size_t need = br + 2 * bk + 2 * bv + align256(temp);
-    if (need > ctx->d_sort_cap) {
-        if (ctx->d_sort) PP_HIP(hipFree(ctx->d_sort));
-        ctx->d_sort = nullptr;
-        ctx->d_sort_cap = 0;
-        if (hipMalloc((void**)&ctx->d_sort, need) != hipSuccess) {
-            (void)hipGetLastError();  // out of device memory: sort on the host
-            ctx->d_sort = nullptr;
-            return PP_OK;
-        }
-        ctx->d_sort_cap = need;
-    }
+    if (!grow(need)) return PP_OK;
     char* base = ctx->d_sort + br;
     uint64_t* k_in = (uint64_t*)base;
     uint64_t* k_out = (uint64_t*)(base + bk);
@@ -2009,10 +2160,25 @@ int pp_copy_hits(pp_ctx* ctx, int64_t first, int64_t n, float* pos3, float* dir3
     // deterministic_order: 0 = buffer order, 1 = sorted on the device (host
     // where the device cannot), 2 = sorted on the host (no device buffer)
     const bool ordered = ctx->cfg.deterministic_order != 0;
+    auto ensure_staging = [&](int64_t records) -> int {
+        if (records <= ctx->h_rec_cap) return PP_OK;
+        if (ctx->h_rec) PP_HIP(hipHostFree(ctx->h_rec));
+        ctx->h_rec = nullptr;
+        ctx->h_rec_cap = 0;
+        PP_HIP(hipHostMalloc((void**)&ctx->h_rec, (size_t)records * sizeof(HitRecord),
+                             hipHostMallocDefault));
+        ctx->h_rec_cap = records;
+        return PP_OK;
+    };
+    bool staged = false;  // every ordered record is on its way to h_rec
     if (ordered && ctx->cfg.deterministic_order != 2 && !ctx->sorted_valid && !ctx->perm_valid) {
         bool done = false;
-        if (int rc = sort_hits_device(ctx, &done)) return rc;
+        const bool few = ctx->n_hits <= kRankMost;
+        if (few)
+            if (int rc = ensure_staging(kRankMost)) return rc;
+        if (int rc = sort_hits_device(ctx, &done, few ? ctx->h_rec : nullptr)) return rc;
         ctx->sorted_valid = done;
+        staged = few && done;
     }
     // the host sorts only where the device could not: it then reads every record
     const bool host_sort = ordered && (ctx->cfg.deterministic_order == 2 || !ctx->sorted_valid);
@@ -2023,14 +2189,8 @@ int pp_copy_hits(pp_ctx* ctx, int64_t first, int64_t n, float* pos3, float* dir3
     // kStageRecords records (kept by the context); the host sort, which
     // needs random access to every record, collects them in pageable memory
     const int64_t stage = std::min<int64_t>(cnt, kStageRecords);
-    if (stage > ctx->h_rec_cap) {
-        if (ctx->h_rec) PP_HIP(hipHostFree(ctx->h_rec));
-        ctx->h_rec = nullptr;
-        ctx->h_rec_cap = 0;
-        PP_HIP(hipHostMalloc((void**)&ctx->h_rec, (size_t)stage * sizeof(HitRecord),
-                             hipHostMallocDefault));
-        ctx->h_rec_cap = stage;
-    }
+    if (!staged)
+        if (int rc = ensure_staging(stage)) return rc;
     const uint64_t pid_mask = kMaxPhotonsPerSource - 1;
     auto scatter = [&](const HitRecord& r, int64_t k) {
         for (int c = 0; c < 3; ++c) {
@@ -2051,6 +2211,11 @@ int pp_copy_hits(pp_ctx* ctx, int64_t first, int64_t n, float* pos3, float* dir3
         if (photon_id) photon_id[k] = r.id & pid_mask;
         if (source_ix) source_ix[k] = r.source_ix;
     };
+    if (staged) {
+        PP_HIP(hipStreamSynchronize(ctx->stream));
+        for (int64_t k = 0; k < n; ++k) scatter(ctx->h_rec[first + k], k);
+        return PP_OK;
+    }
     std::vector<HitRecord> all;
     if (host_sort) all.resize((size_t)cnt);
     for (int64_t off = 0; off < cnt; off += stage) {
