@@ -86,6 +86,49 @@ struct PhotonInit {
     pp::MediumValues mv;
 };
 
+// The launch constants that an emission reads.
+struct EmitParams {
+    pp::Medium med;
+    int32_t spec_n, spec_map;
+    float spec_mono, spec_nf, spec_lastf;
+};
+
+// Launch constants read again from the kernel's arguments (KParams, the first
+// one) through scalar loads, opaque to the optimiser: as values of the whole
+// kernel the constants of the emission and of the walk did not fit the scalar
+// registers, and the compiler kept 90 of them in lanes of vector registers,
+// from which it read them back one by one for every group of photons (about 70
+// v_readlane a group) and every batch of walks (7-10). With this and without a
+// move after the last segment a cascade of 1e8 photons takes 7.29 ms of kernel
+// time instead of 7.67, 1e8 photons of a point source 4.8 instead of 5.3.
+#if defined(__HIP_DEVICE_COMPILE__)
+using ConstParams = const __attribute__((address_space(4))) KParams;
+#else
+using ConstParams = const KParams;
+#endif
+
+__device__ __forceinline__ ConstParams* kernel_params() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    ConstParams* c = (ConstParams*)__builtin_amdgcn_kernarg_segment_ptr();
+    __asm__ volatile("" : "+s"(c));
+    return c;
+#else
+    return nullptr;
+#endif
+}
+
+__device__ __forceinline__ EmitParams emit_params() {
+    ConstParams* c = kernel_params();
+    EmitParams e;
+    e.med = c->med;
+    e.spec_n = c->spec_n;
+    e.spec_map = c->spec_map;
+    e.spec_mono = c->spec_mono;
+    e.spec_nf = c->spec_nf;
+    e.spec_lastf = c->spec_lastf;
+    return e;
+}
+
 // p + s d, each component one FMA (the same bits wherever it is inlined)
 __device__ __forceinline__ f3 add_scaled(f3 p, float s, f3 d) {
     return pp::make3(fmaf(s, d.x, p.x), fmaf(s, d.y, p.y), fmaf(s, d.z, p.z));
@@ -109,7 +152,7 @@ __device__ __forceinline__ f3 cherenkov_dir(const pp_source& src, const pp::Medi
     return pp::rot_from_ez(axis, ph);
 }
 
-__device__ __forceinline__ PhotonInit init_photon(const KParams& p, const pp_source& src,
+__device__ __forceinline__ PhotonInit init_photon(const EmitParams& p, const pp_source& src,
                                                   const float* spec, const pp::Stream& s) {
     const uint4 r = s.block(PP_CTR_INIT);
     PhotonInit st;
@@ -221,14 +264,24 @@ __device__ __forceinline__ bool store_hits(bool has_hit, const HitRec& h, uint32
 // ---------------------------------------------------------------------------
 using pp::lds_bytes;
 
-// kSearchGridGlobal: the grid search on tables read from global memory (L2
-// and the vector cache) instead of LDS copies, for target lists whose records
-// and grid tables exceed the LDS
-enum { kSearchBrute = 0, kSearchGrid = 1, kSearchMixed = 2, kSearchGridGlobal = 3 };
+// kSearchGridMem: the grid search with its cells in LDS and its targets read from
+// memory (L2 and the vector cache), where their LDS copy would cost resident waves
+// kSearchGridGlobal: all its tables read from memory, for target lists whose
+// records and grid tables exceed the LDS
+enum {
+    kSearchBrute = 0,
+    kSearchGrid = 1,
+    kSearchMixed = 2,
+    kSearchGridGlobal = 3,
+    kSearchGridMem = 4,
+    kSearchKinds = 5
+};
+template <int SEARCH>
+constexpr bool kLdsCells = SEARCH == kSearchGrid || SEARCH == kSearchGridMem;
 // the grid searches walk in batches (transport_group); the every-target
 // scans test each step at once (transport_photon)
 template <int SEARCH>
-constexpr bool kDeferredWalk = SEARCH == kSearchGrid || SEARCH == kSearchGridGlobal;
+constexpr bool kDeferredWalk = kLdsCells<SEARCH> || SEARCH == kSearchGridGlobal;
 
 // LDS tables of one workgroup: targets, grid cells and items, spectrum knots
 struct Lds {
@@ -253,17 +306,18 @@ __device__ __forceinline__ Lds stage_lds(const KParams& p) {
         return l;
     }
     // a mixed (sphere and planar) list has two records per target
-    const int n_rec = SEARCH == kSearchMixed ? 2 * p.n_targets : p.n_targets;
+    const int n_rec = SEARCH == kSearchGridMem ? 0
+                      : SEARCH == kSearchMixed ? 2 * p.n_targets : p.n_targets;
     float4* const tgt = lds;
     float4* const cells = lds + n_rec;
     uint16_t* const items =
-        reinterpret_cast<uint16_t*>(cells + (SEARCH == kSearchGrid ? 2 * p.grid.n_cells : 0));
-    l.tgt = tgt;
+        reinterpret_cast<uint16_t*>(cells + (kLdsCells<SEARCH> ? 2 * p.grid.n_cells : 0));
+    l.tgt = SEARCH == kSearchGridMem ? p.targets : tgt;
     l.cells = cells;
     l.items = items;
-    l.spec = reinterpret_cast<float*>(items + (SEARCH == kSearchGrid ? ((p.grid.n_items + 1) & ~1) : 0));
+    l.spec = reinterpret_cast<float*>(items + (kLdsCells<SEARCH> ? ((p.grid.n_items + 1) & ~1) : 0));
     for (int i = threadIdx.x; i < n_rec; i += blockDim.x) tgt[i] = p.targets[i];
-    if (SEARCH == kSearchGrid) {
+    if (kLdsCells<SEARCH>) {
         for (int i = threadIdx.x; i < 2 * p.grid.n_cells; i += blockDim.x) cells[i] = p.cells[i];
         for (int i = threadIdx.x; i < p.grid.n_items; i += blockDim.x) items[i] = p.cell_items[i];
     }
@@ -274,18 +328,24 @@ __device__ __forceinline__ Lds stage_lds(const KParams& p) {
 
 template <int SEARCH>
 using SearchT = typename std::conditional<
-    SEARCH == kSearchGrid || SEARCH == kSearchGridGlobal, pp::GridSearch,
+    kDeferredWalk<SEARCH>, pp::GridSearch,
     typename std::conditional<SEARCH == kSearchMixed, pp::MixedSearch, pp::BruteSearch>::type>::type;
 
 template <int SEARCH>
 __device__ __forceinline__ SearchT<SEARCH> make_search(const KParams& p, const Lds& l) {
-    if constexpr (SEARCH == kSearchGrid || SEARCH == kSearchGridGlobal) {
+    if constexpr (kDeferredWalk<SEARCH>) {
         return pp::GridSearch{l.tgt, l.cells, l.items, p.grid};
     } else if constexpr (SEARCH == kSearchMixed) {
         return pp::MixedSearch{l.tgt, p.n_targets};
     } else {
         return pp::BruteSearch{l.tgt, p.n_targets};
     }
+}
+
+// The search with its grid read again (kernel_params), for a batch of walks;
+// the every-target scans hold nothing worth reading again.
+__device__ __forceinline__ pp::GridSearch reread(const pp::GridSearch& s) {
+    return pp::GridSearch{s.tgt, s.cells, s.items, kernel_params()->grid};
 }
 
 // position, distance and time after moving d along dir
@@ -305,7 +365,7 @@ __device__ __forceinline__ bool transport_photon(const KParams& p, const pp_sour
                                                  pp::Work& work, unsigned long long& n_steps_done,
                                                  HitRec& h) {
     pp::Stream s{p.k0, p.k1, (uint32_t)pid, (uint32_t)(pid >> 32), src_ix};
-    const PhotonInit st = init_photon(p, src, spec, s);
+    const PhotonInit st = init_photon(emit_params(), src, spec, s);
     const pp::StepStream ss(s);
     f3 pos = st.pos, dir = st.dir;
     float time = st.time, dist = 0.0f;
@@ -326,6 +386,7 @@ __device__ __forceinline__ bool transport_photon(const KParams& p, const pp_sour
             n_at = step;
             break;
         }
+        if (step == p.n_steps) break;  // nothing follows the last segment
         move_by(pos, dist, time, dir, step_size, inv_c);
         const float ct = pp::phase_cos_words(phase, r.y, r.z);
         dir = pp::update_direction(dir, ct, pp::u01(r.w));
@@ -401,7 +462,7 @@ __device__ __forceinline__ bool transport_group(const KParams& p, const pp_sourc
     float ln2_sca = 0.0f;
     if (active) {
         // only what the steps need stays live; a hit emits the photon again
-        const PhotonInit st = init_photon(p, src, spec, s);
+        const PhotonInit st = init_photon(emit_params(), src, spec, s);
         pos = st.pos;
         dir = st.dir;
         ln2_sca = st.mv.sca_len * pp::kLn2;
@@ -421,6 +482,7 @@ __device__ __forceinline__ bool transport_group(const KParams& p, const pp_sourc
     // every lane walks one pending job (lanes >= n none)
     auto walk_jobs = [&](uint32_t n) {
         wave_sync();
+        const auto grid = reread(search);
         int found = -1;
         float dt = 0.0f;
         unsigned long long key = 0;
@@ -432,7 +494,7 @@ __device__ __forceinline__ bool transport_group(const KParams& p, const pp_sourc
             const uint32_t meta = __float_as_uint(b.w);
             owner = meta & 63u;
             if (COUNT) work.walks += 1;
-            found = search.template find<COUNT>(pp::make3(a.x, a.y, a.z), pp::make3(b.x, b.y, b.z),
+            found = grid.template find<COUNT>(pp::make3(a.x, a.y, a.z), pp::make3(b.x, b.y, b.z),
                                                 a.w, dt, work);
             if (found >= 0) {
                 key = ((unsigned long long)(meta >> 6) << 16) | (uint32_t)found;
@@ -480,7 +542,8 @@ __device__ __forceinline__ bool transport_group(const KParams& p, const pp_sourc
                 make_float4(dir.x, dir.y, dir.z, __uint_as_float(lane | ((uint32_t)step << 6)));
         }
         count += n_new;
-        if (__builtin_amdgcn_inverse_ballot_w64(move_m)) {
+        // nothing follows the last segment
+        if (step < p.n_steps && __builtin_amdgcn_inverse_ballot_w64(move_m)) {
             pos = next;
             const float ct = pp::phase_cos_words(phase, r.y, r.z);
             dir = pp::update_direction(dir, ct, pp::u01(r.w));
@@ -528,12 +591,14 @@ __device__ __forceinline__ void flush_counts(const KParams& p, unsigned long lon
 // COUNT: instrumented variant that also counts photon steps, sphere tests
 // and grid-cell visits (roofline accounting); the results are identical.
 // Minimum waves per SIMD the register allocation must allow (the VGPR budget
-// is 512 / waves per lane).
-#ifndef PP_WAVES_PER_EU
-#define PP_WAVES_PER_EU 6
-#endif
+// is 512 / waves per lane): 7 for the grid searches, whose walks wait for LDS
+// (1e8-photon cascade on 320 targets: 7.07 ms, at 6 7.29, at 8 8.15; the
+// 256-source batch on 1000 targets: 25.7, at 6 25.9, at 8 29.8, at 5 36.9),
+// 6 for the every-target scans.
+template <int SEARCH>
+constexpr int kWavesPerSimd = kDeferredWalk<SEARCH> ? 7 : 6;
 #define PP_PROPAGATE_ATTRS \
-    __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(PP_WAVES_PER_EU)))
+    __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<SEARCH>)))
 
 // x of the wave's first lane, as a scalar
 __device__ __forceinline__ uint64_t uniform64(uint64_t x) {
@@ -767,7 +832,7 @@ __global__ void __launch_bounds__(256) replay_hits_kernel(KParams p, const pp_so
         const pp_source src = sources[si];
         const pp::Stream s{p.k0, p.k1, (uint32_t)pid, (uint32_t)(pid >> 32), si};
         const pp::StepStream ss(s);
-        const PhotonInit st = init_photon(p, src, p.spec, s);
+        const PhotonInit st = init_photon(emit_params(), src, p.spec, s);
         const float ln2_sca = st.mv.sca_len * pp::kLn2, inv_c = st.mv.inv_c_grp;
         f3 rp = st.pos, rd = st.dir;
         float rt = st.time, rdist = 0.0f;
@@ -979,11 +1044,8 @@ bool finite3(const float* v) {
 // What the automatic block size of a launch depends on.
 struct OccKey {
     const void* fn = nullptr;
-    size_t queue_off = 0, lds = 0;
-    bool grid = false;
-    bool operator==(const OccKey& o) const {
-        return fn == o.fn && queue_off == o.queue_off && lds == o.lds && grid == o.grid;
-    }
+    size_t tables = 0;
+    bool operator==(const OccKey& o) const { return fn == o.fn && tables == o.tables; }
 };
 
 struct pp_ctx {
@@ -1049,9 +1111,9 @@ struct pp_ctx {
     // the last batch launch, for the photons that an overflow left untaken
     BatchParams last_batch{};
     uint64_t last_waves = 0, last_items = 0;
-    // block size and resident blocks of the last launch shape (OccKey)
+    // automatic block size and search kind of the last launch shape
     OccKey occ_key{};
-    int occ_block = 0;
+    int occ_block = 0, occ_skind = 0;
     // PMT detection of the context's hits: targets as (x, y, z, radius), and
     // one device block holding the acceptance table | PMT ids
     float4* d_tgt_r = nullptr;
@@ -1231,8 +1293,9 @@ const void* batch_kernel_fn(int skind, int phase) {
     using BatchFn = void (*)(KParams, BatchParams);
 #define PP_K(PH, S) propagate_batch_kernel<PH, S, false>
 #define PP_K3(S) {PP_K(PP_PHASE_HG, S), PP_K(PP_PHASE_MIXED_HG_ES, S), PP_K(PP_PHASE_MIXED_HG_SL, S)}
-    static const BatchFn kKernels[4][3] = {PP_K3(kSearchBrute), PP_K3(kSearchGrid),
-                                           PP_K3(kSearchMixed), PP_K3(kSearchGridGlobal)};
+    static const BatchFn kKernels[kSearchKinds][3] = {
+        PP_K3(kSearchBrute), PP_K3(kSearchGrid), PP_K3(kSearchMixed), PP_K3(kSearchGridGlobal),
+        PP_K3(kSearchGridMem)};
 #undef PP_K3
 #undef PP_K
     return (const void*)kKernels[skind][phase];
@@ -1245,11 +1308,11 @@ int launch_per_source(pp_ctx* c, KParams& kp, const pp_source* sources,
 #define PP_K(PH, S, C) propagate_kernel<PH, S, C>
 #define PP_K3(S, C) {PP_K(PP_PHASE_HG, S, C), PP_K(PP_PHASE_MIXED_HG_ES, S, C), PP_K(PP_PHASE_MIXED_HG_SL, S, C)}
     // [count][search kind][phase kind]
-    static const KernelFn kKernels[2][4][3] = {
+    static const KernelFn kKernels[2][kSearchKinds][3] = {
         {PP_K3(kSearchBrute, false), PP_K3(kSearchGrid, false), PP_K3(kSearchMixed, false),
-         PP_K3(kSearchGridGlobal, false)},
+         PP_K3(kSearchGridGlobal, false), PP_K3(kSearchGridMem, false)},
         {PP_K3(kSearchBrute, true), PP_K3(kSearchGrid, true), PP_K3(kSearchMixed, true),
-         PP_K3(kSearchGridGlobal, true)}};
+         PP_K3(kSearchGridGlobal, true), PP_K3(kSearchGridMem, true)}};
 #undef PP_K3
 #undef PP_K
     const KernelFn kern = kKernels[count][skind][phase];
@@ -1285,11 +1348,11 @@ int launch_batch(pp_ctx* c, KParams& kp, const pp_source* sources,
     using BatchFn = void (*)(KParams, BatchParams);
 #define PP_K(PH, S, C) propagate_batch_kernel<PH, S, C>
 #define PP_K3(S, C) {PP_K(PP_PHASE_HG, S, C), PP_K(PP_PHASE_MIXED_HG_ES, S, C), PP_K(PP_PHASE_MIXED_HG_SL, S, C)}
-    static const BatchFn kKernels[2][4][3] = {
+    static const BatchFn kKernels[2][kSearchKinds][3] = {
         {PP_K3(kSearchBrute, false), PP_K3(kSearchGrid, false), PP_K3(kSearchMixed, false),
-         PP_K3(kSearchGridGlobal, false)},
+         PP_K3(kSearchGridGlobal, false), PP_K3(kSearchGridMem, false)},
         {PP_K3(kSearchBrute, true), PP_K3(kSearchGrid, true), PP_K3(kSearchMixed, true),
-         PP_K3(kSearchGridGlobal, true)}};
+         PP_K3(kSearchGridGlobal, true), PP_K3(kSearchGridMem, true)}};
 #undef PP_K3
 #undef PP_K
     const BatchFn kern = kKernels[count][skind][phase];
@@ -1765,51 +1828,68 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
     }
     const bool grid = search == PP_SEARCH_GRID;
     const bool global = grid && ctx->grid_global;
-    const int skind = global ? kSearchGridGlobal
-                      : grid ? kSearchGrid : ctx->planar ? kSearchMixed : kSearchBrute;
-    // the global grid stages only the spectrum
-    size_t lds = global ? std::max<size_t>((size_t)ctx->spec_n * 4, 16)
-                        : lds_bytes(ctx->planar ? 2 * ctx->n_targets : ctx->n_targets,
-                                    grid ? ctx->grid.n_cells : 0,
-                                    grid ? ctx->grid.n_items : 0, ctx->spec_n, grid);
+    int skind = global ? kSearchGridGlobal
+                : grid ? kSearchGrid : ctx->planar ? kSearchMixed : kSearchBrute;
+    const int phase = ctx->medium.phase.kind;
+    // LDS tables of a search: the global grid stages only the spectrum
+    auto table_bytes = [&](int kind) {
+        if (kind == kSearchGridGlobal) return std::max<size_t>((size_t)ctx->spec_n * 4, 16);
+        const int n = kind == kSearchGridMem ? 0 : ctx->planar ? 2 * ctx->n_targets : ctx->n_targets;
+        return lds_bytes(n, grid ? ctx->grid.n_cells : 0, grid ? ctx->grid.n_items : 0, ctx->spec_n,
+                         grid);
+    };
     // the grid kernels' per-wave walk queues follow the tables
-    const uint32_t queue_off = (uint32_t)((lds + 15) & ~(size_t)15);
+    auto with_queues = [&](size_t tables, int threads) {
+        return grid ? ((tables + 15) & ~(size_t)15) + (size_t)(threads / 64) * kWaveQueueBytes
+                    : tables;
+    };
     // block size: the set one or, for 0, the one of 256, 384, 512, 768 and 1024
     // threads with the most waves resident per CU: the runtime's occupancy
-    // query (registers: 6 waves per SIMD) and the LDS a workgroup needs (the
+    // query (registers: 6 or 7 waves per SIMD) and the LDS a workgroup needs (the
     // tables once and, with a grid, a walk queue per wave) in 512-byte
     // allocation units, which the query does not apply (it reports three
     // workgroups of 54320 bytes, and they run as two); the smallest on a tie.
-    // (1000 targets: 768 threads, two workgroups of 12 waves, where 256 and
-    // 512 threads leave 16 waves.)
+    // A grid search leaves its targets in memory where that makes room for more
+    // waves: 1000 targets, 16 KB, leave 24 waves in 768-thread blocks (27.0 ms
+    // for the 256-source batch) and 28 in 256-thread blocks without them (25.8
+    // ms); 320 targets leave 28 either way, and are read from LDS (1e8-photon
+    // cascade: 7.07 ms, from memory 7.27).
     int block = ctx->cfg.block_size;
-    const OccKey key{batch_kernel_fn(skind, ctx->medium.phase.kind), queue_off, lds, grid};
-    if (block == 0 && key == ctx->occ_key) block = ctx->occ_block;
     if (block == 0) {
-        const void* fn = key.fn;
-        int best_waves = 0;
-        for (int b : {256, 384, 512, 768, 1024}) {
-            const size_t need = grid ? queue_off + (size_t)(b / 64) * kWaveQueueBytes : lds;
-            if (need > (size_t)kMaxLdsBytes) continue;
-            int occ = 0;
-            PP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, b, need));
-            const size_t alloc = (need + 511) & ~(size_t)511;
-            occ = std::min<int>(occ, (int)((size_t)kMaxLdsBytes / alloc));
-            if (occ * (b / 64) > best_waves) {
-                best_waves = occ * (b / 64);
-                block = b;
+        const OccKey key{batch_kernel_fn(skind, phase), table_bytes(skind)};
+        if (!(key == ctx->occ_key)) {
+            int best_waves = 0;
+            ctx->occ_block = 64;  // the LDS check below reports what does not fit
+            ctx->occ_skind = skind;
+            for (int kind : {skind, (int)kSearchGridMem}) {
+                if (kind != skind && skind != kSearchGrid) continue;
+                const void* fn = batch_kernel_fn(kind, phase);
+                for (int b : {256, 384, 512, 768, 1024}) {
+                    const size_t need = with_queues(table_bytes(kind), b);
+                    if (need > (size_t)kMaxLdsBytes) continue;
+                    int occ = 0;
+                    PP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, b, need));
+                    const size_t alloc = (need + 511) & ~(size_t)511;
+                    occ = std::min<int>(occ, (int)((size_t)kMaxLdsBytes / alloc));
+                    if (occ * (b / 64) > best_waves) {
+                        best_waves = occ * (b / 64);
+                        ctx->occ_block = b;
+                        ctx->occ_skind = kind;
+                    }
+                }
             }
+            ctx->occ_key = key;
         }
-        if (block == 0) block = 64;  // the LDS check below reports what does not fit
-        ctx->occ_key = key;
-        ctx->occ_block = block;
+        block = ctx->occ_block;
+        skind = ctx->occ_skind;
     }
+    const size_t tables = table_bytes(skind);
+    const uint32_t queue_off = (uint32_t)((tables + 15) & ~(size_t)15);
+    const size_t lds = with_queues(tables, block);
     ctx->block = block;
-    if (grid) lds = queue_off + (size_t)(block / 64) * kWaveQueueBytes;
     if (lds > (size_t)kMaxLdsBytes)
         return fail(PP_ERR_INVALID, "pp_propagate: targets, tables and walk queues exceed the LDS "
                                     "of a workgroup (a smaller block_size may fit)");
-    const int phase = ctx->medium.phase.kind;
     const bool count = ctx->cfg.count_work != 0;
     ctx->last_search = search;
     KParams kp{};
@@ -1852,7 +1932,7 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
             return rc;
     }
     // the grid kernels leave their hit records to be completed
-    if (skind == kSearchGrid || skind == kSearchGridGlobal) {
+    if (grid) {
         hipLaunchKernelGGL(replay_hits_kernel, dim3((unsigned)(4 * ctx->n_cu)), dim3(256), 0,
                            ctx->stream, kp, (const pp_source*)(ctx->d_batch + kTableSources),
                            ctx->h_counters);
