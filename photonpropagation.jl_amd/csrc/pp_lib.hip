@@ -1044,8 +1044,10 @@ bool finite3(const float* v) {
 // What the automatic block size of a launch depends on.
 struct OccKey {
     const void* fn = nullptr;
-    size_t tables = 0;
-    bool operator==(const OccKey& o) const { return fn == o.fn && tables == o.tables; }
+    size_t tables = 0, mem_tables = 0;  // LDS tables with and without the targets
+    bool operator==(const OccKey& o) const {
+        return fn == o.fn && tables == o.tables && mem_tables == o.mem_tables;
+    }
 };
 
 struct pp_ctx {
@@ -1266,23 +1268,23 @@ int upload_batch_table(pp_ctx* c, size_t bytes) {
 }
 
 // Photons of the items that no wave took before every wave had met the overflow
-// (taken from the counter: item waves + next_chunk on).
+// (taken from the counter: item waves + next_chunk on), a source at a time.
 uint64_t photons_not_taken(const pp_ctx* c, const Counters& hc, const std::vector<uint64_t>& nph) {
     const BatchParams& b = c->last_batch;
-    uint64_t n = 0;
-    if (c->last_items == 0 || b.dealt) return 0;
-    size_t s = 0;
-    uint64_t chunk0 = 0;  // first chunk of source s
-    for (uint64_t k = c->last_waves + hc.next_chunk; k < c->last_items; ++k) {
-        uint64_t ch = k, off = 0, len = b.chunk;
-        if (k >= b.split_from) {
-            ch = b.split_from + (k - b.split_from) / b.parts;
-            off = (k - b.split_from) % b.parts * b.piece;
-            len = std::min<uint64_t>(b.chunk - off, b.piece);
-        }
-        for (uint64_t m; ch >= chunk0 + (m = (nph[s] + b.chunk - 1) / b.chunk); ++s) chunk0 += m;
-        const uint64_t first = (ch - chunk0) * b.chunk + off;
-        if (first < nph[s]) n += std::min(len, nph[s] - first);
+    const uint64_t k = c->last_waves + hc.next_chunk;
+    if (b.dealt || k >= c->last_items) return 0;
+    // the first item not taken: chunk ch from its photon off on
+    uint64_t ch = k, off = 0;
+    if (k >= b.split_from) {
+        ch = b.split_from + (k - b.split_from) / b.parts;
+        off = (k - b.split_from) % b.parts * b.piece;
+    }
+    uint64_t n = 0, chunk0 = 0;  // first chunk of the source
+    for (const uint64_t m : nph) {
+        const uint64_t chunks = (m + b.chunk - 1) / b.chunk;
+        const uint64_t first = ch < chunk0 ? 0 : (ch - chunk0) * b.chunk + off;
+        if (first < m) n += m - first;
+        chunk0 += chunks;
     }
     return n;
 }
@@ -1856,7 +1858,8 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
     // cascade: 7.07 ms, from memory 7.27).
     int block = ctx->cfg.block_size;
     if (block == 0) {
-        const OccKey key{batch_kernel_fn(skind, phase), table_bytes(skind)};
+        const OccKey key{batch_kernel_fn(skind, phase), table_bytes(skind),
+                         table_bytes(kSearchGridMem)};
         if (!(key == ctx->occ_key)) {
             int best_waves = 0;
             ctx->occ_block = 64;  // the LDS check below reports what does not fit

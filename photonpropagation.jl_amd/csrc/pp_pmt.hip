@@ -438,8 +438,10 @@ int launch(PmtArgs<In>& a, hipStream_t stream, int n_cu) {
     const int64_t blocks = std::min<int64_t>((a.n + 255) / 256, (int64_t)std::max(n_cu, 1) * 8);
     const dim3 grid((unsigned)std::max<int64_t>(blocks, 1));
     const size_t lds = 3 * sizeof(float) * (size_t)a.s.n_wl;
-    hipLaunchKernelGGL(fast_setup(a.s, &a.f) ? pom_pmt_kernel<In> : pom_pmt_full_kernel<In>, grid,
-                       dim3(256), lds, stream, a);
+    // the list's entries hold 32-bit indices
+    const bool fast = a.n <= (int64_t)UINT32_MAX && fast_setup(a.s, &a.f);
+    hipLaunchKernelGGL(fast ? pom_pmt_kernel<In> : pom_pmt_full_kernel<In>, grid, dim3(256), lds,
+                       stream, a);
     PP_HIP(hipGetLastError());
     return PP_OK;
 }

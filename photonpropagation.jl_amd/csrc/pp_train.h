@@ -33,7 +33,7 @@ struct TrainArgs {
     int n_in, n_out;
     bool sample;     // draw the batch's samples (gather_kernel's draw), or take row b as b
     uint32_t k0, k1, step;
-    const bf16* Wf[kTMaxHidden + 1];  // packed by pack_layer: W_l
+    const bf16* Wf[kTMaxHidden + 1];  // packed by pack_weights_kernel: W_l
     const bf16* Wb[kTMaxHidden + 1];  // W_l transposed
     const float* b[kTMaxHidden + 1];
     bf16* H[kTMaxHidden + 1];
