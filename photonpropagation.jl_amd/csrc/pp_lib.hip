@@ -232,6 +232,12 @@ struct HitRec {
     uint64_t pid;
 };
 
+// x of the wave's first lane, as a scalar
+__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
+    return ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(x >> 32)) << 32) |
+           __builtin_amdgcn_readfirstlane((uint32_t)x);
+}
+
 // Returns false if this lane's record did not fit (overflow).
 __device__ __forceinline__ bool store_hits(bool has_hit, const HitRec& h, uint32_t src_ix,
                                            const HitCols& out, Counters* ctr) {
@@ -268,20 +274,38 @@ using pp::lds_bytes;
 // memory (L2 and the vector cache), where their LDS copy would cost resident waves
 // kSearchGridGlobal: all its tables read from memory, for target lists whose
 // records and grid tables exceed the LDS
+// kSearchBruteQueued, kSearchMixedQueued: the every-target scans over queued
+// segments, those that come near the targets' box. The scans are bound by the
+// VALU: a test is 30-40 instructions for 64 lanes, of which few need it (photons
+// leave the targets' box after a step or two). 1e7 photons on 24 panels, discs
+// and spheres: 3.07 ms of kernel in the plain scan, 0.86 queued with the hits
+// held back (take_hits) and the planes filtered (PlaneFilter)
 enum {
     kSearchBrute = 0,
     kSearchGrid = 1,
     kSearchMixed = 2,
     kSearchGridGlobal = 3,
     kSearchGridMem = 4,
-    kSearchKinds = 5
+    kSearchBruteQueued = 5,
+    kSearchMixedQueued = 6,
+    kSearchKinds = 7
 };
 template <int SEARCH>
 constexpr bool kLdsCells = SEARCH == kSearchGrid || SEARCH == kSearchGridMem;
-// the grid searches walk in batches (transport_group); the every-target
-// scans test each step at once (transport_photon)
+// two records per target
 template <int SEARCH>
-constexpr bool kDeferredWalk = kLdsCells<SEARCH> || SEARCH == kSearchGridGlobal;
+constexpr bool kMixedList = SEARCH == kSearchMixed || SEARCH == kSearchMixedQueued;
+// the grid searches and the queued scans search in batches (transport_group);
+// the plain every-target scans test each step at once (transport_photon): they
+// serve small launches, more than 2^26 - 1 steps, lists that leave no LDS for the
+// queues, and callers who ask for them
+constexpr bool deferred_kind(int search) {
+    return search != kSearchBrute && search != kSearchMixed;
+}
+template <int SEARCH>
+constexpr bool kDeferredWalk = deferred_kind(SEARCH);
+template <int SEARCH>
+constexpr bool kQueuedScan = SEARCH == kSearchBruteQueued || SEARCH == kSearchMixedQueued;
 
 // LDS tables of one workgroup: targets, grid cells and items, spectrum knots
 struct Lds {
@@ -307,7 +331,7 @@ __device__ __forceinline__ Lds stage_lds(const KParams& p) {
     }
     // a mixed (sphere and planar) list has two records per target
     const int n_rec = SEARCH == kSearchGridMem ? 0
-                      : SEARCH == kSearchMixed ? 2 * p.n_targets : p.n_targets;
+                      : kMixedList<SEARCH> ? 2 * p.n_targets : p.n_targets;
     float4* const tgt = lds;
     float4* const cells = lds + n_rec;
     uint16_t* const items =
@@ -326,26 +350,50 @@ __device__ __forceinline__ Lds stage_lds(const KParams& p) {
     return l;
 }
 
-template <int SEARCH>
-using SearchT = typename std::conditional<
-    kDeferredWalk<SEARCH>, pp::GridSearch,
-    typename std::conditional<SEARCH == kSearchMixed, pp::MixedSearch, pp::BruteSearch>::type>::type;
+// An every-target scan whose segments near the targets' box are scanned in batches
+template <typename Scan>
+struct QueuedScan {
+    Scan scan;
+    pp::GridDesc box;  // its corners ox..oz, ex..ez alone
+    __device__ __forceinline__ uint64_t touch_mask(f3 a, f3 b) const { return pp::touch_mask(box, a, b); }
+    template <bool COUNT>
+    __device__ __forceinline__ int find(f3 pos, f3 dir, float step, float& dt, pp::Work& w) const {
+        return scan.template find<COUNT>(pos, dir, step, dt, w);
+    }
+};
 
 template <int SEARCH>
-__device__ __forceinline__ SearchT<SEARCH> make_search(const KParams& p, const Lds& l) {
-    if constexpr (kDeferredWalk<SEARCH>) {
-        return pp::GridSearch{l.tgt, l.cells, l.items, p.grid};
+__device__ __forceinline__ auto make_search(const KParams& p, const Lds& l) {
+    if constexpr (SEARCH == kSearchBrute) {
+        return pp::BruteSearch{l.tgt, p.n_targets};
     } else if constexpr (SEARCH == kSearchMixed) {
         return pp::MixedSearch{l.tgt, p.n_targets};
+    } else if constexpr (SEARCH == kSearchBruteQueued) {
+        return QueuedScan<pp::BruteSearch>{{l.tgt, p.n_targets}, p.grid};
+    } else if constexpr (SEARCH == kSearchMixedQueued) {
+        return QueuedScan<pp::MixedSearch>{{l.tgt, p.n_targets}, p.grid};
     } else {
-        return pp::BruteSearch{l.tgt, p.n_targets};
+        return pp::GridSearch{l.tgt, l.cells, l.items, p.grid};
     }
 }
+template <int SEARCH>
+using SearchT = decltype(make_search<SEARCH>(std::declval<const KParams&>(), std::declval<const Lds&>()));
 
-// The search with its grid read again (kernel_params), for a batch of walks;
-// the every-target scans hold nothing worth reading again.
-__device__ __forceinline__ pp::GridSearch reread(const pp::GridSearch& s) {
-    return pp::GridSearch{s.tgt, s.cells, s.items, kernel_params()->grid};
+// The search for a batch: a grid search with its grid, and what it reads from
+// memory, read again (kernel_params); the scans hold nothing worth reading again.
+template <int SEARCH>
+__device__ __forceinline__ SearchT<SEARCH> reread(const SearchT<SEARCH>& s) {
+    if constexpr (SEARCH == kSearchGrid) {
+        return pp::GridSearch{s.tgt, s.cells, s.items, kernel_params()->grid};
+    } else if constexpr (SEARCH == kSearchGridMem) {
+        ConstParams* const p = kernel_params();
+        return pp::GridSearch{p->targets, s.cells, s.items, p->grid};
+    } else if constexpr (SEARCH == kSearchGridGlobal) {
+        ConstParams* const p = kernel_params();
+        return pp::GridSearch{p->targets, p->cells, p->cell_items, p->grid};
+    } else {
+        return s;
+    }
 }
 
 // position, distance and time after moving d along dir
@@ -396,7 +444,7 @@ __device__ __forceinline__ bool transport_photon(const KParams& p, const pp_sour
 }
 
 // ---------------------------------------------------------------------------
-// Deferred walk of the grid searches. A wave transports its 64 photons step
+// Deferred walk of the grid searches and queued scans. A wave transports its 64 photons step
 // by step as in transport_photon, but a step whose segment comes near the
 // grid box (its end points' box meets it) does not walk the grid at once: the
 // segment becomes a job in the wave's LDS queue, the photon moves on as if
@@ -418,21 +466,34 @@ __device__ __forceinline__ bool transport_photon(const KParams& p, const pp_sour
 // or more are pending or the step's new jobs would not fit, so at most kQueue
 // are pending after any step.
 constexpr uint32_t kQueue = 96;
+constexpr uint32_t kHitSlots = 16;  // hits a wave of a queued scan holds back
 constexpr uint32_t kWaveQueueBytes = kQueue * 32 + 64 * 8;
+constexpr uint32_t kScanQueueBytes = kWaveQueueBytes + kHitSlots * 16;
+constexpr uint32_t wave_queue_bytes(int search) {
+    return search == kSearchBruteQueued || search == kSearchMixedQueued ? kScanQueueBytes
+                                                                        : kWaveQueueBytes;
+}
 constexpr int32_t kDeferredMaxSteps = (1 << 26) - 1;  // step index of a job: 26 bits
 
 struct WaveQueue {
-    float4* job;               // 2 per job: (position, step length), (direction, lane | step << 6)
-    unsigned long long* key;   // per lane: earliest (step << 16 | target) hit, ~0 if none
+    char* base;  // one address: the parts lie at constant offsets
+    // 2 per job: (position, step length), (direction, lane | step << 6)
+    __device__ __forceinline__ float4* job() const { return reinterpret_cast<float4*>(base); }
+    // per lane: earliest (step << 16 | target) hit, ~0 if none
+    __device__ __forceinline__ unsigned long long* key() const {
+        return reinterpret_cast<unsigned long long*>(base + kQueue * 32);
+    }
+    // queued scans: hits not yet stored, a record's last 16 bytes each
+    __device__ __forceinline__ uint4* out() const {
+        return reinterpret_cast<uint4*>(base + kQueue * 32 + 64 * 8);
+    }
 };
 
+template <int SEARCH>
 __device__ __forceinline__ WaveQueue wave_queue(const KParams& p) {
     extern __shared__ float4 lds[];
-    char* base = reinterpret_cast<char*>(lds) + p.queue_off + (threadIdx.x >> 6) * kWaveQueueBytes;
-    WaveQueue q;
-    q.job = reinterpret_cast<float4*>(base);
-    q.key = reinterpret_cast<unsigned long long*>(base + kQueue * 32);
-    return q;
+    return WaveQueue{reinterpret_cast<char*>(lds) + p.queue_off +
+                     (threadIdx.x >> 6) * wave_queue_bytes(SEARCH)};
 }
 
 // Orders the wave's LDS accesses: the LDS executes one wave's accesses in
@@ -442,14 +503,86 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// One photon per lane (active lanes), the whole wave together.
-template <bool COUNT, typename Search>
-__device__ __forceinline__ bool transport_group(const KParams& p, const pp_source& src,
-                                                uint32_t src_ix, uint64_t pid, bool active,
-                                                const float* spec, const Search& search,
-                                                const pp::Phase& phase, const WaveQueue& q,
-                                                pp::Work& work, unsigned long long& n_steps_done,
-                                                HitRec& h) {
+// `n` slots of the hit buffer for the wave, the first of them in `first`. Returns
+// those that lie beyond its end.
+__device__ __forceinline__ uint32_t reserve_hits(uint32_t n, uint64_t& first) {
+    ConstParams* const p = kernel_params();
+    unsigned long long got = 0;
+    if (__lane_id() == 0) got = atomicAdd(&p->counters->n_hits, (unsigned long long)n);
+    first = uniform64(got);
+    const uint64_t cap = (uint64_t)p->hits.capacity;
+    const uint32_t fit = first >= cap ? 0u : cap - first < n ? (uint32_t)(cap - first) : n;
+    if (fit < n && __lane_id() == 0) atomicOr(&p->counters->err, 1u);
+    return n - fit;
+}
+
+// Of a hit record only the last 16 bytes: replay_hits_kernel writes the rest.
+__device__ __forceinline__ void store_hit(uint64_t i, uint4 v) {
+    ConstParams* const p = kernel_params();
+    if (i < (uint64_t)p->hits.capacity) reinterpret_cast<uint4*>(p->hits.rec + i)[3] = v;
+}
+
+// The wave's `n` hits in q.out to the hit buffer. Returns those that did not fit.
+__device__ __forceinline__ uint32_t store_queued(const WaveQueue& q, uint32_t n) {
+    if (n == 0) return 0;
+    wave_sync();
+    const uint32_t lane = __lane_id();
+    uint64_t first;
+    const uint32_t lost = reserve_hits(n, first);
+    if (lane < n) store_hit(first + lane, q.out()[lane]);
+    wave_sync();
+    return lost;
+}
+
+// The hits of a group (key: per lane, ~0 if none): a grid search stores them, a
+// queued scan (HOLD) adds them to the wave's `count` in q.out, which are stored
+// kHitSlots at a time. One atomic on the hit count per group with a hit was what
+// bounded lists that most groups hit (the device serves them at one per 12 ns:
+// 1e7 photons on 24 panels, discs and spheres 1.90 ms, with the slots 0.93); in
+// the grid searches, with a hit in one group of ten, the slots' LDS and registers
+// cost more than they save (1e8-photon cascade 7.1 -> 8.0 ms).
+// Returns the hits that did not fit the buffer.
+template <bool HOLD>
+__device__ __forceinline__ uint32_t take_hits(const WaveQueue& q, bool hit, unsigned long long key,
+                                              uint64_t first_pid, uint32_t src_ix,
+                                              uint32_t& count) {
+    const uint64_t m = __ballot(hit);
+    if (m == 0) return 0;
+    const uint32_t lane = __lane_id();
+    const uint32_t n = (uint32_t)__popcll(m);
+    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    const uint64_t id = (first_pid + lane) | ((uint64_t)((uint32_t)(key & 0xFFFFu) + 1u) << kPidBits);
+    const uint4 v = make_uint4((uint32_t)id, (uint32_t)(id >> 32), (uint32_t)(key >> 16), src_ix);
+    uint32_t lost = 0;
+    if constexpr (!HOLD) {
+        uint64_t first;
+        lost = reserve_hits(n, first);
+        if (hit) store_hit(first + rank, v);
+        return lost;
+    }
+    for (uint32_t done = 0; done < n;) {
+        const uint32_t take = kHitSlots - count < n - done ? kHitSlots - count : n - done;
+        if (hit && rank - done < take) q.out()[count + rank - done] = v;
+        count += take;
+        done += take;
+        if (count == kHitSlots) {
+            lost += store_queued(q, count);
+            count = 0;
+        }
+    }
+    return lost;
+}
+
+// One photon per lane (active lanes), the whole wave together. Hits go to the
+// wave's queue; returns those that did not fit the hit buffer (wave-uniform).
+template <bool COUNT, int SEARCH>
+__device__ __forceinline__ uint32_t transport_group(const KParams& p, const pp_source& src,
+                                                    uint32_t src_ix, uint64_t pid, bool active,
+                                                    const float* spec, const SearchT<SEARCH>& search,
+                                                    const pp::Phase& phase, const WaveQueue& q,
+                                                    uint32_t& n_queued, pp::Work& work,
+                                                    unsigned long long& n_steps_done) {
     const uint32_t lane = __lane_id();
     pp::Stream s{p.k0, p.k1, (uint32_t)pid, (uint32_t)(pid >> 32), src_ix};
     const pp::StepStream ss(s);
@@ -471,18 +604,19 @@ __device__ __forceinline__ bool transport_group(const KParams& p, const pp_sourc
     // register pair across the photon loop was spilled and reloaded per photon)
     uint32_t ones;
     __asm__ volatile("v_mov_b32 %0, -1" : "=v"(ones));
-    *reinterpret_cast<uint2*>(q.key + lane) = make_uint2(ones, ones);
+    *reinterpret_cast<uint2*>(q.key() + lane) = make_uint2(ones, ones);
     // the stepping lanes as a wave mask (scalar). A photon whose hit is known
-    // keeps stepping: its later steps cannot change the earliest (step,
-    // target), and with ~1e-3 of the photons hit, stopping them would cost a
-    // read of every lane's key after each batch (an LDS round trip) for
-    // nothing
-    const uint64_t going_m = __ballot(active);
+    // keeps stepping in a grid search: its later steps cannot change the earliest
+    // (step, target), and with ~1e-3 of the photons hit, stopping them would cost
+    // a read of every lane's key after each batch (an LDS round trip) for
+    // nothing. The queued scans, whose targets may fill the sky, read the keys
+    // after a batch that hit.
+    uint64_t going_m = __ballot(active);
     uint32_t head = 0, count = 0;  // wave-uniform ring of pending jobs
     // every lane walks one pending job (lanes >= n none)
     auto walk_jobs = [&](uint32_t n) {
         wave_sync();
-        const auto grid = reread(search);
+        const auto grid = reread<SEARCH>(search);
         int found = -1;
         float dt = 0.0f;
         unsigned long long key = 0;
@@ -490,7 +624,7 @@ __device__ __forceinline__ bool transport_group(const KParams& p, const pp_sourc
         if (lane < n) {
             uint32_t slot = head + lane;
             if (slot >= kQueue) slot -= kQueue;
-            const float4 a = q.job[2 * slot], b = q.job[2 * slot + 1];
+            const float4 a = q.job()[2 * slot], b = q.job()[2 * slot + 1];
             const uint32_t meta = __float_as_uint(b.w);
             owner = meta & 63u;
             if (COUNT) work.walks += 1;
@@ -498,7 +632,13 @@ __device__ __forceinline__ bool transport_group(const KParams& p, const pp_sourc
                                                 a.w, dt, work);
             if (found >= 0) {
                 key = ((unsigned long long)(meta >> 6) << 16) | (uint32_t)found;
-                atomicMin(q.key + owner, key);
+                atomicMin(q.key() + owner, key);
+            }
+        }
+        if constexpr (kQueuedScan<SEARCH>) {
+            if (__ballot(found >= 0)) {
+                wave_sync();
+                going_m &= ~__ballot(q.key()[lane] != ~0ull);
             }
         }
         head += n;
@@ -537,8 +677,8 @@ __device__ __forceinline__ bool transport_group(const KParams& p, const pp_sourc
                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
             uint32_t slot = head + count + rank;
             if (slot >= kQueue) slot -= kQueue;
-            q.job[2 * slot] = make_float4(pos.x, pos.y, pos.z, step_size);
-            q.job[2 * slot + 1] =
+            q.job()[2 * slot] = make_float4(pos.x, pos.y, pos.z, step_size);
+            q.job()[2 * slot + 1] =
                 make_float4(dir.x, dir.y, dir.z, __uint_as_float(lane | ((uint32_t)step << 6)));
         }
         count += n_new;
@@ -550,40 +690,18 @@ __device__ __forceinline__ bool transport_group(const KParams& p, const pp_sourc
         }
     }
     wave_sync();
-    const unsigned long long key = q.key[lane];
+    const unsigned long long key = q.key()[lane];
     const bool hit = active && key != ~0ull;
     if (COUNT && active) n_steps_done += hit ? (unsigned long long)(key >> 16) : (unsigned long long)p.n_steps;
-    if (hit) {
-        // the record holds the photon id, module and step; replay_hits_kernel
-        // completes it (emission again, steps 1..k-1, the sphere test of step
-        // k for the distance within it), so that neither
-        // the emission's state nor a second inlined emission stays in this
-        // kernel's registers. The photon id is recomputed from the wave's first
-        // id (scalar) and the lane.
-        uint64_t first = wave_first;
-        __asm__ volatile("" : "+s"(first));
-        const uint64_t id = first + lane;
-        const f3 zero = pp::make3(0.0f, 0.0f, 0.0f);
-        h = HitRec{zero, zero, zero, 0.0f, 0.0f, 0.0f, (int32_t)(key & 0xFFFFu) + 1,
-                   (int32_t)(key >> 16), id};
-    }
-    return hit;
-}
-
-// lost: the wave's photons that were not completed, 0 unless the hit buffer
-// overflowed (the completed ones are the launch's photons less these: counting
-// them took an atomic per lane or wave at the end of every launch, 18 us of the
-// README example's 36)
-template <bool COUNT>
-__device__ __forceinline__ void flush_counts(const KParams& p, unsigned long long lost,
-                                             unsigned long long n_steps_done, const pp::Work& work) {
-    if (lost && __lane_id() == 0) atomicAdd(&p.counters->n_lost, lost);
-    if (COUNT) {
-        atomicAdd(&p.counters->steps, n_steps_done);
-        atomicAdd(&p.counters->tests, (unsigned long long)work.tests);
-        atomicAdd(&p.counters->cells, (unsigned long long)work.cells);
-        atomicAdd(&p.counters->walks, (unsigned long long)work.walks);
-    }
+    // the record holds the photon id, module and step; replay_hits_kernel
+    // completes it (emission again, steps 1..k-1, the target's test of step
+    // k for the distance within it), so that neither
+    // the emission's state nor a second inlined emission stays in this
+    // kernel's registers. The photon id is recomputed from the wave's first
+    // id (scalar) and the lane.
+    uint64_t first = wave_first;
+    __asm__ volatile("" : "+s"(first));
+    return take_hits<kQueuedScan<SEARCH>>(q, hit, key, first, src_ix, n_queued);
 }
 
 // Propagation of one source: cuda_propagate_photons! (src/photon_prop_cuda.jl:
@@ -599,12 +717,6 @@ template <int SEARCH>
 constexpr int kWavesPerSimd = kDeferredWalk<SEARCH> ? 7 : 6;
 #define PP_PROPAGATE_ATTRS \
     __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<SEARCH>)))
-
-// x of the wave's first lane, as a scalar
-__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
-    return ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(x >> 32)) << 32) |
-           __builtin_amdgcn_readfirstlane((uint32_t)x);
-}
 
 // *p read through the constant address space: a scalar load into SGPRs for
 // a wave-uniform address (the tables the kernels read are not written
@@ -634,28 +746,64 @@ __device__ __forceinline__ pp_source source_record(const pp_source* sp, uint32_t
 #endif
 }
 
-// One photon per lane (active lanes), the whole wave together, hits stored.
-// False where this lane's hit did not fit the buffer.
+// What a wave carries from group to group.
+struct WaveState {
+    WaveQueue q{};
+    uint32_t n_queued = 0;    // hits in q.out
+    bool overflow = false;    // the hit buffer was full: per lane in the plain scans, else uniform
+    unsigned long long n_steps_done = 0;
+    pp::Work work;
+};
+
+// n photons (wave-uniform) that were not completed, only after the hit buffer
+// overflowed: the completed ones are the launch's photons less these (counting
+// them took an atomic per lane or wave at the end of every launch, 18 us of the
+// README example's 36).
+__device__ __forceinline__ void add_lost(uint64_t n) {
+    if (n && __lane_id() == 0)
+        atomicAdd(&kernel_params()->counters->n_lost, (unsigned long long)n);
+}
+
+// 64 photons from base on (up to end), one per lane, the whole wave together,
+// hits stored or queued. A lane or wave that met a full hit buffer takes no more
+// photons and counts those it is given as lost.
 template <bool COUNT, int SEARCH>
-__device__ __forceinline__ bool propagate_group(const KParams& p, const pp_source& src,
-                                                uint32_t src_ix, uint64_t pid, bool active,
+__device__ __forceinline__ void propagate_group(const KParams& p, const pp_source& src,
+                                                uint32_t src_ix, uint64_t base, uint64_t end,
                                                 const float* spec, const SearchT<SEARCH>& search,
-                                                const pp::Phase& phase, const WaveQueue& q,
-                                                pp::Work& work, unsigned long long& n_steps_done) {
-    bool stored = true;
+                                                const pp::Phase& phase, WaveState& w) {
+    const uint64_t pid = base + __lane_id();
     if constexpr (kDeferredWalk<SEARCH>) {
-        HitRec h;
-        const bool hit = transport_group<COUNT>(p, src, src_ix, pid, active, spec, search, phase, q,
-                                                work, n_steps_done, h);
-        stored = store_hits(hit, h, src_ix, p.hits, p.counters);
-    } else if (active) {
-        HitRec h;
-        const bool hit = transport_photon<COUNT>(p, src, src_ix, pid, spec, search, phase, work,
-                                                 n_steps_done, h);
-        stored = store_hits(hit, h, src_ix, p.hits, p.counters);
+        if (w.overflow) {
+            add_lost(end - base < 64 ? end - base : 64);
+            return;
+        }
+        const uint32_t lost = transport_group<COUNT, SEARCH>(p, src, src_ix, pid, pid < end, spec, search,
+                                                     phase, w.q, w.n_queued, w.work, w.n_steps_done);
+        add_lost(lost);
+        w.overflow = lost != 0;
+    } else {
+        if (pid < end && !w.overflow) {
+            HitRec h;
+            const bool hit = transport_photon<COUNT>(p, src, src_ix, pid, spec, search, phase,
+                                                     w.work, w.n_steps_done, h);
+            w.overflow = !store_hits(hit, h, src_ix, p.hits, p.counters);
+            if (w.overflow) atomicOr(&p.counters->err, 1u);
+        }
+        add_lost((uint64_t)__popcll(__ballot(w.overflow && pid < end)));
     }
-    if (!stored) atomicOr(&p.counters->err, 1u);
-    return stored;
+}
+
+// The wave's queued hits stored, and its counts added.
+template <bool COUNT, int SEARCH>
+__device__ __forceinline__ void finish_wave(const KParams& p, WaveState& w) {
+    if constexpr (kDeferredWalk<SEARCH>) add_lost(store_queued(w.q, w.n_queued));
+    if (COUNT) {
+        atomicAdd(&p.counters->steps, w.n_steps_done);
+        atomicAdd(&p.counters->tests, (unsigned long long)w.work.tests);
+        atomicAdd(&p.counters->cells, (unsigned long long)w.work.cells);
+        atomicAdd(&p.counters->walks, (unsigned long long)w.work.walks);
+    }
 }
 
 template <int PHASE, int SEARCH, bool COUNT = false>
@@ -665,31 +813,16 @@ __global__ void PP_PROPAGATE_ATTRS propagate_kernel(KParams p) {
     phase.kind = PHASE;
     const auto search = make_search<SEARCH>(p, l);
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    unsigned long long lost = 0, n_steps_done = 0;
-    pp::Work work;
-    WaveQueue q{};
-    if constexpr (kDeferredWalk<SEARCH>) q = wave_queue(p);
+    WaveState w;
+    if constexpr (kDeferredWalk<SEARCH>) w.q = wave_queue<SEARCH>(p);
     // whole waves of photons, the loop condition uniform across the wave
-    bool overflow = false;
     for (uint64_t base = (uint64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
          base < p.n_photons; base += stride) {
         uint32_t si = p.src_ix;
         const pp_source src = source_record(p.sources + p.src_ix, si);
-        const uint64_t pid = base + __lane_id();
-        overflow |= !propagate_group<COUNT, SEARCH>(p, src, si, pid, pid < p.n_photons && !overflow,
-                                                    l.spec, search, phase, q, work, n_steps_done);
-        const uint64_t bad = __ballot(overflow);
-        if (bad) {
-            lost += (unsigned long long)__popcll(__ballot(overflow && pid < p.n_photons));
-            if constexpr (kDeferredWalk<SEARCH>) {
-                // the wave ends here: its later groups too
-                for (uint64_t k = base + stride; k < p.n_photons; k += stride)
-                    lost += p.n_photons - k < 64 ? p.n_photons - k : 64;
-                break;
-            }
-        }
+        propagate_group<COUNT, SEARCH>(p, src, si, base, p.n_photons, l.spec, search, phase, w);
     }
-    flush_counts<COUNT>(p, lost, n_steps_done, work);
+    finish_wave<COUNT, SEARCH>(p, w);
 }
 
 // Batch of sources in one persistent launch. Work items are chunks of
@@ -709,9 +842,23 @@ struct BatchParams {
     int32_t n_sources;
     uint32_t chunk;                // multiple of 64
     uint32_t parts, piece;         // pieces per split chunk; photons per piece, a multiple of 64
-    uint64_t split_from;           // first split chunk (chunk_prefix[n_sources]: none)
+    uint64_t split_from;           // first split chunk (the number of chunks: none)
+    uint64_t n_items;              // chunks and pieces
     bool dealt;                    // every item by wave index, none from the counter
 };
+
+// A batch kernel's arguments, for the second of them read again like the first
+struct BatchKernelArgs {
+    KParams p;
+    BatchParams b;
+};
+__device__ __forceinline__ BatchParams batch_params() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return reinterpret_cast<const __attribute__((address_space(4))) BatchKernelArgs*>(kernel_params())->b;
+#else
+    return BatchParams{};
+#endif
+}
 
 struct BatchItem {
     int source;
@@ -719,7 +866,8 @@ struct BatchItem {
 };
 
 // Work item k of the batch (k wave-uniform).
-__device__ __forceinline__ BatchItem batch_item(const BatchParams& b, uint64_t k) {
+__device__ __forceinline__ BatchItem batch_item(uint64_t k) {
+    const BatchParams b = batch_params();
     // chunk c, photons [off, off + len) of it
     uint64_t c = k;
     uint32_t off = 0, len = b.chunk;
@@ -747,53 +895,45 @@ __device__ __forceinline__ BatchItem batch_item(const BatchParams& b, uint64_t k
 }
 
 template <int PHASE, int SEARCH, bool COUNT = false>
-__global__ void PP_PROPAGATE_ATTRS propagate_batch_kernel(KParams p, BatchParams b) {
+__global__ void PP_PROPAGATE_ATTRS propagate_batch_kernel(KParams p, BatchParams) {
     const Lds l = stage_lds<SEARCH>(p);
     pp::Phase phase = p.med.phase;
     phase.kind = PHASE;
     const auto search = make_search<SEARCH>(p, l);
-    const uint64_t n_chunks = load_constant(b.chunk_prefix + b.n_sources);
-    const uint64_t total = b.split_from + (n_chunks - b.split_from) * b.parts;
-    const uint32_t lane = __lane_id();
-    WaveQueue q{};
-    if constexpr (kDeferredWalk<SEARCH>) q = wave_queue(p);
-    unsigned long long lost = 0, n_steps_done = 0;
-    pp::Work work;
-    bool overflow = false;
+    WaveState w;
+    if constexpr (kDeferredWalk<SEARCH>) w.q = wave_queue<SEARCH>(p);
     const uint32_t waves = gridDim.x * (blockDim.x >> 6);
     // the first item by the wave's index
     uint64_t next = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     for (;;) {
         const uint64_t ck = uniform64(next);
-        if (ck >= total) break;
-        const BatchItem it = batch_item(b, ck);
+        if (ck >= batch_params().n_items) break;
+        const BatchItem it = batch_item(ck);
         for (uint64_t base = it.first; base < it.end; base += 64) {
             // the source index and record, opaque to the optimiser in every
             // iteration: what the emission derives from them is computed here
             // (one scalar reload per 64 photons) instead of being hoisted out
             // of the loop into registers that then spill to scratch
             uint32_t si = (uint32_t)it.source;
-            const pp_source src = source_record(b.sources + it.source, si);
-            const uint64_t pid = base + lane;
-            overflow |= !propagate_group<COUNT, SEARCH>(p, src, si, pid, pid < it.end && !overflow,
-                                                        l.spec, search, phase, q, work,
-                                                        n_steps_done);
-            lost += (unsigned long long)__popcll(__ballot(overflow && pid < it.end));
+            const pp_source src = source_record(batch_params().sources + it.source, si);
+            propagate_group<COUNT, SEARCH>(p, src, si, base, it.end, l.spec, search, phase, w);
         }
-        if (__ballot(overflow)) {
+        if (__ballot(w.overflow)) {
             // the call fails; take no more chunks, and give those dealt to this wave up
+            const BatchParams b = batch_params();
             if (b.dealt)
-                for (uint64_t k = ck + waves; k < total; k += waves) {
-                    const BatchItem rest = batch_item(b, k);
-                    lost += rest.end - rest.first;
+                for (uint64_t k = ck + waves; k < b.n_items; k += waves) {
+                    const BatchItem rest = batch_item(k);
+                    add_lost(rest.end - rest.first);
                 }
             break;
         }
         next = ck;
-        if (!b.dealt && lane == 0) next = atomicAdd(&p.counters->next_chunk, 1ull);
+        if (!batch_params().dealt && __lane_id() == 0)
+            next = atomicAdd(&kernel_params()->counters->next_chunk, 1ull);
         next += waves;
     }
-    flush_counts<COUNT>(p, lost, n_steps_done, work);
+    finish_wave<COUNT, SEARCH>(p, w);
 }
 
 // The counters to pinned host memory, where the host reads them once the stream
@@ -815,7 +955,7 @@ __global__ void publish_counters_kernel(const Counters* c, Counters* host) { pub
 // position, directions, wavelength, time and distance.
 // sources: the call's source list on the device.
 __global__ void __launch_bounds__(256) replay_hits_kernel(KParams p, const pp_source* sources,
-                                                          Counters* host) {
+                                                          Counters* host, bool mixed) {
     if (blockIdx.x == 0) publish(p.counters, host);
     const pp::Phase phase = p.med.phase;
     const unsigned long long n_hits = p.counters->n_hits;
@@ -843,11 +983,17 @@ __global__ void __launch_bounds__(256) replay_hits_kernel(KParams p, const pp_so
             const float ct = pp::phase_cos_words(phase, w.y, w.z);
             rd = pp::update_direction(rd, ct, pp::u01(w.w));
         }
-        // step k, cut at the target: the distance as GridSearch's walk finds it
+        // step k, cut at the target: the distance as the search finds it
         const uint4 w = ss.block((uint32_t)k);
         const float step_size = pp::step_length(pp::u01_open0(w.x), ln2_sca);
         float d = 0.0f;
-        pp::sphere_hit(p.targets[target], rp, rd, pp::dir_excess(rd), step_size, d);
+        const float4 t = p.targets[mixed ? 2 * target : target];
+        const float4 e = mixed ? p.targets[2 * target + 1] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        const uint32_t kind = mixed ? __float_as_uint(e.x) : (uint32_t)PP_SHAPE_SPHERE;
+        if (kind == PP_SHAPE_SPHERE)
+            pp::sphere_hit(t, rp, rd, pp::dir_excess(rd), step_size, d);
+        else
+            pp::plane_hit(kind, t, e, rp, rd, step_size, d);
         move_by(rp, rdist, rt, rd, d, inv_c);
         r[0] = make_float4(rp.x, rp.y, rp.z, rd.x);
         r[1] = make_float4(rd.y, rd.z, st.dir.x, st.dir.y);
@@ -1199,6 +1345,83 @@ int build_grid(pp_ctx* c, float cell_req, float cell_z_req) {
     return PP_OK;
 }
 
+// A bound of the scattering length over the spectrum's wavelengths, or infinity.
+double longest_scattering(const pp_ctx* c) {
+    const pp::Medium& m = c->medium;
+    if (m.kind == PP_MEDIUM_SIMPLE) return m.sca_len;
+    const auto ends = std::minmax_element(c->h_spec.begin(), c->h_spec.end());
+    const double wl[2] = {c->spec_n > 0 ? *ends.first : c->spec_mono,
+                          c->spec_n > 0 ? *ends.second : c->spec_mono};
+    double longest = 0.0;
+    for (double l : wl) {  // monotonic in between
+        if (m.kind == PP_MEDIUM_ICE) {
+            longest = std::max(longest, m.ice_pref * std::pow(l / 400.0, (double)m.ice_alpha));
+        } else {
+            if (!(m.kop1 >= 0.0 && m.kop2 >= 0.0 && m.kop3 >= 0.0)) return INFINITY;
+            const double x = l / 550.0;
+            longest = std::max(longest, m.sca_scale / (m.kop1 * std::pow(x, -4.3) +
+                                                       m.kop2 * std::pow(x, -1.7) +
+                                                       m.kop3 * std::pow(x, -0.3)));
+        }
+    }
+    return longest;
+}
+
+// The box that a segment meets if it hits a target, for the queued scans; false
+// where there is no useful one. A direction that has drifted to |dir|^2 = 1 + e
+// hits a sphere at a point within sqrt(r^2 + e d^2) of its centre (the reference's
+// discriminant keeps the drift), d being at most the longest step: 24 ln 2
+// scattering lengths for the smallest uniform number. e grows by some 2e-7 a step
+// from a unit direction, and is taken as five times that. The margin is far above
+// the rounding of the hit tests and of the segment's end.
+bool scan_box(const pp_ctx* c, const pp_source* sources, int n_sources, int32_t n_steps,
+              pp::GridDesc* g) {
+    const double step = 16.64 * 1.01 * longest_scattering(c), e = 1e-6 * ((double)n_steps + 4.0);
+    if (!(step < 1e6) || !(e < 1e-3)) return false;
+    double size = 0.0, far = 0.0;
+    for (int i = 0; i < n_sources; ++i) {
+        const pp_source& x = sources[i];
+        double d2 = 0.0;
+        for (int a = 0; a < 3; ++a) {
+            far = std::max(far, (double)std::fabs(x.position[a]));
+            d2 += (double)x.direction[a] * x.direction[a];
+        }
+        if (x.kind != PP_SRC_POINTLIKE_ISOTROPIC && x.kind != PP_SRC_POINTLIKE_TIME_RANGE &&
+            !(std::fabs(d2 - 1.0) <= 2e-6))
+            return false;
+    }
+    double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (const pp_target& t : c->h_pods) {
+        double r[3] = {0.5 * t.length[0], 0.5 * t.length[1], 0.0};
+        if (t.shape_kind != PP_SHAPE_RECTANGLE) r[0] = r[1] = t.radius;
+        if (t.shape_kind == PP_SHAPE_SPHERE)
+            r[0] = r[1] = r[2] = std::sqrt((double)t.radius * t.radius + e * step * step);
+        for (int a = 0; a < 3; ++a) {
+            lo[a] = std::min(lo[a], t.position[a] - r[a]);
+            hi[a] = std::max(hi[a], t.position[a] + r[a]);
+            size = std::max(size, std::max(std::fabs(lo[a]), std::fabs(hi[a])));
+        }
+    }
+    const double m = 0.02 + 1e-4 * size + 1e-5 * far + 1e-6 * step * n_steps;
+    g->ox = (float)(lo[0] - m);
+    g->oy = (float)(lo[1] - m);
+    g->oz = (float)(lo[2] - m);
+    g->ex = (float)(hi[0] + m);
+    g->ey = (float)(hi[1] + m);
+    g->ez = (float)(hi[2] + m);
+    return true;
+}
+
+// Whether an automatic every-target scan queues its segments. The queues save tests
+// and the hit's emission state; the replay of the hits adds 3-6 us to a launch.
+// Plain and queued kernel time meet at about 1.5e6 photons x targets: one sphere
+// 0.080 / 0.081 ms at 1e6 photons, 0.529 / 0.501 at 1e7; three spheres 0.096 /
+// 0.087 at 1e6; eight 0.031 / 0.030 at 1e5; 24 panels, discs and spheres 0.090 /
+// 0.049 at 1e5, 2.62 / 0.86 at 1e7.
+bool queue_scan(const pp_ctx* c, uint64_t photons) {
+    return c->n_targets > 0 && photons > (3u << 19) / (uint64_t)c->n_targets;
+}
+
 // Defaults and range checks of a pp_config.
 int normalise_config(pp_config& c, const char* who) {
     const std::string w(who);
@@ -1297,7 +1520,7 @@ const void* batch_kernel_fn(int skind, int phase) {
 #define PP_K3(S) {PP_K(PP_PHASE_HG, S), PP_K(PP_PHASE_MIXED_HG_ES, S), PP_K(PP_PHASE_MIXED_HG_SL, S)}
     static const BatchFn kKernels[kSearchKinds][3] = {
         PP_K3(kSearchBrute), PP_K3(kSearchGrid), PP_K3(kSearchMixed), PP_K3(kSearchGridGlobal),
-        PP_K3(kSearchGridMem)};
+        PP_K3(kSearchGridMem), PP_K3(kSearchBruteQueued), PP_K3(kSearchMixedQueued)};
 #undef PP_K3
 #undef PP_K
     return (const void*)kKernels[skind][phase];
@@ -1312,9 +1535,11 @@ int launch_per_source(pp_ctx* c, KParams& kp, const pp_source* sources,
     // [count][search kind][phase kind]
     static const KernelFn kKernels[2][kSearchKinds][3] = {
         {PP_K3(kSearchBrute, false), PP_K3(kSearchGrid, false), PP_K3(kSearchMixed, false),
-         PP_K3(kSearchGridGlobal, false), PP_K3(kSearchGridMem, false)},
+         PP_K3(kSearchGridGlobal, false), PP_K3(kSearchGridMem, false),
+         PP_K3(kSearchBruteQueued, false), PP_K3(kSearchMixedQueued, false)},
         {PP_K3(kSearchBrute, true), PP_K3(kSearchGrid, true), PP_K3(kSearchMixed, true),
-         PP_K3(kSearchGridGlobal, true), PP_K3(kSearchGridMem, true)}};
+         PP_K3(kSearchGridGlobal, true), PP_K3(kSearchGridMem, true),
+         PP_K3(kSearchBruteQueued, true), PP_K3(kSearchMixedQueued, true)}};
 #undef PP_K3
 #undef PP_K
     const KernelFn kern = kKernels[count][skind][phase];
@@ -1352,9 +1577,11 @@ int launch_batch(pp_ctx* c, KParams& kp, const pp_source* sources,
 #define PP_K3(S, C) {PP_K(PP_PHASE_HG, S, C), PP_K(PP_PHASE_MIXED_HG_ES, S, C), PP_K(PP_PHASE_MIXED_HG_SL, S, C)}
     static const BatchFn kKernels[2][kSearchKinds][3] = {
         {PP_K3(kSearchBrute, false), PP_K3(kSearchGrid, false), PP_K3(kSearchMixed, false),
-         PP_K3(kSearchGridGlobal, false), PP_K3(kSearchGridMem, false)},
+         PP_K3(kSearchGridGlobal, false), PP_K3(kSearchGridMem, false),
+         PP_K3(kSearchBruteQueued, false), PP_K3(kSearchMixedQueued, false)},
         {PP_K3(kSearchBrute, true), PP_K3(kSearchGrid, true), PP_K3(kSearchMixed, true),
-         PP_K3(kSearchGridGlobal, true), PP_K3(kSearchGridMem, true)}};
+         PP_K3(kSearchGridGlobal, true), PP_K3(kSearchGridMem, true),
+         PP_K3(kSearchBruteQueued, true), PP_K3(kSearchMixedQueued, true)}};
 #undef PP_K3
 #undef PP_K
     const BatchFn kern = kKernels[count][skind][phase];
@@ -1433,6 +1660,7 @@ int launch_batch(pp_ctx* c, KParams& kp, const pp_source* sources,
     const uint64_t n_items = bp.split_from + (n_chunks - bp.split_from) * bp.parts;
     const int64_t want = (int64_t)((n_items + block / 64 - 1) / (block / 64));
     const unsigned blocks = (unsigned)std::min<int64_t>(want, max_blocks);
+    bp.n_items = n_items;
     bp.dealt = dealt;
     c->last_batch = bp;
     c->last_waves = (uint64_t)blocks * (block / 64);
@@ -1732,7 +1960,7 @@ int pp_set_targets(pp_ctx* ctx, const pp_target* t, int n) {
             std::memcpy(&kf, &kind, 4);
             h[(size_t)i * per + 1] = x.shape_kind == PP_SHAPE_RECTANGLE
                                          ? make_float4(kf, x.length[0] / 2.0f, x.length[1] / 2.0f, 0.0f)
-                                         : make_float4(kf, 0.0f, 0.0f, 0.0f);
+                                         : make_float4(kf, x.radius, x.radius, 0.0f);
         }
     }
     // (x, y, z, radius) per target for the PMT detection of hits
@@ -1828,6 +2056,18 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
             }
         }
     }
+    // photon count of src/photon_prop_cuda.jl:456 (Float32 product)
+    std::vector<uint64_t> nph((size_t)n_sources);
+    uint64_t n_sim = 0;
+    for (int i = 0; i < n_sources; ++i) {
+        // the limit is checked on the float product, before it is converted
+        const float prod = std::floor((float)sources[i].photons * photon_scaling);
+        if (!(prod < (float)kMaxPhotonsPerSource))
+            return fail(PP_ERR_INVALID, "pp_propagate: source " + std::to_string(i) +
+                                            " has 2^40 or more photons after scaling");
+        nph[(size_t)i] = prod > 0.0f ? (uint64_t)prod : 0;
+        n_sim += nph[(size_t)i];
+    }
     const bool grid = search == PP_SEARCH_GRID;
     const bool global = grid && ctx->grid_global;
     int skind = global ? kSearchGridGlobal
@@ -1840,11 +2080,20 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
         return lds_bytes(n, grid ? ctx->grid.n_cells : 0, grid ? ctx->grid.n_items : 0, ctx->spec_n,
                          grid);
     };
-    // the grid kernels' per-wave walk queues follow the tables
-    auto with_queues = [&](size_t tables, int threads) {
-        return grid ? ((tables + 15) & ~(size_t)15) + (size_t)(threads / 64) * kWaveQueueBytes
-                    : tables;
+    // the walk queues of the waves that search in batches follow the tables
+    auto with_queues = [&](int kind, int threads) {
+        const size_t tables = table_bytes(kind);
+        return deferred_kind(kind)
+                   ? ((tables + 15) & ~(size_t)15) + (size_t)(threads / 64) * wave_queue_bytes(kind)
+                   : tables;
     };
+    pp::GridDesc box{};
+    if (automatic && !grid && n_steps <= kDeferredMaxSteps && queue_scan(ctx, n_sim) &&
+        scan_box(ctx, sources, n_sources, n_steps, &box)) {
+        const int kind = ctx->planar ? kSearchMixedQueued : kSearchBruteQueued;
+        if (with_queues(kind, ctx->cfg.block_size ? ctx->cfg.block_size : 256) <= (size_t)kMaxLdsBytes)
+            skind = kind;
+    }
     // block size: the set one or, for 0, the one of 256, 384, 512, 768 and 1024
     // threads with the most waves resident per CU: the runtime's occupancy
     // query (registers: 6 or 7 waves per SIMD) and the LDS a workgroup needs (the
@@ -1868,7 +2117,7 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
                 if (kind != skind && skind != kSearchGrid) continue;
                 const void* fn = batch_kernel_fn(kind, phase);
                 for (int b : {256, 384, 512, 768, 1024}) {
-                    const size_t need = with_queues(table_bytes(kind), b);
+                    const size_t need = with_queues(kind, b);
                     if (need > (size_t)kMaxLdsBytes) continue;
                     int occ = 0;
                     PP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, b, need));
@@ -1888,7 +2137,7 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
     }
     const size_t tables = table_bytes(skind);
     const uint32_t queue_off = (uint32_t)((tables + 15) & ~(size_t)15);
-    const size_t lds = with_queues(tables, block);
+    const size_t lds = with_queues(skind, block);
     ctx->block = block;
     if (lds > (size_t)kMaxLdsBytes)
         return fail(PP_ERR_INVALID, "pp_propagate: targets, tables and walk queues exceed the LDS "
@@ -1907,6 +2156,8 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
         kp.grid = ctx->grid;
         kp.cells = ctx->d_cells;
         kp.cell_items = ctx->d_cell_items;
+    } else if (deferred_kind(skind)) {
+        kp.grid = box;
     }
     kp.spec_n = ctx->spec_n;
     kp.spec_map = ctx->spec_map;
@@ -1915,16 +2166,6 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
     kp.spec_lastf = (float)(ctx->spec_n - 1);
     kp.spec = ctx->d_spec;
     kp.hits = ctx->hits;
-    // photon count of src/photon_prop_cuda.jl:456 (Float32 product)
-    std::vector<uint64_t> nph((size_t)n_sources);
-    for (int i = 0; i < n_sources; ++i) {
-        // the limit is checked on the float product, before it is converted
-        const float prod = std::floor((float)sources[i].photons * photon_scaling);
-        if (!(prod < (float)kMaxPhotonsPerSource))
-            return fail(PP_ERR_INVALID, "pp_propagate: source " + std::to_string(i) +
-                                            " has 2^40 or more photons after scaling");
-        nph[(size_t)i] = prod > 0.0f ? (uint64_t)prod : 0;
-    }
     ctx->n_launch = 0;
     ctx->last_items = 0;
     const int mode = ctx->cfg.batch_mode == PP_BATCH_AUTO ? PP_BATCH_PERSISTENT : ctx->cfg.batch_mode;
@@ -1934,11 +2175,11 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
         if (int rc = launch_batch(ctx, kp, sources, nph, skind, phase, count, lds, mode == PP_BATCH_GRAPH))
             return rc;
     }
-    // the grid kernels leave their hit records to be completed
-    if (grid) {
+    // the kernels that search in batches leave their hit records to be completed
+    if (deferred_kind(skind)) {
         hipLaunchKernelGGL(replay_hits_kernel, dim3((unsigned)(4 * ctx->n_cu)), dim3(256), 0,
                            ctx->stream, kp, (const pp_source*)(ctx->d_batch + kTableSources),
-                           ctx->h_counters);
+                           ctx->h_counters, ctx->planar);
     } else {
         hipLaunchKernelGGL(publish_counters_kernel, dim3(1), dim3(64), 0, ctx->stream, kp.counters,
                            ctx->h_counters);
@@ -1950,8 +2191,6 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
     const Counters hc = *ctx->h_counters;
     PP_HIP(hipEventElapsedTime(&ctx->last_ms, ctx->ev0, ctx->ev1));
     ctx->n_hits = (int64_t)std::min<unsigned long long>(hc.n_hits, ctx->hits.capacity);
-    uint64_t n_sim = 0;
-    for (uint64_t v : nph) n_sim += v;
     ctx->n_ph_sim = (int64_t)(n_sim - hc.n_lost - (hc.err ? photons_not_taken(ctx, hc, nph) : 0));
     ctx->work_steps = (int64_t)hc.steps;
     ctx->work_tests = (int64_t)hc.tests;

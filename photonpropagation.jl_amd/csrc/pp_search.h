@@ -33,6 +33,23 @@ struct GridDesc {
     float ex, ey, ez;  // upper corner, ox + nx h etc. (rounded once, on the host)
 };
 
+// Lanes whose segment a-b comes near the box of g, as a wave mask: whether the
+// bounding box of the segment meets it. Each compare is a ballot of its
+// own (one v_cmp writing a scalar mask) and the masks are combined by
+// scalar instructions; as one lane condition the compiler merged the
+// pairs of compares into minima and maxima, which need a canonicalising
+// instruction per operand, and copied the result out of and back into a
+// mask
+__device__ __forceinline__ uint64_t touch_mask(const GridDesc& g, f3 a, f3 b) {
+    const uint64_t x = (__ballot(a.x >= g.ox) | __ballot(b.x >= g.ox)) &
+                       (__ballot(a.x <= g.ex) | __ballot(b.x <= g.ex));
+    const uint64_t y = (__ballot(a.y >= g.oy) | __ballot(b.y >= g.oy)) &
+                       (__ballot(a.y <= g.ey) | __ballot(b.y <= g.ey));
+    const uint64_t z = (__ballot(a.z >= g.oz) | __ballot(b.z >= g.oz)) &
+                       (__ballot(a.z <= g.ez) | __ballot(b.z <= g.ez));
+    return x & y & z;
+}
+
 // The step segment clipped to the grid box: reciprocal direction components,
 // plane offsets and the parameter interval [t_in, t_out] inside the box
 // (empty if t_in > t_out). Every operation is spelled out (explicit FMAs,
@@ -117,10 +134,39 @@ __host__ __device__ __forceinline__ uint32_t float_bits(float x) {
 #endif
 }
 
+// What decides most planar targets without plane_hit's correctly rounded division:
+// its values from an approximate 1 / dir_z, taken once per segment, with bounds that
+// only let through more. d and d' = (t.z - z) rcp(dir_z) differ by 2.5e-7 of their
+// size at most, and with the roundings of the crossing point that moves x and y
+// by less than 5e-7 (step + |x|) + 2e-7 |x - t.x|. A target is passed over
+// where d' lies outside [0, step] or the point outside the square around
+// the shape by more than eight times that; everything else, a NaN among it, is
+// decided by plane_hit.
+struct PlaneFilter {
+    float inv_z, lim, slack;
+    __host__ __device__ __forceinline__ PlaneFilter(f3 pos, f3 dir, float step) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        inv_z = __builtin_amdgcn_rcpf(dir.z);
+#else
+        inv_z = 1.0f / dir.z;
+#endif
+        lim = step * 1.000004f;
+        slack = 4e-6f * (step + fmaxf(fabsf(pos.x), fabsf(pos.y)));
+    }
+    // e.y, e.z: the half lengths (a disc's radius)
+    __host__ __device__ __forceinline__ bool misses(float4 t, float4 e, f3 pos, f3 dir) const {
+        const float d = (t.z - pos.z) * inv_z;
+        const float x = fmaf(dir.x, d, pos.x) - t.x, y = fmaf(dir.y, d, pos.y) - t.y;
+        return (d < -1e-30f) | (d > lim) | (fabsf(x) > fmaf(e.y, 1.000004f, slack)) |
+               (fabsf(y) > fmaf(e.z, 1.000004f, slack));
+    }
+};
+
 // Target lists with planar shapes: every target in index order, as
 // BruteSearch, with the shape test chosen per target (the kind is the same
 // for all lanes, so the branch is wave-uniform). Two records per target:
-// (x, y, z, r^2) and (kind bits, length_x/2, length_y/2, 0).
+// (x, y, z, r^2) and (kind bits, length_x/2, length_y/2, 0), a disc's lengths
+// being its diameter.
 struct MixedSearch {
     const float4* tgt;
     int n;
@@ -133,13 +179,19 @@ struct MixedSearch {
                                                  Work& w) const {
         if (COUNT) w.tests += (uint32_t)n;
         const float ex = dir_excess(dir);
+        const PlaneFilter plane(pos, dir, step);
         int found = -1;
         for (int t = 0; t < n; ++t) {
             const float4 a = tgt[2 * t], e = tgt[2 * t + 1];
             const uint32_t kind = float_bits(e.x);
             float d;
-            const bool h = kind == PP_SHAPE_SPHERE ? sphere_hit(a, pos, dir, ex, step, d)
-                                                   : plane_hit(kind, a, e, pos, dir, step, d);
+            bool h;
+            if (kind == PP_SHAPE_SPHERE) {
+                h = sphere_hit(a, pos, dir, ex, step, d);
+            } else {
+                if (plane.misses(a, e, pos, dir)) continue;
+                h = plane_hit(kind, a, e, pos, dir, step, d);
+            }
             if (h && found < 0) {
                 found = t;
                 dt = d;
@@ -198,21 +250,8 @@ struct GridSearch {
         const bool z = ((a.z >= g.oz) | (b.z >= g.oz)) & ((a.z <= g.ez) | (b.z <= g.ez));
         return x & y & z;
     }
-    // touches() of every lane as a wave mask: each compare is a ballot of its
-    // own (one v_cmp writing a scalar mask) and the masks are combined by
-    // scalar instructions; as one lane condition the compiler merged the
-    // pairs of compares into minima and maxima, which need a canonicalising
-    // instruction per operand, and copied the result out of and back into a
-    // mask
-    __device__ __forceinline__ uint64_t touch_mask(f3 a, f3 b) const {
-        const uint64_t x = (__ballot(a.x >= g.ox) | __ballot(b.x >= g.ox)) &
-                           (__ballot(a.x <= g.ex) | __ballot(b.x <= g.ex));
-        const uint64_t y = (__ballot(a.y >= g.oy) | __ballot(b.y >= g.oy)) &
-                           (__ballot(a.y <= g.ey) | __ballot(b.y <= g.ey));
-        const uint64_t z = (__ballot(a.z >= g.oz) | __ballot(b.z >= g.oz)) &
-                           (__ballot(a.z <= g.ez) | __ballot(b.z <= g.ez));
-        return x & y & z;
-    }
+    // touches() of every lane as a wave mask
+    __device__ __forceinline__ uint64_t touch_mask(f3 a, f3 b) const { return pp::touch_mask(g, a, b); }
     template <bool COUNT, bool COLS>
     __host__ __device__ __forceinline__ int walk(f3 pos, f3 dir, float step, float& dt,
                                                  Work& w) const {
