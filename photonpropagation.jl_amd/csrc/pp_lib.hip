@@ -232,10 +232,11 @@ struct HitRec {
     uint64_t pid;
 };
 
-// x of the wave's first lane, as a scalar
+// x of the wave's first lane, as a scalar (the builtin returns an int, which would
+// extend its sign into the high word)
 __device__ __forceinline__ uint64_t uniform64(uint64_t x) {
-    return ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(x >> 32)) << 32) |
-           __builtin_amdgcn_readfirstlane((uint32_t)x);
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(x >> 32)) << 32) |
+           (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)x);
 }
 
 // Returns false if this lane's record did not fit (overflow).
@@ -587,10 +588,7 @@ __device__ __forceinline__ uint32_t transport_group(const KParams& p, const pp_s
     pp::Stream s{p.k0, p.k1, (uint32_t)pid, (uint32_t)(pid >> 32), src_ix};
     const pp::StepStream ss(s);
     // the wave's photon ids are consecutive: pid = wave_first + lane
-    const uint64_t pid0 = pid - lane;
-    const uint64_t wave_first =
-        ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(pid0 >> 32)) << 32) |
-        __builtin_amdgcn_readfirstlane((uint32_t)pid0);
+    const uint64_t wave_first = uniform64(pid - lane);
     f3 pos = pp::make3(0.0f, 0.0f, 0.0f), dir = pos;
     float ln2_sca = 0.0f;
     if (active) {

@@ -97,3 +97,17 @@ def test_overflow(P, gpu_lib, capacity):
                                   ctypes.byref(n_hits), ctypes.byref(n_sim))
             assert rc == P._lib.PP_ERR_HIT_OVERFLOW and n_hits.value == capacity
             assert capacity <= n_sim.value <= photons - (full - capacity)
+
+
+@pytest.mark.parametrize("n_targets", [1, 12])  # queued scan, grid
+def test_photon_ids_beyond_31_bits(P, gpu_lib, n_targets):
+    rng = np.random.default_rng(4)
+    targets = [P.spherical_target(12.0 * P.workloads.isotropic_unit(rng), 0.3, i + 1)
+               for i in range(n_targets)]
+    medium = P.SimpleMediumProperties(500.0, 300.0, 1.35, 0.95, 0.22)
+    sources = [P.PointlikeIsotropicEmitter(np.zeros(3, np.float32), 0.0, (1 << 31) + 40_000_000)]
+    out = [propagate(P, targets, medium, sources, s, 1, P._lib.BATCH_PERSISTENT, 1 << 24)
+           for s in (P._lib.SEARCH_BRUTE, P._lib.SEARCH_AUTO)]
+    assert out[0][0]["photon_id"].max() > 1 << 31
+    for c in out[0][0]:
+        assert np.array_equal(out[0][0][c], out[1][0][c]), c
