@@ -206,7 +206,10 @@ __device__ __forceinline__ f3 rot_from_ez(f3 a, f3 b) {
     o.x = fmaf(-a.y, hv, fmaf(c, b.x, a.x * b.z));
     o.y = fmaf(a.x, hv, fmaf(c, b.y, a.y * b.z));
     o.z = fmaf(c, b.z, -fmaf(a.x, b.x, a.y * b.y));
-    if (!up && s2 == 0.0f) o = make3(b.x, -b.y, -b.z);
+    // (a wave's branch: as selects the case took three instructions of every step)
+    const bool down = !up && s2 == 0.0f;
+    if (__builtin_expect(__ballot(down) != 0, 0))
+        if (down) o = make3(b.x, -b.y, -b.z);
     return o;
 }
 

@@ -33,21 +33,26 @@ struct GridDesc {
     float ex, ey, ez;  // upper corner, ox + nx h etc. (rounded once, on the host)
 };
 
-// Lanes whose segment a-b comes near the box of g, as a wave mask: whether the
-// bounding box of the segment meets it. Each compare is a ballot of its
-// own (one v_cmp writing a scalar mask) and the masks are combined by
-// scalar instructions; as one lane condition the compiler merged the
-// pairs of compares into minima and maxima, which need a canonicalising
-// instruction per operand, and copied the result out of and back into a
-// mask
-__device__ __forceinline__ uint64_t touch_mask(const GridDesc& g, f3 a, f3 b) {
-    const uint64_t x = (__ballot(a.x >= g.ox) | __ballot(b.x >= g.ox)) &
-                       (__ballot(a.x <= g.ex) | __ballot(b.x <= g.ex));
-    const uint64_t y = (__ballot(a.y >= g.oy) | __ballot(b.y >= g.oy)) &
-                       (__ballot(a.y <= g.ey) | __ballot(b.y <= g.ey));
-    const uint64_t z = (__ballot(a.z >= g.oz) | __ballot(b.z >= g.oz)) &
-                       (__ballot(a.z <= g.ez) | __ballot(b.z <= g.ez));
-    return x & y & z;
+// The lanes whose point lies at or beyond each face of g's box, inwards, as wave
+// masks. Each compare is a ballot of its own (one v_cmp writing a scalar mask);
+// as one lane condition the compiler merged pairs of compares into minima and
+// maxima, which need a canonicalising instruction per operand, and copied the
+// result out of and back into a mask.
+struct BoxSides {
+    uint64_t lo[3], hi[3];
+};
+__device__ __forceinline__ BoxSides box_sides(const GridDesc& g, f3 p) {
+    return BoxSides{{__ballot(p.x >= g.ox), __ballot(p.y >= g.oy), __ballot(p.z >= g.oz)},
+                    {__ballot(p.x <= g.ex), __ballot(p.y <= g.ey), __ballot(p.z <= g.ez)}};
+}
+// Lanes whose segment comes near the box: whether the bounding box of the segment
+// between the points of a and b meets it. One step's end is the next one's start,
+// so that a step takes the six compares of its end alone.
+__device__ __forceinline__ uint64_t touch_mask(const BoxSides& a, const BoxSides& b) {
+    uint64_t m = ~0ull;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) m &= (a.lo[k] | b.lo[k]) & (a.hi[k] | b.hi[k]);
+    return m;
 }
 
 // The step segment clipped to the grid box: reciprocal direction components,
@@ -240,18 +245,10 @@ struct GridSearch {
         c.t_out = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fminf(fmaxf(tz0, tz1), step));
         return c;
     }
-    // Whether the bounding box of the segment a-b meets the grid box: a
-    // superset of the segments that clip() keeps (the grid box holds every
-    // target's box with a margin of at least 2 mm, far beyond the rounding of
-    // the end point b), by compares alone, combined without branches
-    __host__ __device__ __forceinline__ bool touches(f3 a, f3 b) const {
-        const bool x = ((a.x >= g.ox) | (b.x >= g.ox)) & ((a.x <= g.ex) | (b.x <= g.ex));
-        const bool y = ((a.y >= g.oy) | (b.y >= g.oy)) & ((a.y <= g.ey) | (b.y <= g.ey));
-        const bool z = ((a.z >= g.oz) | (b.z >= g.oz)) & ((a.z <= g.ez) | (b.z <= g.ez));
-        return x & y & z;
-    }
-    // touches() of every lane as a wave mask
-    __device__ __forceinline__ uint64_t touch_mask(f3 a, f3 b) const { return pp::touch_mask(g, a, b); }
+    // touch_mask of these is a superset of the segments that clip() keeps: the grid
+    // box holds every target's box with a margin of at least 2 mm, far beyond the
+    // rounding of a segment's end point
+    __device__ __forceinline__ BoxSides sides(f3 p) const { return box_sides(g, p); }
     template <bool COUNT, bool COLS>
     __host__ __device__ __forceinline__ int walk(f3 pos, f3 dir, float step, float& dt,
                                                  Work& w) const {
