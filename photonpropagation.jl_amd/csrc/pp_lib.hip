@@ -1211,7 +1211,8 @@ struct pp_ctx {
     void* hit_mem = nullptr;
     HitCols hits{};
     Counters* d_counters = nullptr;  // at the front of d_batch
-    Counters* h_counters = nullptr;  // pinned: the last propagation's, written by its last kernel
+    // in h_batch, after the staged zeros: the last propagation's, written by its last kernel
+    Counters* h_counters = nullptr;
     bool has_medium = false;
     pp_medium medium_in{};
     pp::Medium medium{};
@@ -1466,8 +1467,10 @@ int max_resident_blocks(pp_ctx* c, const void* fn, int block, size_t lds, int64_
     return PP_OK;
 }
 
-constexpr size_t kTableSources = 256;  // offset of the sources in the table, after the counters
-static_assert(sizeof(Counters) <= kTableSources, "counters precede the sources");
+// offset of the sources in the table, after the counters (in the pinned table: the
+// staged zeros, then the counters that come back)
+constexpr size_t kCounterBytes = 256, kTableSources = 2 * kCounterBytes;
+static_assert(sizeof(Counters) <= kCounterBytes, "counters precede the sources");
 
 // The context's table (device) and its pinned staging, grown to at least
 // `bytes`, the staged counters zeroed. Waits for the stream where earlier work
@@ -1479,15 +1482,16 @@ int ensure_batch_table(pp_ctx* c, size_t bytes) {
         if (c->d_batch) PP_HIP(hipFree(c->d_batch));
         if (c->h_batch) PP_HIP(hipHostFree(c->h_batch));
         c->d_batch = c->h_batch = nullptr;
-        c->d_counters = nullptr;
+        c->d_counters = c->h_counters = nullptr;
         c->batch_cap = 0;
         const size_t cap = std::max<size_t>(bytes, 64 * 1024);
         PP_HIP(hipMalloc((void**)&c->d_batch, cap));
         PP_HIP(hipHostMalloc((void**)&c->h_batch, cap, hipHostMallocDefault));
         c->batch_cap = cap;
         c->d_counters = (Counters*)c->d_batch;
+        c->h_counters = (Counters*)(c->h_batch + kCounterBytes);
     }
-    std::memset(c->h_batch, 0, kTableSources);
+    std::memset(c->h_batch, 0, kCounterBytes);
     return PP_OK;
 }
 
@@ -1814,8 +1818,6 @@ int pp_create(pp_ctx** out, int device, int64_t hit_capacity, const pp_config* c
     }
     ctx->hits.rec = (HitRecord*)ctx->hit_mem;
     ctx->hits.capacity = cap;
-    if (hipHostMalloc((void**)&ctx->h_counters, sizeof(Counters), hipHostMallocDefault) != hipSuccess)
-        return cleanup(fail(PP_ERR_NOMEM, "pp_create: counters"));
     *out = ctx;
     return PP_OK;
 }
@@ -1825,7 +1827,6 @@ int pp_destroy(pp_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->hit_mem) (void)hipFree(ctx->hit_mem);
-    if (ctx->h_counters) (void)hipHostFree(ctx->h_counters);
     if (ctx->d_spec) (void)hipFree(ctx->d_spec);
     if (ctx->d_targets) (void)hipFree(ctx->d_targets);
     if (ctx->d_cells) (void)hipFree(ctx->d_cells);

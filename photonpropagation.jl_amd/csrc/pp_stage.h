@@ -26,8 +26,11 @@ struct PinnedPair {
             if (!e)
                 if (hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming)) return r;
         if (bytes <= half) return hipSuccess;
+        // in eighths of a power of two: pinning takes its time by the page
         size_t want = (size_t)64 << 10;
         while (want < bytes) want *= 2;
+        const size_t step = want / 8;
+        want = std::max((size_t)64 << 10, (bytes + step - 1) / step * step);
         if (p) (void)hipHostFree(p);
         p = nullptr;
         half = 0;
