@@ -138,6 +138,9 @@ enum pp_spectrum_mapping {
 };
 
 /* ---- configuration ---------------------------------------------------- */
+/* AUTO: the grid beyond eight spheres, else every target in index order; large
+ * launches queue the segments near the targets and test those alone. BRUTE tests
+ * every target at every step. The hits are the same bits. */
 enum pp_search_kind { PP_SEARCH_AUTO = 0, PP_SEARCH_BRUTE = 1, PP_SEARCH_GRID = 2 };
 
 /* How pp_propagate schedules a source list. The reference launches one
