@@ -120,15 +120,18 @@ def check_pmt_hit(hit_positions, hit_directions, hit_wavelengths, target: POM, o
 def _relative(pos, center, radius, rows=8192):
     """(pos - center) / radius in Float64, rounded to Float32: block by block in
     a temporary that stays in the cache, and on flat arrays, since NumPy's inner
-    loop over rows of three costs more than the arithmetic (300000 hits: 1.1 ms as
-    one expression on the rows, 0.5 ms here)."""
+    loop over rows of three costs more than the arithmetic (300000 hits: 1.2 ms as
+    one expression on the rows, 0.5 ms here). The block is no longer than the
+    list: 1 hit takes 3 us as one expression and here, 13 us with a whole block."""
     flat = np.ascontiguousarray(pos).reshape(-1)
-    tiled = np.tile(np.asarray(center, np.float64), rows)
+    tiled = np.tile(np.asarray(center, np.float64), max(1, min(rows, len(pos))))
     rel = np.empty(pos.shape, np.float32)
     out = rel.reshape(-1)
+    work = np.empty(tiled.size)
     for i in range(0, flat.size, tiled.size):
         block = flat[i:i + tiled.size]
-        d = block - tiled[:block.size]
+        d = work[:block.size]
+        np.subtract(block, tiled[:block.size], out=d)
         d /= radius
         out[i:i + block.size] = d
     return rel
