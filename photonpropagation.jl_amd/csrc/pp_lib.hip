@@ -756,7 +756,6 @@ __device__ __forceinline__ pp_source source_record(const pp_source* sp, uint32_t
 struct WaveState {
     WaveQueue q{};
     uint32_t n_queued = 0;    // hits in q.out
-    bool overflow = false;    // the hit buffer was full: per lane in the plain scans, else uniform
     unsigned long long n_steps_done = 0;
     pp::Work work;
 };
@@ -770,34 +769,40 @@ __device__ __forceinline__ void add_lost(uint64_t n) {
         atomicAdd(&kernel_params()->counters->n_lost, (unsigned long long)n);
 }
 
+// Photons of the groups of 64 that start at first, first + stride, ... before end.
+__device__ __forceinline__ uint64_t strided_photons(uint64_t first, uint64_t end, uint64_t stride) {
+    if (first >= end) return 0;
+    const uint64_t more = (end - 1 - first) / stride;  // groups after the first
+    const uint64_t last = first + more * stride;
+    return more * 64 + (end - last < 64 ? end - last : 64);
+}
+
 // 64 photons from base on (up to end), one per lane, the whole wave together,
-// hits stored or queued. A lane or wave that met a full hit buffer takes no more
-// photons and counts those it is given as lost.
+// hits stored or queued. False if the hit buffer was full: the photons whose hits
+// did not fit are counted as lost, and the wave takes no more of them.
 template <bool COUNT, int SEARCH>
-__device__ __forceinline__ void propagate_group(const KParams& p, const pp_source& src,
+__device__ __forceinline__ bool propagate_group(const KParams& p, const pp_source& src,
                                                 uint32_t src_ix, uint64_t base, uint64_t end,
                                                 const float* spec, const SearchT<SEARCH>& search,
                                                 const pp::Phase& phase, WaveState& w) {
     const uint64_t pid = base + __lane_id();
+    uint32_t lost;
     if constexpr (kDeferredWalk<SEARCH>) {
-        if (w.overflow) {
-            add_lost(end - base < 64 ? end - base : 64);
-            return;
-        }
-        const uint32_t lost = transport_group<COUNT, SEARCH>(p, src, src_ix, pid, pid < end, spec, search,
-                                                     phase, w.q, w.n_queued, w.work, w.n_steps_done);
-        add_lost(lost);
-        w.overflow = lost != 0;
+        lost = transport_group<COUNT, SEARCH>(p, src, src_ix, pid, pid < end, spec, search, phase, w.q,
+                                              w.n_queued, w.work, w.n_steps_done);
     } else {
-        if (pid < end && !w.overflow) {
+        bool stored = true;
+        if (pid < end) {
             HitRec h;
             const bool hit = transport_photon<COUNT>(p, src, src_ix, pid, spec, search, phase,
                                                      w.work, w.n_steps_done, h);
-            w.overflow = !store_hits(hit, h, src_ix, p.hits, p.counters);
-            if (w.overflow) atomicOr(&p.counters->err, 1u);
+            stored = store_hits(hit, h, src_ix, p.hits, p.counters);
+            if (!stored) atomicOr(&p.counters->err, 1u);
         }
-        add_lost((uint64_t)__popcll(__ballot(w.overflow && pid < end)));
+        lost = (uint32_t)__popcll(__ballot(!stored));
     }
+    add_lost(lost);
+    return lost == 0;
 }
 
 // The wave's queued hits stored, and its counts added.
@@ -826,7 +831,12 @@ __global__ void PP_PROPAGATE_ATTRS propagate_kernel(KParams p) {
          base < p.n_photons; base += stride) {
         uint32_t si = p.src_ix;
         const pp_source src = source_record(p.sources + p.src_ix, si);
-        propagate_group<COUNT, SEARCH>(p, src, si, base, p.n_photons, l.spec, search, phase, w);
+        if (!propagate_group<COUNT, SEARCH>(p, src, si, base, p.n_photons, l.spec, search, phase, w)) {
+            // the call fails: the wave's later groups are given up in one sum (an
+            // atomic for each held a launch of 1e9 photons for 190 ms)
+            add_lost(strided_photons(base + stride, p.n_photons, stride));
+            break;
+        }
     }
     finish_wave<COUNT, SEARCH>(p, w);
 }
@@ -915,23 +925,27 @@ __global__ void PP_PROPAGATE_ATTRS propagate_batch_kernel(KParams p, BatchParams
         const uint64_t ck = uniform64(next);
         if (ck >= batch_params().n_items) break;
         const BatchItem it = batch_item(ck);
-        for (uint64_t base = it.first; base < it.end; base += 64) {
+        bool fits = true;
+        for (uint64_t base = it.first; base < it.end && fits; base += 64) {
             // the source index and record, opaque to the optimiser in every
             // iteration: what the emission derives from them is computed here
             // (one scalar reload per 64 photons) instead of being hoisted out
             // of the loop into registers that then spill to scratch
             uint32_t si = (uint32_t)it.source;
             const pp_source src = source_record(batch_params().sources + it.source, si);
-            propagate_group<COUNT, SEARCH>(p, src, si, base, it.end, l.spec, search, phase, w);
+            fits = propagate_group<COUNT, SEARCH>(p, src, si, base, it.end, l.spec, search, phase, w);
+            if (!fits && it.end - base > 64) add_lost(it.end - base - 64);
         }
-        if (__ballot(w.overflow)) {
+        if (!fits) {
             // the call fails; take no more chunks, and give those dealt to this wave up
             const BatchParams b = batch_params();
+            uint64_t left = 0;
             if (b.dealt)
                 for (uint64_t k = ck + waves; k < b.n_items; k += waves) {
                     const BatchItem rest = batch_item(k);
-                    add_lost(rest.end - rest.first);
+                    left += rest.end - rest.first;
                 }
+            add_lost(left);
             break;
         }
         next = ck;
