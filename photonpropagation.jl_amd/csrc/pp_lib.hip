@@ -1207,12 +1207,13 @@ bool finite3(const float* v) {
 
 }  // namespace
 
-// What the automatic block size of a launch depends on.
+// What the automatic block size and placement of a launch depend on.
 struct OccKey {
     const void* fn = nullptr;
     size_t tables = 0, mem_tables = 0;  // LDS tables with and without the targets
+    int block = 0;                      // the set block size
     bool operator==(const OccKey& o) const {
-        return fn == o.fn && tables == o.tables && mem_tables == o.mem_tables;
+        return fn == o.fn && tables == o.tables && mem_tables == o.mem_tables && block == o.block;
     }
 };
 
@@ -2128,19 +2129,21 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
     // waves: 1000 targets, 16 KB, leave 24 waves in 768-thread blocks (27.0 ms
     // for the 256-source batch) and 28 in 256-thread blocks without them (25.8
     // ms); 320 targets leave 28 either way, and are read from LDS (1e8-photon
-    // cascade: 7.07 ms, from memory 7.27).
+    // cascade: 7.07 ms, from memory 7.27). With a set block size the placement
+    // follows the same rule (another 256-source batch at a set 256: 17.0 ms, with
+    // the targets held in LDS 20.4; automatic 17.0).
     int block = ctx->cfg.block_size;
-    if (block == 0) {
+    if (block == 0 || skind == kSearchGrid) {
         const OccKey key{batch_kernel_fn(skind, phase), table_bytes(skind),
-                         table_bytes(kSearchGridMem)};
+                         table_bytes(kSearchGridMem), block};
         if (!(key == ctx->occ_key)) {
             int best_waves = 0;
-            ctx->occ_block = 64;  // the LDS check below reports what does not fit
+            ctx->occ_block = block ? block : 64;  // the LDS check below reports what does not fit
             ctx->occ_skind = skind;
             for (int kind : {skind, (int)kSearchGridMem}) {
-                if (kind != skind && skind != kSearchGrid) continue;
+                if (kind != skind && (skind != kSearchGrid || best_waves == 0)) continue;
                 const void* fn = batch_kernel_fn(kind, phase);
-                for (int b : {256, 384, 512, 768, 1024}) {
+                for (int b : block ? std::vector<int>{block} : std::vector<int>{256, 384, 512, 768, 1024}) {
                     const size_t need = with_queues(kind, b);
                     if (need > (size_t)kMaxLdsBytes) continue;
                     int occ = 0;
