@@ -1265,8 +1265,6 @@ struct pp_ctx {
     HitRecord* h_rec = nullptr;
     int64_t h_rec_cap = 0;
     pp::PinnedPair pin;  // PMT ids and hit columns on their way to pageable host memory
-    char* d_cols = nullptr;  // two slices of hit columns
-    size_t cols_cap = 0;
     // device sort of the hits by (source, photon id): the records in that
     // order, keys, indices and the radix sort's scratch, in one allocation
     char* d_sort = nullptr;
@@ -1852,7 +1850,6 @@ int pp_destroy(pp_ctx* ctx) {
     if (ctx->h_batch) (void)hipHostFree(ctx->h_batch);
     if (ctx->h_rec) (void)hipHostFree(ctx->h_rec);
     if (ctx->d_sort) (void)hipFree(ctx->d_sort);
-    if (ctx->d_cols) (void)hipFree(ctx->d_cols);
     if (ctx->d_tgt_r) (void)hipFree(ctx->d_tgt_r);
     if (ctx->d_pmt) (void)hipFree(ctx->d_pmt);
     ctx->pin.release();
@@ -2498,20 +2495,28 @@ static int sort_hits_device(pp_ctx* ctx, bool* done, HitRecord* host = nullptr) 
 }
 
 // The caller's columns of a hit table, and where each lies in a slice of
-// kSliceRows rows of them (kNoColumn: not asked for).
+// its rows (kNoColumn: not asked for).
 enum { kColPos, kColDir, kColInit, kColWl, kColTime, kColDist, kColModule, kColSteps, kColPid, kColSrc,
        kColumns };
-constexpr int64_t kSliceRows = 32768;
+constexpr int64_t kSliceRows = 16384;  // of tables of up to 8 such slices; longer ones: twice
 constexpr uint32_t kNoColumn = ~0u;
 struct ColumnSet {
     uint32_t off[kColumns];
     int32_t time_f64;
 };
 
-// Rows of hit records as columns. Splitting the records up on the host cost 7 ns a
-// row and could not run beside the copy of the next ones (381970 hits: 2.9 ms);
-// the columns of a slice are copied to pinned memory while the host moves those of
-// the slice before, one memcpy a column (1.2 ms).
+// Rows of hit records as columns, `out` being pinned host memory. Splitting the
+// records up on the host cost 7 ns a row and could not run beside the copy of the
+// next ones (383224 hits: 2.8-3.2 ms a call); the columns of a slice are written
+// while the host moves those of the slice before, one memcpy a column (1.0 ms).
+// Written to device memory and copied from there, the first four copies of a
+// context were slow: first and fourth call on 15430 hits 0.28 and 0.12 ms (split up
+// on the host: 0.24-0.28 and 0.17-0.19), on 65177 hits 0.63 and 0.25 (0.74-0.82 and
+// 0.50-0.56); straight to host memory 0.12 and 0.11, 0.26 and 0.23. Pinned memory
+// that is new to the process costs the host 0.35 ms a MB when it is first touched:
+// a table of one slice takes one half, and the slices of a few are half as long
+// (65177 hits in a process's first context: 1.1-2.5 ms of call, else 3.6-4.3). Beyond
+// 131072 rows the longer ones save more (383224 hits: 0.97-1.03 and 1.06-1.08 ms).
 __global__ void __launch_bounds__(256) hit_columns_kernel(const HitRecord* __restrict__ rec, int n,
                                                           char* __restrict__ out, ColumnSet cs) {
     const int k = blockIdx.x * 256 + threadIdx.x;
@@ -2544,13 +2549,13 @@ __global__ void __launch_bounds__(256) hit_columns_kernel(const HitRecord* __res
 
 // Rows [0, n) of the device records src to the caller's columns (NULL: not asked
 // for), slice by slice. Sets *done = false and does nothing where the slices do
-// not fit device or pinned memory.
+// not fit pinned memory.
 static int copy_columns(pp_ctx* ctx, const HitRecord* src, int64_t n, void* const col[kColumns],
                         const uint32_t width[kColumns], int time_f64, bool* done) {
     *done = false;
     ColumnSet cs{};
     cs.time_f64 = time_f64;
-    const int64_t rows = std::min<int64_t>(n, kSliceRows);
+    const int64_t rows = std::min<int64_t>(n, n <= 8 * kSliceRows ? kSliceRows : 2 * kSliceRows);
     size_t bytes = 0;
     for (int c = 0; c < kColumns; ++c) {
         cs.off[c] = col[c] ? (uint32_t)bytes : kNoColumn;
@@ -2560,32 +2565,18 @@ static int copy_columns(pp_ctx* ctx, const HitRecord* src, int64_t n, void* cons
         *done = true;
         return PP_OK;
     }
-    if (2 * bytes > ctx->cols_cap) {
-        if (ctx->d_cols) PP_HIP(hipFree(ctx->d_cols));
-        ctx->d_cols = nullptr;
-        ctx->cols_cap = 0;
-        if (hipMalloc((void**)&ctx->d_cols, 2 * bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            ctx->d_cols = nullptr;
-            return PP_OK;
-        }
-        ctx->cols_cap = 2 * bytes;
-    }
-    if (ctx->pin.ensure(bytes) != hipSuccess) {
+    const int64_t slices = (n + rows - 1) / rows;
+    if (ctx->pin.ensure(bytes, slices > 1 ? 2 : 1) != hipSuccess) {
         (void)hipGetLastError();
         return PP_OK;
     }
-    const int64_t slices = (n + rows - 1) / rows;
     auto slice_rows = [&](int64_t k) { return std::min<int64_t>(rows, n - k * rows); };
     auto move = [&](int64_t k) -> int {
         if (k < slices) {
             const int64_t m = slice_rows(k);
-            char* out = ctx->d_cols + (k & 1) * bytes;
             hipLaunchKernelGGL(hit_columns_kernel, dim3((unsigned)((m + 255) / 256)), dim3(256), 0,
-                               ctx->stream, src + k * rows, (int)m, out, cs);
+                               ctx->stream, src + k * rows, (int)m, ctx->pin.at((int)(k & 1)), cs);
             PP_HIP(hipGetLastError());
-            PP_HIP(hipMemcpyAsync(ctx->pin.at((int)(k & 1)), out, bytes, hipMemcpyDeviceToHost,
-                                  ctx->stream));
             PP_HIP(hipEventRecord(ctx->pin.ev[k & 1], ctx->stream));
         }
         if (k > 0) {
@@ -2747,9 +2738,6 @@ int pp_release_scratch(pp_ctx* ctx) {
     ctx->h_rec_cap = 0;
     ctx->d_pmt = nullptr;
     ctx->pmt_cap = 0;
-    if (ctx->d_cols) PP_HIP(hipFree(ctx->d_cols));
-    ctx->d_cols = nullptr;
-    ctx->cols_cap = 0;
     ctx->pin.release();
     std::vector<int64_t>().swap(ctx->perm);
     ctx->perm_valid = false;

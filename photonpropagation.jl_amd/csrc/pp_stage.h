@@ -1,8 +1,10 @@
-// pp_stage.h - copies between device memory and pageable host memory through
-// two pinned halves that their owner keeps. The runtime's own copy from device
-// to pageable memory took 408 us for 1 MB and 1450 us for 20 MB (to fresh
+// pp_stage.h - results on their way from the device to pageable host memory,
+// through two pinned halves that their owner keeps. The runtime's own copy from
+// device to pageable memory took 408 us for 1 MB and 1450 us for 20 MB (to fresh
 // pages); through the pinned halves, one being filled by the device while the
 // other is emptied by the host, 40 us and 700 us. Measured on MI355X.
+// Kernels may write the halves themselves: the memory is coherent, so that their
+// stores are visible once an event or stream behind them is done.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -14,18 +16,21 @@
 namespace pp {
 
 struct PinnedPair {
-    char* p = nullptr;  // two halves
-    size_t half = 0;    // bytes of each
+    char* p = nullptr;
+    size_t half = 0;    // bytes of each half
+    int halves = 0;     // one where all the work is a single piece, else two
     hipEvent_t ev[2] = {nullptr, nullptr};
 
     static constexpr size_t kMost = (size_t)4 << 20;  // half of copy_out's own choice
 
     // At least `bytes` per half. Work that still uses the old halves must be done.
-    hipError_t ensure(size_t bytes) {
+    hipError_t ensure(size_t bytes, int n = 2) {
         for (auto& e : ev)
             if (!e)
                 if (hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming)) return r;
-        if (bytes <= half) return hipSuccess;
+        if (bytes <= half && n <= halves) return hipSuccess;
+        bytes = std::max(bytes, half);
+        n = std::max(n, halves);
         // in eighths of a power of two: pinning takes its time by the page
         size_t want = (size_t)64 << 10;
         while (want < bytes) want *= 2;
@@ -34,8 +39,10 @@ struct PinnedPair {
         if (p) (void)hipHostFree(p);
         p = nullptr;
         half = 0;
-        if (hipError_t r = hipHostMalloc((void**)&p, 2 * want, hipHostMallocDefault)) return r;
+        halves = 0;
+        if (hipError_t r = hipHostMalloc((void**)&p, n * want, hipHostMallocCoherent)) return r;
         half = want;
+        halves = n;
         return hipSuccess;
     }
     char* at(int k) const { return p + (size_t)(k & 1) * half; }
@@ -47,12 +54,13 @@ struct PinnedPair {
         }
         p = nullptr;
         half = 0;
+        halves = 0;
     }
 
     // dst (host) <- src (device), ordered on the stream; returns when dst is written
     hipError_t copy_out(hipStream_t st, void* dst, const void* src, size_t bytes) {
         if (bytes == 0) return hipStreamSynchronize(st);
-        if (hipError_t r = ensure(std::min(bytes, kMost))) return r;
+        if (hipError_t r = ensure(std::min(bytes, kMost), bytes > kMost ? 2 : 1)) return r;
         const size_t n = (bytes + half - 1) / half;
         auto part = [&](size_t k) { return std::min(half, bytes - k * half); };
         for (size_t k = 0; k <= n; ++k) {
