@@ -123,8 +123,8 @@ int pp_sur_features(pp_mlp* m, const pp_cascade* cascades, const float* module_x
  * (n_events x n_modules, host), the mixture parameters (n_events x
  * n_modules x 9: weights, shapes, scales in ns; may be NULL) and a fallback
  * mask (1 where the pair is outside `dom`, e.g. closer than min_dist: the
- * caller runs the Monte Carlo for those). All on the device, in chunks of
- * max_batch pairs; *kernel_ms (may be NULL) is the device time. */
+ * caller runs the Monte Carlo for those). All on the device, slice by slice;
+ * *kernel_ms (may be NULL) is the device time. */
 int pp_sur_eval_pairs(pp_mlp* m, const pp_cascade* events, int n_events, const float* module_xyz,
                       int n_modules, const pp_sur_domain* dom, float* expected_hits,
                       float* mixture, uint8_t* fallback, float* kernel_ms);

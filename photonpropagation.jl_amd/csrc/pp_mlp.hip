@@ -868,14 +868,15 @@ struct pp_mlp {
     // training set
     float *dsX = nullptr, *dsL = nullptr;
     int64_t ds_cap = 0;
-    // pair evaluation: events | modules, the outputs of two slices of the list,
-    // the stream their copies run on and the slices' events
+    // pair evaluation: events | modules, the outputs of a list of one slice, the
+    // stream of every other slice of a longer one and the timing events of three
+    // slices in a row
     char* d_in = nullptr;
     size_t in_cap = 0;
     char* d_out = nullptr;
     size_t out_cap = 0;
-    hipStream_t copy = nullptr;
-    hipEvent_t t0[2] = {nullptr, nullptr}, t1[2] = {nullptr, nullptr};
+    hipStream_t other = nullptr;
+    hipEvent_t t0[3] = {}, t1[3] = {};
     float* logy = nullptr;
     pp::PinnedPair pin;  // results on their way to pageable host memory
 };
@@ -934,9 +935,10 @@ int ensure_packed(pp_mlp* M, bool train = false) {
 
 // The fused kernel over `rows` rows: the bf16 input in H[0] to the fp32
 // outputs in Y, or, with pairs set, the pair list's features to the head's
-// outputs (hits, mix, pairs->fb).
-int forward_fused(pp_mlp* M, int64_t rows, const PairArgs* pairs = nullptr, float* hits = nullptr,
-                  float* mix = nullptr) {
+// outputs (hits, mix, pairs->fb). The weights are packed on M->stream, which
+// another `stream` has to have waited for.
+int forward_fused(pp_mlp* M, int64_t rows, hipStream_t stream, const PairArgs* pairs = nullptr,
+                  float* hits = nullptr, float* mix = nullptr) {
     if (int rc = ensure_packed(M)) return rc;
     if (rows <= 0) return PP_OK;
     FusedArgs f{};
@@ -962,7 +964,7 @@ int forward_fused(pp_mlp* M, int64_t rows, const PairArgs* pairs = nullptr, floa
     const auto fn = small ? (pairs ? mlp_small_kernel<true> : mlp_small_kernel<false>)
                           : (pairs ? mlp_fused_kernel<true> : mlp_fused_kernel<false>);
     hipLaunchKernelGGL(fn, dim3(blocks_for(rows, small ? kTRows : kFRows)),
-                       dim3(small ? kTThreads : kFThreads), 0, M->stream, f);
+                       dim3(small ? kTThreads : kFThreads), 0, stream, f);
     PP_HIP(hipGetLastError());
     return PP_OK;
 }
@@ -971,7 +973,7 @@ int forward_fused(pp_mlp* M, int64_t rows, const PairArgs* pairs = nullptr, floa
 // pre-activations that the backward pass needs (and uses the layer-by-layer
 // kernels); inference runs the fused kernel where the shape allows
 int forward(pp_mlp* M, int rows, bool keep_z) {
-    if (!keep_z && M->fused && M->wpk) return forward_fused(M, rows);
+    if (!keep_z && M->fused && M->wpk) return forward_fused(M, rows, M->stream);
     for (int l = 0; l < M->n_mat; ++l) {
         GemmArgs a{};
         a.A = M->H[l];
@@ -1082,7 +1084,9 @@ int backward(pp_mlp* M, int rows) {
     return PP_OK;
 }
 
-constexpr int64_t kPairSlice = (int64_t)1 << 18;  // pairs per slice of a list
+// Pairs per slice of a list (5 bytes each, with mixtures 41): a whole number of
+// rounds of the 128-row tiles (two per CU), so that no CU waits for the last of them.
+constexpr int64_t kPairSlice = (int64_t)3 << 16, kPairMixSlice = (int64_t)1 << 16;
 constexpr size_t kPairPinnedIn = 256 << 10;       // inputs that go through pinned memory (bytes)
 
 // Whether a training step runs as the two launches of pp_train.h: the shapes
@@ -1393,7 +1397,7 @@ int pp_mlp_destroy(pp_mlp* M) {
     if (!M) return PP_OK;
     (void)hipSetDevice(M->device);
     if (M->stream) (void)hipStreamSynchronize(M->stream);
-    if (M->copy) (void)hipStreamSynchronize(M->copy);
+    if (M->other) (void)hipStreamSynchronize(M->other);
     void* ptrs[] = {M->p, M->g, M->m, M->v, M->pb, M->Y, M->dY, M->dYb, M->dA, M->dB, M->Lb, M->xs,
                     M->part, M->wpk, M->wpb, M->ws,
                     M->loss, M->step, M->dsX, M->dsL, M->logy, M->d_in,
@@ -1405,9 +1409,10 @@ int pp_mlp_destroy(pp_mlp* M) {
     for (auto* p : M->Z)
         if (p) (void)hipFree(p);
     M->pin.release();
-    for (hipEvent_t e : {M->t0[0], M->t0[1], M->t1[0], M->t1[1]})
-        if (e) (void)hipEventDestroy(e);
-    if (M->copy) (void)hipStreamDestroy(M->copy);
+    for (int i = 0; i < 3; ++i)
+        for (hipEvent_t e : {M->t0[i], M->t1[i]})
+            if (e) (void)hipEventDestroy(e);
+    if (M->other) (void)hipStreamDestroy(M->other);
     if (M->stream) (void)hipStreamDestroy(M->stream);
     delete M;
     return PP_OK;
@@ -1665,20 +1670,28 @@ int pp_sur_eval_pairs(pp_mlp* M, const pp_cascade* events, int n_events, const f
     const int64_t n = (int64_t)n_events * n_modules;
     if (n == 0) return PP_OK;
     if (int rc = set_dev(M)) return rc;
-    // Lists of up to kPairSlice pairs run at once; longer ones in slices, whose
-    // results go to pinned memory on a stream of their own and from there to the
-    // caller while the next slice is computed (5e6 pairs: 4.2 ms with the copies
-    // after the kernel, 2.9 ms sliced). A slice is a whole number of rounds of
-    // the 128-row tiles (two per CU), so that no CU waits for the last of them.
+    // Lists of one slice run at once; longer ones slice by slice, the kernels writing
+    // to two pinned halves in turn and the host moving a slice to the caller while
+    // the next is computed. Without mixtures every other slice runs on a second
+    // stream: a launch behind another on one stream waits until the other's last
+    // store to host memory has arrived (16 us a slice). Copies from device buffers on
+    // a stream of their own ran at a quarter of the bus beside the kernels for the
+    // first 30 to 80 of them, which shorter lists never got past: first and later
+    // calls of a network on 3e5 pairs 0.70 and 0.59 ms (copies after the kernel, in
+    // one piece: 0.47 and 0.53; like this 0.36 and 0.27), 1e6 pairs 1.26 and 1.18 (1.02
+    // and 0.83; 0.76 and 0.68), 5e6 pairs 4.8-5.4 and 2.9 (4.65 and 4.3; 3.1 and 2.8),
+    // with mixtures 3e5 pairs 1.5 and 1.4 (1.2 and 2.4; 0.74 and 0.69), 2e6 pairs 6.7
+    // and 6.2 (8.6 and 8.5; 5.8 and 5.7). Their stores of 36 bytes a pair stretch the
+    // kernels of the last from 1.0 to 2.5 ms, which the host's part hides.
     const bool fused = M->fused && M->wpk;
-    const int64_t slice = std::min<int64_t>(n, fused ? kPairSlice : std::min<int64_t>(kPairSlice,
-                                                                                     M->max_batch));
+    const int64_t most = mixture ? kPairMixSlice : kPairSlice;
+    const int64_t slice = std::min<int64_t>(n, fused ? most : std::min<int64_t>(most, M->max_batch));
     const size_t off_mod = ((size_t)n_events * sizeof(pp_cascade) + 255) & ~(size_t)255;
     const size_t in_b = off_mod + (size_t)n_modules * 12;
     const size_t off_mix = (size_t)slice * 4;
     const size_t off_fb = off_mix + (mixture ? (size_t)slice * 36 : 0);
     const size_t out_b = (off_fb + (size_t)slice + 255) & ~(size_t)255;
-    const int n_buf = slice < n ? 2 : 1;
+    const bool sliced = slice < n, two = sliced && fused && !mixture;
     auto grow = [&](char** p, size_t* cap, size_t need) -> int {
         if (need <= *cap) return PP_OK;
         if (*p) PP_HIP(hipFree(*p));
@@ -1689,13 +1702,13 @@ int pp_sur_eval_pairs(pp_mlp* M, const pp_cascade* events, int n_events, const f
         return PP_OK;
     };
     if (int rc = grow(&M->d_in, &M->in_cap, in_b)) return rc;
-    if (int rc = grow(&M->d_out, &M->out_cap, out_b * n_buf)) return rc;
+    if (!sliced)
+        if (int rc = grow(&M->d_out, &M->out_cap, out_b)) return rc;
     if (!fused && !M->logy) PP_HIP(hipMalloc(&M->logy, (size_t)M->max_batch * 4));
-    if (n_buf == 2 && !M->copy) {
-        PP_HIP(hipStreamCreateWithFlags(&M->copy, hipStreamNonBlocking));
-        PP_HIP(hipEventCreate(&M->t0[1]));
-        PP_HIP(hipEventCreate(&M->t1[1]));
-    }
+    if (two && !M->other) PP_HIP(hipStreamCreateWithFlags(&M->other, hipStreamNonBlocking));
+    for (int i = 0; i < (sliced ? 3 : 1); ++i)
+        for (hipEvent_t* e : {&M->t0[i], &M->t1[i]})
+            if (!*e) PP_HIP(hipEventCreate(e));
     PP_HIP(M->pin.ensure(std::max(out_b, in_b <= kPairPinnedIn ? in_b : (size_t)0)));
     auto* d_ev = (pp_cascade*)M->d_in;
     auto* d_mod = (float*)(M->d_in + off_mod);
@@ -1709,14 +1722,19 @@ int pp_sur_eval_pairs(pp_mlp* M, const pp_cascade* events, int n_events, const f
         PP_HIP(hipMemcpyAsync(d_mod, module_xyz, (size_t)n_modules * 12, hipMemcpyHostToDevice,
                               M->stream));
     }
-    const hipStream_t out_stream = n_buf == 2 ? M->copy : M->stream;
+    if (two) {  // the inputs and the packed weights, for the other stream too
+        if (int rc = ensure_packed(M)) return rc;
+        PP_HIP(hipEventRecord(M->t1[0], M->stream));
+        PP_HIP(hipStreamWaitEvent(M->other, M->t1[0], 0));
+    }
     float device_ms = 0.0f;
-    // the slice's launches and, behind them, the copy of its results
+    // the slice's launches
     auto start = [&](int64_t k) -> int {
-        const int b = (int)(k & 1);
+        const int b = (int)(k & 1), e = (int)(k % 3);
+        const hipStream_t st = two && b ? M->other : M->stream;
         const int64_t r0 = k * slice;
         const int64_t rows = std::min<int64_t>(slice, n - r0);
-        char* out = M->d_out + (n_buf == 2 ? b : 0) * out_b;
+        char* out = sliced ? M->pin.at(b) : M->d_out;
         PairArgs a{};
         a.ev = d_ev;
         a.mod = d_mod;
@@ -1728,10 +1746,10 @@ int pp_sur_eval_pairs(pp_mlp* M, const pp_cascade* events, int n_events, const f
         a.dom = *dom;
         float* hits = (float*)out;
         float* mix = mixture ? (float*)(out + off_mix) : nullptr;
-        PP_HIP(hipEventRecord(M->t0[b], M->stream));
+        PP_HIP(hipEventRecord(M->t0[e], st));
         if (fused) {
             // features, network and head in one kernel
-            if (int rc = forward_fused(M, rows, &a, hits, mix)) return rc;
+            if (int rc = forward_fused(M, rows, st, &a, hits, mix)) return rc;
         } else {
             a.xb = M->H[0];
             a.logy = M->logy;
@@ -1743,10 +1761,10 @@ int pp_sur_eval_pairs(pp_mlp* M, const pp_cascade* events, int n_events, const f
                                M->stream, M->Y, M->dims.back(), rows, M->logy, hits, mix);
             PP_HIP(hipGetLastError());
         }
-        PP_HIP(hipEventRecord(M->t1[b], M->stream));
-        if (n_buf == 2) PP_HIP(hipStreamWaitEvent(M->copy, M->t1[b], 0));
-        PP_HIP(hipMemcpyAsync(M->pin.at(b), out, out_b, hipMemcpyDeviceToHost, out_stream));
-        PP_HIP(hipEventRecord(M->pin.ev[b], out_stream));
+        PP_HIP(hipEventRecord(M->t1[e], st));
+        if (!sliced)
+            PP_HIP(hipMemcpyAsync(M->pin.at(b), out, out_b, hipMemcpyDeviceToHost, st));
+        PP_HIP(hipEventRecord(M->pin.ev[b], st));
         return PP_OK;
     };
     // the slice's results to the caller
@@ -1760,22 +1778,25 @@ int pp_sur_eval_pairs(pp_mlp* M, const pp_cascade* events, int n_events, const f
         if (mixture) std::memcpy(mixture + r0 * 9, src + off_mix, rows * 36);
         if (fallback) std::memcpy(fallback + r0, src + off_fb, rows);
         if (kernel_ms) {
-            float ms = 0.0f;
-            PP_HIP(hipEventElapsedTime(&ms, M->t0[b], M->t1[b]));
-            device_ms += ms;
+            // of a slice that ran beside the one before, what came after that one
+            const hipEvent_t end = M->t1[k % 3];
+            float ms = 0.0f, after = INFINITY;
+            PP_HIP(hipEventElapsedTime(&ms, M->t0[k % 3], end));
+            if (two && k > 0) PP_HIP(hipEventElapsedTime(&after, M->t1[(k - 1) % 3], end));
+            device_ms += std::max(std::min(ms, after), 0.0f);
         }
         return PP_OK;
     };
     const int64_t slices = (n + slice - 1) / slice;
     int rc = PP_OK;
-    // the second pinned half holds the inputs until the first slice has run
+    // the second pinned half holds the inputs until the first slice can run
     for (int64_t k = 0; k <= slices && rc == PP_OK; ++k) {
         if (k < slices) rc = start(k);
         if (k > 0 && rc == PP_OK) rc = finish(k - 1);
     }
     if (rc != PP_OK) {  // nothing may still use the workspace
         (void)hipStreamSynchronize(M->stream);
-        if (M->copy) (void)hipStreamSynchronize(M->copy);
+        if (M->other) (void)hipStreamSynchronize(M->other);
         return rc;
     }
     if (kernel_ms) *kernel_ms = device_ms;
