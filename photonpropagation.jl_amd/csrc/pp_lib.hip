@@ -1249,7 +1249,7 @@ struct pp_ctx {
     float grid_cell_built = -1.0f;  // requested cell size of the built grid
     bool grid_global = false;        // the built grid's tables exceed the LDS: read from memory
     float grid_cell_z_built = 0.0f;
-    int grid_spec_built = -1;        // spectrum knots the built grid's LDS budget left room for
+    size_t grid_budget = 0;          // LDS bytes the built grid and a spectrum may take
     float4* d_cells = nullptr;
     uint16_t* d_cell_items = nullptr;
     size_t cell_cap = 0, item_cap = 0;
@@ -1329,15 +1329,14 @@ int build_grid(pp_ctx* c, float cell_req, float cell_z_req) {
     // the occupancy-friendly budget first; for many targets (their records
     // alone may fill it) the whole LDS, at fewer workgroups per CU; beyond
     // that, tables in device memory that the search reads through the caches
-    bool global = false;
-    if (!pp::build_grid_tables(xyz.data(), c->h_radius.data(), c->n_targets, cell_req, cell_z_req,
-                               c->spec_n, kGridLdsBudget, t) &&
-        !pp::build_grid_tables(xyz.data(), c->h_radius.data(), c->n_targets, cell_req, cell_z_req,
-                               c->spec_n, kGridLdsMax, t)) {
-        global = true;
-        if (!pp::build_grid_tables(xyz.data(), c->h_radius.data(), c->n_targets, cell_req,
-                                   cell_z_req, c->spec_n, kGridGlobalBudget, t))
-            return fail(PP_ERR_INVALID, "grid: no cell size fits");
+    auto build = [&](size_t budget) {
+        return pp::build_grid_tables(xyz.data(), c->h_radius.data(), c->n_targets, cell_req,
+                                     cell_z_req, c->spec_n, budget, t);
+    };
+    size_t budget = kGridLdsBudget;
+    if (!build(budget) && !build(budget = kGridLdsMax)) {
+        if (!build(kGridGlobalBudget)) return fail(PP_ERR_INVALID, "grid: no cell size fits");
+        budget = 0;
     }
     if (t.cells.size() > c->cell_cap) {
         if (c->d_cells) PP_HIP(hipFree(c->d_cells));
@@ -1360,10 +1359,10 @@ int build_grid(pp_ctx* c, float cell_req, float cell_z_req) {
                           hipMemcpyHostToDevice, c->stream));
     PP_HIP(hipStreamSynchronize(c->stream));
     c->grid = t.g;
-    c->grid_global = global;
+    c->grid_global = budget == 0;
+    c->grid_budget = budget;
     c->grid_cell_built = cell_req;
     c->grid_cell_z_built = cell_z_req;
-    c->grid_spec_built = c->spec_n;
     return PP_OK;
 }
 
@@ -2070,8 +2069,14 @@ int pp_propagate(pp_ctx* ctx, const pp_source* sources, int n_sources, uint64_t 
     }
     if (search == PP_SEARCH_GRID) {
         const float want = ctx->cfg.grid_cell, want_z = ctx->cfg.grid_cell_z;
+        // a grid in the LDS stands as long as the spectrum fits beside it, one in memory
+        // for any (built again for every other length, a call on 3000 targets between
+        // two spectra took 602 us, on 7680 targets 1444; like this 225 and 300)
+        const bool full = !ctx->grid_global &&
+                          lds_bytes(ctx->n_targets, ctx->grid.n_cells, ctx->grid.n_items,
+                                    ctx->spec_n, true) > ctx->grid_budget;
         if (ctx->grid_cell_built != want || ctx->grid_cell_z_built != want_z ||
-            ctx->grid_spec_built != ctx->spec_n || ctx->grid_cell_built < -0.5f) {
+            ctx->grid_cell_built < -0.5f || full) {
             if (int rc = build_grid(ctx, want, want_z)) {
                 if (!automatic) return rc;
                 search = PP_SEARCH_BRUTE;  // no grid fits: the every-target scan
