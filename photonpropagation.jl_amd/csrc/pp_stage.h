@@ -57,10 +57,15 @@ struct PinnedPair {
         halves = 0;
     }
 
-    // dst (host) <- src (device), ordered on the stream; returns when dst is written
+    // dst (host) <- src (device), ordered on the stream; returns when dst is written.
+    // Where no pinned memory is left, the runtime's own copy.
     hipError_t copy_out(hipStream_t st, void* dst, const void* src, size_t bytes) {
         if (bytes == 0) return hipStreamSynchronize(st);
-        if (hipError_t r = ensure(std::min(bytes, kMost), bytes > kMost ? 2 : 1)) return r;
+        if (ensure(std::min(bytes, kMost), bytes > kMost ? 2 : 1) != hipSuccess) {
+            (void)hipGetLastError();
+            if (hipError_t r = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st)) return r;
+            return hipStreamSynchronize(st);
+        }
         const size_t n = (bytes + half - 1) / half;
         auto part = [&](size_t k) { return std::min(half, bytes - k * half); };
         for (size_t k = 0; k <= n; ++k) {
