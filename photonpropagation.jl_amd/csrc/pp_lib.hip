@@ -778,17 +778,16 @@ __device__ __forceinline__ uint64_t strided_photons(uint64_t first, uint64_t end
 }
 
 // 64 photons from base on (up to end), one per lane, the whole wave together,
-// hits stored or queued. False if the hit buffer was full: the photons whose hits
-// did not fit are counted as lost, and the wave takes no more of them.
+// hits stored or queued. Returns the photons (wave-uniform) whose hits the full buffer
+// did not take: they are lost, and the wave takes no more.
 template <bool COUNT, int SEARCH>
-__device__ __forceinline__ bool propagate_group(const KParams& p, const pp_source& src,
-                                                uint32_t src_ix, uint64_t base, uint64_t end,
-                                                const float* spec, const SearchT<SEARCH>& search,
-                                                const pp::Phase& phase, WaveState& w) {
+__device__ __forceinline__ uint32_t propagate_group(const KParams& p, const pp_source& src,
+                                                    uint32_t src_ix, uint64_t base, uint64_t end,
+                                                    const float* spec, const SearchT<SEARCH>& search,
+                                                    const pp::Phase& phase, WaveState& w) {
     const uint64_t pid = base + __lane_id();
-    uint32_t lost;
     if constexpr (kDeferredWalk<SEARCH>) {
-        lost = transport_group<COUNT, SEARCH>(p, src, src_ix, pid, pid < end, spec, search, phase, w.q,
+        return transport_group<COUNT, SEARCH>(p, src, src_ix, pid, pid < end, spec, search, phase, w.q,
                                               w.n_queued, w.work, w.n_steps_done);
     } else {
         bool stored = true;
@@ -799,10 +798,8 @@ __device__ __forceinline__ bool propagate_group(const KParams& p, const pp_sourc
             stored = store_hits(hit, h, src_ix, p.hits, p.counters);
             if (!stored) atomicOr(&p.counters->err, 1u);
         }
-        lost = (uint32_t)__popcll(__ballot(!stored));
+        return (uint32_t)__popcll(__ballot(!stored));
     }
-    add_lost(lost);
-    return lost == 0;
 }
 
 // The wave's queued hits stored, and its counts added.
@@ -831,10 +828,12 @@ __global__ void PP_PROPAGATE_ATTRS propagate_kernel(KParams p) {
          base < p.n_photons; base += stride) {
         uint32_t si = p.src_ix;
         const pp_source src = source_record(p.sources + p.src_ix, si);
-        if (!propagate_group<COUNT, SEARCH>(p, src, si, base, p.n_photons, l.spec, search, phase, w)) {
+        const uint32_t lost =
+            propagate_group<COUNT, SEARCH>(p, src, si, base, p.n_photons, l.spec, search, phase, w);
+        if (__builtin_expect(lost != 0, 0)) {
             // the call fails: the wave's later groups are given up in one sum (an
             // atomic for each held a launch of 1e9 photons for 190 ms)
-            add_lost(strided_photons(base + stride, p.n_photons, stride));
+            add_lost(lost + strided_photons(base + stride, p.n_photons, stride));
             break;
         }
     }
@@ -925,21 +924,24 @@ __global__ void PP_PROPAGATE_ATTRS propagate_batch_kernel(KParams p, BatchParams
         const uint64_t ck = uniform64(next);
         if (ck >= batch_params().n_items) break;
         const BatchItem it = batch_item(ck);
-        bool fits = true;
-        for (uint64_t base = it.first; base < it.end && fits; base += 64) {
+        uint32_t lost = 0;
+        for (uint64_t base = it.first; base < it.end; base += 64) {
             // the source index and record, opaque to the optimiser in every
             // iteration: what the emission derives from them is computed here
             // (one scalar reload per 64 photons) instead of being hoisted out
             // of the loop into registers that then spill to scratch
             uint32_t si = (uint32_t)it.source;
             const pp_source src = source_record(batch_params().sources + it.source, si);
-            fits = propagate_group<COUNT, SEARCH>(p, src, si, base, it.end, l.spec, search, phase, w);
-            if (!fits && it.end - base > 64) add_lost(it.end - base - 64);
+            lost = propagate_group<COUNT, SEARCH>(p, src, si, base, it.end, l.spec, search, phase, w);
+            if (__builtin_expect(lost != 0, 0)) {
+                lost += (uint32_t)(it.end - base > 64 ? it.end - base - 64 : 0);
+                break;
+            }
         }
-        if (!fits) {
+        if (__builtin_expect(lost != 0, 0)) {
             // the call fails; take no more chunks, and give those dealt to this wave up
             const BatchParams b = batch_params();
-            uint64_t left = 0;
+            uint64_t left = lost;
             if (b.dealt)
                 for (uint64_t k = ck + waves; k < b.n_items; k += waves) {
                     const BatchItem rest = batch_item(k);
