@@ -869,14 +869,14 @@ struct pp_mlp {
     float *dsX = nullptr, *dsL = nullptr;
     int64_t ds_cap = 0;
     // pair evaluation: events | modules, the outputs of a list of one slice, the
-    // stream of every other slice of a longer one and the timing events of three
+    // stream of every other slice of a longer one and the timing events of four
     // slices in a row
     char* d_in = nullptr;
     size_t in_cap = 0;
     char* d_out = nullptr;
     size_t out_cap = 0;
     hipStream_t other = nullptr;
-    hipEvent_t t0[3] = {}, t1[3] = {};
+    hipEvent_t t0[4] = {}, t1[4] = {};
     float* logy = nullptr;
     pp::PinnedPair pin;  // results on their way to pageable host memory
 };
@@ -1409,7 +1409,7 @@ int pp_mlp_destroy(pp_mlp* M) {
     for (auto* p : M->Z)
         if (p) (void)hipFree(p);
     M->pin.release();
-    for (int i = 0; i < 3; ++i)
+    for (int i = 0; i < 4; ++i)
         for (hipEvent_t e : {M->t0[i], M->t1[i]})
             if (e) (void)hipEventDestroy(e);
     if (M->other) (void)hipStreamDestroy(M->other);
@@ -1671,18 +1671,20 @@ int pp_sur_eval_pairs(pp_mlp* M, const pp_cascade* events, int n_events, const f
     if (n == 0) return PP_OK;
     if (int rc = set_dev(M)) return rc;
     // Lists of one slice run at once; longer ones slice by slice, the kernels writing
-    // to two pinned halves in turn and the host moving a slice to the caller while
-    // the next is computed. Without mixtures every other slice runs on a second
-    // stream: a launch behind another on one stream waits until the other's last
-    // store to host memory has arrived (16 us a slice). Copies from device buffers on
+    // to pinned parts in turn and the host moving a slice to the caller while the
+    // next is computed. Without mixtures every other slice runs on a second
+    // stream, two ahead of the host: a launch behind another on one stream waits until
+    // the other's last store to host memory has arrived (16 us a slice). Copies from device buffers on
     // a stream of their own ran at a quarter of the bus beside the kernels for the
     // first 30 to 80 of them, which shorter lists never got past: first and later
-    // calls of a network on 3e5 pairs 0.70 and 0.59 ms (copies after the kernel, in
-    // one piece: 0.47 and 0.53; like this 0.36 and 0.27), 1e6 pairs 1.26 and 1.18 (1.02
-    // and 0.83; 0.76 and 0.68), 5e6 pairs 4.8-5.4 and 2.9 (4.65 and 4.3; 3.1 and 2.8),
-    // with mixtures 3e5 pairs 1.5 and 1.4 (1.2 and 2.4; 0.74 and 0.69), 2e6 pairs 6.7
-    // and 6.2 (8.6 and 8.5; 5.8 and 5.7). Their stores of 36 bytes a pair stretch the
-    // kernels of the last from 1.0 to 2.5 ms, which the host's part hides.
+    // calls of a network on 3e5 pairs 0.74 and 0.59 ms (copies after the kernel, in
+    // one piece: 0.47 and 0.53; like this 0.36 and 0.27), 1e6 pairs 1.24 and 1.18 (1.02
+    // and 0.83; 0.73 and 0.63), 5e6 pairs 5.1 and 2.86 (4.65 and 4.3; 3.0 and 2.65),
+    // 1e7 pairs later 6.1 (10.7; 6.3); with mixtures 3e5 pairs 1.5 and 1.4 (1.2 and
+    // 2.4; 0.74 and 0.69), 2e6 pairs 6.7 and 6.2 (8.6 and 8.5; 5.8 and 5.7). The
+    // stores to host memory stretch the kernels, of 1e7 pairs from 4.4 to 4.8 ms, of
+    // 2e6 with mixtures (36 bytes a pair apart) from 1.0 to 2.5, beside a host that
+    // takes longer.
     const bool fused = M->fused && M->wpk;
     const int64_t most = mixture ? kPairMixSlice : kPairSlice;
     const int64_t slice = std::min<int64_t>(n, fused ? most : std::min<int64_t>(most, M->max_batch));
@@ -1692,6 +1694,7 @@ int pp_sur_eval_pairs(pp_mlp* M, const pp_cascade* events, int n_events, const f
     const size_t off_fb = off_mix + (mixture ? (size_t)slice * 36 : 0);
     const size_t out_b = (off_fb + (size_t)slice + 255) & ~(size_t)255;
     const bool sliced = slice < n, two = sliced && fused && !mixture;
+    const int64_t ahead = two ? 2 : 1, parts = ahead + 1;  // slices in flight, pinned parts
     auto grow = [&](char** p, size_t* cap, size_t need) -> int {
         if (need <= *cap) return PP_OK;
         if (*p) PP_HIP(hipFree(*p));
@@ -1706,10 +1709,10 @@ int pp_sur_eval_pairs(pp_mlp* M, const pp_cascade* events, int n_events, const f
         if (int rc = grow(&M->d_out, &M->out_cap, out_b)) return rc;
     if (!fused && !M->logy) PP_HIP(hipMalloc(&M->logy, (size_t)M->max_batch * 4));
     if (two && !M->other) PP_HIP(hipStreamCreateWithFlags(&M->other, hipStreamNonBlocking));
-    for (int i = 0; i < (sliced ? 3 : 1); ++i)
+    for (int i = 0; i < (sliced ? 4 : 1); ++i)
         for (hipEvent_t* e : {&M->t0[i], &M->t1[i]})
             if (!*e) PP_HIP(hipEventCreate(e));
-    PP_HIP(M->pin.ensure(std::max(out_b, in_b <= kPairPinnedIn ? in_b : (size_t)0)));
+    PP_HIP(M->pin.ensure(std::max(out_b, in_b <= kPairPinnedIn ? in_b : (size_t)0), (int)parts));
     auto* d_ev = (pp_cascade*)M->d_in;
     auto* d_mod = (float*)(M->d_in + off_mod);
     if (in_b <= kPairPinnedIn) {  // one copy from pinned memory
@@ -1730,8 +1733,8 @@ int pp_sur_eval_pairs(pp_mlp* M, const pp_cascade* events, int n_events, const f
     float device_ms = 0.0f;
     // the slice's launches
     auto start = [&](int64_t k) -> int {
-        const int b = (int)(k & 1), e = (int)(k % 3);
-        const hipStream_t st = two && b ? M->other : M->stream;
+        const int b = (int)(k % parts), e = (int)(k & 3);
+        const hipStream_t st = two && (k & 1) ? M->other : M->stream;
         const int64_t r0 = k * slice;
         const int64_t rows = std::min<int64_t>(slice, n - r0);
         char* out = sliced ? M->pin.at(b) : M->d_out;
@@ -1769,7 +1772,7 @@ int pp_sur_eval_pairs(pp_mlp* M, const pp_cascade* events, int n_events, const f
     };
     // the slice's results to the caller
     auto finish = [&](int64_t k) -> int {
-        const int b = (int)(k & 1);
+        const int b = (int)(k % parts);
         const int64_t r0 = k * slice;
         const size_t rows = (size_t)std::min<int64_t>(slice, n - r0);
         PP_HIP(hipEventSynchronize(M->pin.ev[b]));
@@ -1779,20 +1782,20 @@ int pp_sur_eval_pairs(pp_mlp* M, const pp_cascade* events, int n_events, const f
         if (fallback) std::memcpy(fallback + r0, src + off_fb, rows);
         if (kernel_ms) {
             // of a slice that ran beside the one before, what came after that one
-            const hipEvent_t end = M->t1[k % 3];
+            const hipEvent_t end = M->t1[k & 3];
             float ms = 0.0f, after = INFINITY;
-            PP_HIP(hipEventElapsedTime(&ms, M->t0[k % 3], end));
-            if (two && k > 0) PP_HIP(hipEventElapsedTime(&after, M->t1[(k - 1) % 3], end));
+            PP_HIP(hipEventElapsedTime(&ms, M->t0[k & 3], end));
+            if (two && k > 0) PP_HIP(hipEventElapsedTime(&after, M->t1[(k - 1) & 3], end));
             device_ms += std::max(std::min(ms, after), 0.0f);
         }
         return PP_OK;
     };
     const int64_t slices = (n + slice - 1) / slice;
     int rc = PP_OK;
-    // the second pinned half holds the inputs until the first slice can run
-    for (int64_t k = 0; k <= slices && rc == PP_OK; ++k) {
+    // the second pinned part holds the inputs until the first slice can run
+    for (int64_t k = 0; k < slices + ahead && rc == PP_OK; ++k) {
         if (k < slices) rc = start(k);
-        if (k > 0 && rc == PP_OK) rc = finish(k - 1);
+        if (k >= ahead && rc == PP_OK) rc = finish(k - ahead);
     }
     if (rc != PP_OK) {  // nothing may still use the workspace
         (void)hipStreamSynchronize(M->stream);

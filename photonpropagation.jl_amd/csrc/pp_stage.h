@@ -18,8 +18,9 @@ namespace pp {
 struct PinnedPair {
     char* p = nullptr;
     size_t half = 0;    // bytes of each half
-    int halves = 0;     // one where all the work is a single piece, else two
-    hipEvent_t ev[2] = {nullptr, nullptr};
+    int halves = 0;     // one where all the work is a single piece, two, or a third for
+                        // work that runs two pieces ahead
+    hipEvent_t ev[3] = {};
 
     static constexpr size_t kMost = (size_t)4 << 20;  // half of copy_out's own choice
 
@@ -45,7 +46,7 @@ struct PinnedPair {
         halves = n;
         return hipSuccess;
     }
-    char* at(int k) const { return p + (size_t)(k & 1) * half; }
+    char* at(int k) const { return p + (size_t)k * half; }
     void release() {
         if (p) (void)hipHostFree(p);
         for (auto& e : ev) {
@@ -70,14 +71,14 @@ struct PinnedPair {
         auto part = [&](size_t k) { return std::min(half, bytes - k * half); };
         for (size_t k = 0; k <= n; ++k) {
             if (k < n) {
-                if (hipError_t r = hipMemcpyAsync(at((int)k), (const char*)src + k * half, part(k),
+                if (hipError_t r = hipMemcpyAsync(at((int)(k & 1)), (const char*)src + k * half, part(k),
                                                   hipMemcpyDeviceToHost, st))
                     return r;
                 if (hipError_t r = hipEventRecord(ev[k & 1], st)) return r;
             }
             if (k > 0) {
                 if (hipError_t r = hipEventSynchronize(ev[(k - 1) & 1])) return r;
-                std::memcpy((char*)dst + (k - 1) * half, at((int)(k - 1)), part(k - 1));
+                std::memcpy((char*)dst + (k - 1) * half, at((int)((k - 1) & 1)), part(k - 1));
             }
         }
         return hipSuccess;
