@@ -236,8 +236,10 @@ def pmt_leg():
     return {"hits": n, "kernel_ms": k, "hits_per_s": n / (k * 1e-3),
             "detected_frac": det / n, "bytes_per_hit": bytes_per_hit,
             "achieved_gbps": gbps, "hbm_frac": gbps / 8000.0,
-            "note": "16 PMTs per hit: acos, a square root, exp and a reciprocal each, one "
-                    "Philox block; vector-ALU bound, not HBM bound",
+            "note": "one Philox block per hit; hits whose draw exceeds every possible sum of "
+                    "weights need none, the others take approximate weights of the 16 PMTs "
+                    "and those too close to call the full ones; bound by HBM and the vector "
+                    "ALU about equally",
             "end_to_end": pmt_end_to_end()}
 
 

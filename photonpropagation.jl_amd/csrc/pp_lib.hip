@@ -2410,7 +2410,7 @@ __global__ void gather_hits_kernel(const HitRecord* __restrict__ rec,
 // too (the copy of a small hit table). 64 hits per workgroup, the keys in tiles
 // of LDS, a quarter of each tile per wave. For a few thousand hits the radix sort
 // is five launches of a few workgroups and the copy a sixth: 25-45 us of a call
-// for the README example's 14 hits or a small shower's 1200; 3-9 us here. The
+// for the README example's 14 hits or a small shower's 1200; 2.5 and 13 us here. The
 // compares grow with the square of the count, and at 4096 the two are near.
 constexpr int kRankMost = 4096;
 

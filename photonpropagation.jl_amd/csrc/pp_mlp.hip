@@ -1091,7 +1091,7 @@ constexpr size_t kPairPinnedIn = 256 << 10;       // inputs that go through pinn
 
 // Whether a training step runs as the two launches of pp_train.h: the shapes
 // of the fused inference kernel with at most kTMaxHidden hidden layers, and the
-// workspace for `rows` rows, which is kept (2.1 KB per row for the default
+// workspace for `rows` rows, which is kept (4.2 KB per row for the default
 // network). Where it does not fit device memory the step runs layer by layer.
 // Measured (batch 4096 of the 8-256x4-10 network): 347 us a step layer by layer,
 // 47 us in two launches.

@@ -11,14 +11,17 @@
 // sums over the batch - weight and bias gradients and the Adam update they
 // feed - runs in train_grads_kernel. Only the bf16 operands of the weight
 // gradients pass through memory between the two (17 MB at batch 4096, in the
-// caches); pre-activations stay in registers, activations in LDS.
+// caches); activations stay in LDS, pre-activations in registers, of which they
+// leave too few from four hidden layers on: the rows kernel then spills (104 bytes
+// of scratch a lane at four, 248 at five, 376 at six; steps of 55, 73 and 88 us at
+// batch 4096 against 360, 422 and 489 layer by layer).
 //
 // Every number is the one the layer-by-layer kernels give: the same 16-term
 // MFMA products in the same K order from the same accumulator inputs, the same
 // slices of the batch summed in the same order, the same epilogues, and the
 // loss's sums over the bins taken bin by bin.
 
-constexpr int kTMaxHidden = 6;  // hidden layers (their pre-activations stay in registers)
+constexpr int kTMaxHidden = 6;  // hidden layers the rows kernel is built for
 
 // Row operands of the weight gradients, H (a layer's input) and D (the gradient
 // of its pre-activations), are stored as MFMA operands with the batch as K:
